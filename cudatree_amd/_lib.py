@@ -20,6 +20,7 @@ CTA_MODE_HYBRID = 1
 CTA_MODE_PER_NODE = 2
 MODES = {"batched": CTA_MODE_BATCHED, "hybrid": CTA_MODE_HYBRID, "per_node": CTA_MODE_PER_NODE}
 CTA_HIST_AUTO, CTA_HIST_REGS, CTA_HIST_LDS = 0, 1, 2
+CTA_SEARCH_AUTO, CTA_SEARCH_ROWS, CTA_SEARCH_LISTS = 0, 1, 2
 
 MAX_SAMPLES = 4194303
 MAX_FEATURES = 65535
@@ -55,7 +56,7 @@ class FitOpts(ctypes.Structure):
         ("fill_global", ctypes.c_int32),
         ("hist_layout", ctypes.c_int32),
         ("subtree_max", ctypes.c_int32),
-        ("reserved", ctypes.c_int32 * 1),
+        ("search", ctypes.c_int32),
     ]
 
 

@@ -25,6 +25,7 @@
 #include "../../include/cudatree_amd.h"
 #include "aux_kernels.hip"
 #include "fit_kernels.hip"
+#include "list_kernels.hip"
 #include "subtree_kernels.hip"
 
 using namespace cta;
@@ -256,6 +257,11 @@ struct cta_dataset {
   int32_t N = 0, F = 0, K = 0, idx_bits = 32, lab_bits = 8;
   DevMem XT, y, si0;
   DevMem codes, fcode;  // value code columns (see k_code_index)
+  // list search, made by the first fit that uses it: words by sample, the
+  // features' distinct values, and per feature where they start and the index
+  // distance that needs no test
+  bool listed = false;
+  DevMem rank, dval, voff, gapw;
   // row-free features (two-valued, other than feature 0): tables of the fits
   // that keep no rows for them, and identity tables for fits that keep all
   int32_t Frl = 0, Wsig = 0, Fr = 0;
@@ -451,6 +457,62 @@ constexpr uint32_t kLevelGroup = CTA_LEVEL_GROUP;
 constexpr uint32_t kScanChunk = 1024, kReshChunk = 4096, kFillChunk = CTA_FILL_CHUNK;
 
 
+// Whether a fit searches its splits from sample lists (list_kernels.hip)
+// instead of sorted rows; Fr: the rows it would keep.
+bool list_fits(const cta_ctx &ctx, const cta_dataset &ds, const cta_fit_opts &o, uint32_t Fr) {
+  if (o.search == CTA_SEARCH_ROWS || o.mode != CTA_MODE_BATCHED || o.all_rows || o.subtree_max > 0) return false;
+  // every node must fit a workgroup's sort, and its class counts the LDS left
+  if ((uint32_t)ds.N > kListWg[1] || (size_t)list_wg_words(1, (uint32_t)ds.K) * 4 > ctx.lds_per_block) return false;
+  if (o.search == CTA_SEARCH_LISTS) return true;
+  // Rows move Fr rows per level where lists sort max_features of them, but a
+  // node's sort takes one workgroup where rows split it into chunks.  Rows /
+  // lists, ms: 20,000 x 4,096 (Fr / m = 64) 238 / 51; 7,490 x 233 (14) 7.5 /
+  // 5.3; 10,253 x 151, 6 trees (12) 3.8 / 3.8; 1,797 x 64 (8) 2.0 / 2.3;
+  // 29,894 x 48 (7) 3.5 / 4.5.
+  return (uint64_t)Fr >= 10ull * (uint64_t)o.max_features;
+}
+
+// The list search's tables of a training set (kept with it; built on the
+// context's stream before the fit's own work).
+template <class IdxT, class LabT>
+void list_tables(cta_ctx *ctx, cta_dataset *ds) {
+  if (ds->listed) return;
+  const uint32_t N = ds->N, F = ds->F;
+  hipStream_t st = ctx->stream;
+  Timed tm(ctx, "k_list_tables");
+  const uint32_t ntiles = (N + kCodeTile - 1) / kCodeTile;
+  uint32_t *pre = ctx->ws_as<uint32_t>("code_pre", (size_t)N * F);
+  uint32_t *tsum = ctx->ws_as<uint32_t>("code_tsum", (size_t)ntiles * F);
+  uint32_t *db = ctx->ws_as<uint32_t>("code_meta", 2 * (size_t)F);  // distinct values, then the bad flags
+  const IdxT *rows = ds->si0.as<IdxT>();
+  const float *XT = ds->XT.as<float>();
+  k_fill_u32<<<grid_for(2 * (size_t)F), 256, 0, st>>>(db, 2 * (size_t)F, 0u);
+  k_list_flags<IdxT><<<dim3(ntiles, F), kCodeThreads, 0, st>>>(rows, XT, N, ntiles, pre, tsum, db + F);
+  k_code_tscan<<<F, 1024, 0, st>>>(tsum, ntiles, db);
+  uint32_t *h = static_cast<uint32_t *>(ctx->host("code_meta", 2 * (size_t)F * 4));
+  HIPC(hipMemcpyAsync(h, db, (size_t)F * 4, hipMemcpyDeviceToHost, st));
+  ds->rank.alloc((size_t)N * F * 4);
+  ds->voff.alloc((size_t)F * 8);
+  ds->gapw.alloc((size_t)F * 4);
+  uint64_t *hv = static_cast<uint64_t *>(ctx->host("list_voff", (size_t)F * 8));
+  ctx->sync();
+  uint64_t nval = 0;
+  for (uint32_t f = 0; f < F; ++f) {
+    hv[f] = nval;
+    nval += h[f];
+  }
+  ds->dval.alloc(nval * 4);
+  HIPC(hipMemcpyAsync(ds->voff.p, hv, (size_t)F * 8, hipMemcpyHostToDevice, st));
+  k_fill_u32<<<grid_for(F), 256, 0, st>>>(ds->gapw.as<uint32_t>(), F, 1u);
+  k_list_tables<IdxT, LabT><<<dim3(ntiles, F), kCodeThreads, 0, st>>>(
+      rows, XT, ds->y.as<LabT>(), pre, tsum, N, ntiles, ds->voff.as<uint64_t>(), ds->rank.as<uint32_t>(),
+      ds->dval.as<float>());
+  k_list_gapw<<<dim3(std::min<uint32_t>(64, ntiles), F), kCodeThreads, 0, st>>>(
+      ds->dval.as<float>(), ds->voff.as<uint64_t>(), db, db + F, ds->gapw.as<uint32_t>());
+  HIPC(hipGetLastError());
+  ds->listed = true;
+}
+
 template <class IdxT, class LabT>
 struct Fitter {
   cta_ctx *ctx;
@@ -459,6 +521,9 @@ struct Fitter {
   int32_t N, F, K, m;
   uint32_t Cs, Cf, Cr;
   uint32_t sub_max;  // small-subtree threshold of batched fits (0: none)
+  bool list;         // list search: only feature 0's row is kept
+  uint32_t Fc = 0;   // features the split-scan classes are laid over
+  uint32_t Glist = 0, Gwg[2] = {0, 0};  // blocks of k_list_scan and k_list_wg
   hipStream_t st;
   uint32_t G;      // blocks of the wave-loop kernels
   uint32_t Gscan;  // blocks of k_scan: all resident at once, a multiple of kXcd
@@ -493,6 +558,9 @@ struct Fitter {
     rl_of_d = (rowfree ? d->rl_of : d->rl_none).as<int32_t>();
     slot_of_d = (rowfree ? d->slot_of : d->ident).as<int32_t>();
     row_feat_d = (rowfree ? d->row_feat : d->ident).as<int32_t>();
+    Fc = Fr;
+    list = list_fits(*c, *d, opts, Fr);
+    if (list) Fr = 1;  // (feature 0 has the first row slot)
     // a wave-loop grid larger than what stays resident leaves a tail of
     // late workgroups; k_scan's registers allow fewer than 8 per CU
     int nb = 0;
@@ -500,16 +568,34 @@ struct Fitter {
     HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &nb, scan_regs ? k_scan<IdxT, LabT, true> : k_scan<IdxT, LabT, false>, kBlock, smem()));
     nb = std::min(std::max(nb, 1), 8);
+    if (list) {
+      auto grid = [&](const void *k, int threads, size_t lds) {
+        int b = 0;
+        HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k, threads, lds));
+        return std::max<uint32_t>(kXcd, (uint32_t)(ctx->num_cu * std::max(b, 1)) / kXcd * kXcd);
+      };
+      const void *wg[2] = {scan_regs ? (const void *)k_list_wg<IdxT, LabT, 0, true> : (const void *)k_list_wg<IdxT, LabT, 0, false>,
+                           scan_regs ? (const void *)k_list_wg<IdxT, LabT, 1, true> : (const void *)k_list_wg<IdxT, LabT, 1, false>};
+      for (int w = 0; w < 2; ++w) {
+        HIPC(hipFuncSetAttribute(wg[w], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_per_block));
+        Gwg[w] = grid(wg[w], kListWaves[w] * kWave, list_wg_words(w, (uint32_t)K) * 4);
+      }
+      Glist = grid(scan_regs ? (const void *)k_list_scan<IdxT, LabT, true> : (const void *)k_list_scan<IdxT, LabT, false>,
+                   kBlock, list_lds());
+    }
     Gscan = std::max<uint32_t>(kXcd, (uint32_t)(ctx->num_cu * nb) / kXcd * kXcd);
   }
 
   // side bitmap, then each wave's row-free counters
   size_t fill_lds_bytes() const { return (((size_t)N + 31) / 32) * 4 + (size_t)kFillWaves * Frl * K * 4; }
 
+  size_t list_lds() const { return (size_t)kWavesPerBlock * list_wave_words((uint32_t)K, scan_regs) * 4; }
+
   size_t smem() const { return (size_t)kWavesPerBlock * 2 * K * sizeof(uint32_t); }
 
   // Bytes of device memory one resident tree needs (rows, marks, level state).
-  size_t bytes_per_tree() const { return tree_bytes(N, Fr, K, m, sizeof(IdxT)); }
+  // (a list fit counts the rows it does not keep too: room for its task lists)
+  size_t bytes_per_tree() const { return tree_bytes(N, Fc, K, m, sizeof(IdxT)); }
 
   // Grows trees [t0, t0 + Tb) and appends them to `out` in pre-order.
   void run_batch(int32_t t0, int32_t Tb, int32_t total_trees, const uint32_t *boot_ids, const int64_t *boot_off,
@@ -557,9 +643,12 @@ struct Fitter {
     const uint64_t cap_big = (uint64_t)Fr * (n_tot / kBigN + Tb + 1);
     const uint64_t cap_small = cap_q + 2ull * Fr * n_tot / Cr + 64;
     const uint64_t cap_fill = cap_q + n_tot / Cf + 64;
-    const uint64_t cap_hist = (uint64_t)m * K * (2 * n_tot / Cs + 64);
+    const uint64_t cap_hist = (uint64_t)m * K * ((list ? n_tot / kListWave : 2 * n_tot / Cs) + 64);
+    // (node, feature) tasks of nodes of more than kListWave / kListWg[0] samples
+    const uint64_t cap_wg[2] = {list ? (uint64_t)m * (n_tot / kListWave) + 64 : 0,
+                                list ? (uint64_t)m * (n_tot / kListWg[0]) + 64 : 0};
     if (cap_scan > 0xFFFFFFF0ull || cap_small > 0xFFFFFFF0ull || cap_big > 0xFFFFFFF0ull ||
-        cap_nodes > 0xFFFFFFF0ull || cap_hist > 0xFFFFFFF0ull)
+        cap_nodes > 0xFFFFFFF0ull || cap_hist > 0xFFFFFFF0ull || cap_wg[0] > 0xFFFFFFF0ull)
       fail(CTA_EUNSUPPORTED, "batch of %d trees too large for 32-bit task indices", Tb);
 
     IdxT *buf0 = ctx->ws_as<IdxT>("buf0", (size_t)Tb * Fr * N), *buf1 = ctx->ws_as<IdxT>("buf1", (size_t)Tb * Fr * N);
@@ -610,6 +699,17 @@ struct Fitter {
     a.Frl = Frl;
     a.Wsig = Wsig;
     a.Fr = Fr;
+    a.Fc = Fc;
+    if (list) {
+      a.rank = ds->rank.as<uint32_t>();
+      a.dval = ds->dval.as<float>();
+      a.voff = ds->voff.as<uint64_t>();
+      a.gapw = ds->gapw.as<uint32_t>();
+      for (int w = 0; w < 2; ++w) {
+        a.wg_tasks[w] = ctx->ws_as<Task>(w ? "wg_tasks1" : "wg_tasks0", cap_wg[w] * kXcd);
+        a.cap_wg[w] = (uint32_t)cap_wg[w];
+      }
+    }
     a.rl_of = rl_of_d;
     a.slot_of = slot_of_d;
     a.row_feat = row_feat_d;
@@ -946,12 +1046,15 @@ struct Fitter {
           Jcap, std::max<uint64_t>(1, (est + kFillTasksPerGroup - 1) / kFillTasksPerGroup));
       static std::once_flag attr;
       std::call_once(attr, [&] {
-        HIPC(hipFuncSetAttribute((const void *)k_fill_lds<IdxT, LabT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)ctx->lds_per_block));
+        for (const void *k : {(const void *)k_fill_lds<IdxT, LabT, false>, (const void *)k_fill_lds<IdxT, LabT, true>})
+          HIPC(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_per_block));
       });
-      k_fill_lds<IdxT, LabT><<<a.T * J, kFillThreads, fill_lds_bytes(), st>>>(a, J);
+      if (list) k_fill_lds<IdxT, LabT, true><<<a.T * J, kFillThreads, fill_lds_bytes(), st>>>(a, J);
+      else k_fill_lds<IdxT, LabT, false><<<a.T * J, kFillThreads, fill_lds_bytes(), st>>>(a, J);
     } else {
-      k_fill_global<IdxT, LabT><<<G, kBlock, (size_t)kWavesPerBlock * Frl * K * 4, st>>>(a);
+      const size_t lds = (size_t)kWavesPerBlock * Frl * K * 4;
+      if (list) k_fill_global<IdxT, LabT, true><<<G, kBlock, lds, st>>>(a);
+      else k_fill_global<IdxT, LabT, false><<<G, kBlock, lds, st>>>(a);
     }
   }
 
@@ -1003,7 +1106,9 @@ struct Fitter {
   // down to give a small frontier kScanTaskTarget tasks, ceil(nf / fpt)
   // sums to at most q + 2 kScanTaskTarget.
   uint64_t units_for(uint64_t q) const {
-    return q + 3 * (uint64_t)m * (n_tot / Cs + 1) + 2 * (uint64_t)kScanTaskTarget + 64;
+    // (list search: one per feature of a node of more than kListWave)
+    return q + 3 * (uint64_t)m * (n_tot / Cs + 1) + (list ? (uint64_t)m * (n_tot / kListWave) : 0) +
+           2 * (uint64_t)kScanTaskTarget + 64;
   }
 
   // Grows the task and result lists for q nodes.
@@ -1018,6 +1123,38 @@ struct Fitter {
     a.cap_scan = (uint32_t)cap;
   }
 
+  // The level's split scans over sorted rows.
+  void row_scan(const FitArgs<IdxT, LabT> &a) {
+    const size_t sm = smem();
+    {
+      Timed tm(ctx, "k_scan_hist");
+      k_scan_hist<IdxT, LabT><<<G, kBlock, sm, st>>>(a);
+    }
+    k_scan_carry<IdxT, LabT><<<G, kBlock, 0, st>>>(a);
+    Timed tm(ctx, "k_scan");
+    if (scan_regs) k_scan<IdxT, LabT, true><<<Gscan, kBlock, sm, st>>>(a);
+    else k_scan<IdxT, LabT, false><<<Gscan, kBlock, sm, st>>>(a);
+  }
+
+  // The level's split scans from the nodes' sample lists, large nodes first.
+  template <bool kRegs>
+  void list_scan_k(const FitArgs<IdxT, LabT> &a) {
+    {
+      Timed tm(ctx, "k_list_big");
+      k_list_wg<IdxT, LabT, 1, kRegs><<<Gwg[1], kListWaves[1] * kWave, list_wg_words(1, (uint32_t)K) * 4, st>>>(a);
+    }
+    {
+      Timed tm(ctx, "k_list_mid");
+      k_list_wg<IdxT, LabT, 0, kRegs><<<Gwg[0], kListWaves[0] * kWave, list_wg_words(0, (uint32_t)K) * 4, st>>>(a);
+    }
+    Timed tm(ctx, "k_scan");
+    k_list_scan<IdxT, LabT, kRegs><<<Glist, kBlock, list_lds(), st>>>(a);
+  }
+  void list_scan(const FitArgs<IdxT, LabT> &a) {
+    if (scan_regs) list_scan_k<true>(a);
+    else list_scan_k<false>(a);
+  }
+
   // One level over the frontier in a.front (ctl->q nodes, sorted by tree;
   // the host knows only a bound q on that count).
   // ev (optional): recorded after the level's plan kernel, which ends the
@@ -1027,23 +1164,18 @@ struct Fitter {
     ensure_units(a, q);
     {
       Timed tm(ctx, "k_select");
-      k_select<IdxT, LabT><<<G, kBlock, 0, st>>>(a);
+      if (list) k_select<IdxT, LabT, true><<<G, kBlock, 0, st>>>(a);
+      else k_select<IdxT, LabT, false><<<G, kBlock, 0, st>>>(a);
       offsets<kSelFields>(a, q, &a.ctl->n_scan);
-      k_select_emit<IdxT, LabT><<<G, kBlock, 0, st>>>(a);
+      if (list) k_select_emit<IdxT, LabT, true><<<G, kBlock, 0, st>>>(a);
+      else k_select_emit<IdxT, LabT, false><<<G, kBlock, 0, st>>>(a);
     }
-    {
-      Timed tm(ctx, "k_scan_hist");
-      k_scan_hist<IdxT, LabT><<<G, kBlock, sm, st>>>(a);
-    }
-    k_scan_carry<IdxT, LabT><<<G, kBlock, 0, st>>>(a);
-    {
-      Timed tm(ctx, "k_scan");
-      if (scan_regs) k_scan<IdxT, LabT, true><<<Gscan, kBlock, sm, st>>>(a);
-      else k_scan<IdxT, LabT, false><<<Gscan, kBlock, sm, st>>>(a);
-    }
+    if (list) list_scan(a);
+    else row_scan(a);
     {
       Timed tm(ctx, "k_decide");
-      k_decide<IdxT, LabT><<<G, kBlock, sm, st>>>(a);
+      if (list) k_decide<IdxT, LabT, true><<<G, kBlock, sm, st>>>(a);
+      else k_decide<IdxT, LabT, false><<<G, kBlock, sm, st>>>(a);
     }
     fill(a, q);
     {
@@ -1250,6 +1382,10 @@ template <class IdxT, class LabT>
 void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, const int64_t *off,
               const cta_fit_opts &o, cta_forest *out) {
   Fitter<IdxT, LabT> fz(ctx, ds, o);
+  if (fz.list) {
+    list_tables<IdxT, LabT>(ctx, ds);
+    if (o.lanes == 2) ctx->sync();  // (the other lane's stream reads them too)
+  }
   // trees resident at once on one stream: as asked, else what 60% of the
   // free memory holds (workspaces are reused by this fit)
   int32_t per = o.trees_per_batch;
@@ -2159,8 +2295,9 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
     // the dataset's own buffers: X_T, labels, presorted rows, code columns
     // (at most 16 bits per value), row-free signatures and feature tables,
     // plus the copies of host X and y while it is built
+    // and the list search's words and distinct values
     *dataset_bytes = nf * 4 + n * lab + nf * b + 2 * nf + 256 * f + 4 * n * ((f + 31) / 32) + 64 * f + 4096 +
-                     nf * 4 + n * 4;
+                     nf * 4 + n * 4 + nf * 8 + 16 * f;
     // the context's workspaces: radix-sort and code-column temporaries of the
     // build, then per resident tree (every feature keeping rows), the node
     // arena and canonical export of at most two nodes per in-bag sample, and
@@ -2329,7 +2466,7 @@ static void hook_split_scan(cta_ctx *ctx, cta_dataset *ds, const uint32_t *rows,
   k_scan_carry<IdxT, LabT><<<G, kBlock, 0, st>>>(a);
   if ((uint32_t)K <= kScanRegsK && !a.hist_lds) k_scan<IdxT, LabT, true><<<G, kBlock, sm, st>>>(a);
   else k_scan<IdxT, LabT, false><<<G, kBlock, sm, st>>>(a);
-  k_decide<IdxT, LabT><<<G, kBlock, sm, st>>>(a);
+  k_decide<IdxT, LabT, false><<<G, kBlock, sm, st>>>(a);
   HIPC(hipGetLastError());
   NAux out = {};
   std::vector<ScanRes> res(std::max(ntask, 1u));

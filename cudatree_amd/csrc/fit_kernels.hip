@@ -75,12 +75,12 @@ constexpr uint32_t kScanTaskTarget = CTA_SCAN_TASK_TARGET;
 // Workgroups are dispatched to the XCDs round-robin (workgroup b on XCD
 // b % kXcd, each XCD with its own L2) and k_scan's workgroup b takes class
 // b % kXcd.  Row slot s owns kXcd units, s kXcd .. s kXcd + kXcd - 1, the
-// node picks one of them, and class x holds units x Fr .. x Fr + Fr - 1: the
-// classes get equal shares of the work and a feature's tasks span at most
-// 1 + ceil(kXcd / Fr) classes, so its gathered column sits in few L2s.
+// node picks one of them, and class x holds units x Fc .. x Fc + Fc - 1 (Fc
+// slots): the classes get equal shares of the work and a feature's tasks span
+// at most 1 + ceil(kXcd / Fc) classes, so its gathered column sits in few L2s.
 template <class IdxT, class LabT>
 __device__ __forceinline__ uint32_t scan_cls(const FitArgs<IdxT, LabT> &a, uint32_t f, uint32_t i) {
-  return ((uint32_t)a.slot_of[f] * kXcd + i % kXcd) / a.Fr;
+  return ((uint32_t)a.slot_of[f] * kXcd + i % kXcd) / a.Fc;
 }
 
 template <class IdxT, class LabT>
@@ -257,12 +257,70 @@ __global__ __launch_bounds__(kOffThreads) void k_off_apply(const uint32_t *v, co
   }
 }
 
+// Node sizes of the list search: up to kListWave samples one wave sorts a
+// feature's words, up to kListWg[0] / kListWg[1] a workgroup of 4 / 16 waves.
+constexpr uint32_t kListE = 16, kListWave = kWave * kListE;
+constexpr uint32_t kListWg[2] = {4096, 32768};
+constexpr int kListWaves[2] = {4, 16};
+
 // ------------------------------------------------------------------------
 // k_select: visiting order of every frontier node, its task and slot counts
 // (scan tasks, histogram words, fill-task slots) and the frontier range of
 // each tree.
 // ------------------------------------------------------------------------
-template <class IdxT, class LabT>
+// List search: the node's order of a feature is not at hand, so the constant
+// test compares the value indices of its samples with the first sample's.
+// True in the lanes with `want` set whose column (col) differs somewhere over
+// the node's samples list[0, n), as far as it takes to know the first `need`
+// features that are not constant, `known` being those already known.
+template <class IdxT>
+__device__ __forceinline__ bool list_varies(const IdxT *list, uint32_t n, const uint32_t *col, bool want,
+                                            uint64_t known, uint32_t need) {
+  const uint32_t lane = lane_id();
+  bool diff = false;
+  const uint32_t w0 = want ? col[sample_of(list[0])] >> kLabBits : 0u;
+  // the lanes still to be decided, none once the need-th known one comes
+  // before all of them
+  auto open = [&]() -> uint64_t {
+    const uint64_t und = ballot(want && !diff), got = known | ballot(diff);
+    if (!und) return 0;
+    const uint64_t below = (und & (0ull - und)) - 1ull;
+    return (uint32_t)__popcll(got & below) >= need ? 0ull : und;
+  };
+  constexpr uint32_t U = 4;
+  const uint32_t near = min(n, 64u);
+  for (uint32_t j = 1; j < near; j += U) {
+    if (!open()) return diff;
+    uint32_t x[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) x[u] = want && !diff ? col[sample_of(list[min(j + u, n - 1u)])] >> kLabBits : w0;
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) diff |= x[u] != w0;
+  }
+  // rarely further: the wave reads one lane's column 64 U samples at a time
+  for (uint64_t und = n > near ? open() : 0ull; und; und = open()) {
+    const uint32_t L = (uint32_t)__ffsll((unsigned long long)und) - 1u;
+    const uint64_t cp = reinterpret_cast<uint64_t>(col);
+    const uint32_t *c = reinterpret_cast<const uint32_t *>((uint64_t)readlane((uint32_t)(cp >> 32), L) << 32 |
+                                                           readlane((uint32_t)cp, L));
+    const uint32_t first = readlane(w0, L);
+    bool found = false;
+    for (uint32_t pb = near; pb < n && !found; pb += U * kWave) {
+      bool d = false;
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u)
+        d |= (c[sample_of(list[min(pb + u * kWave + lane, n - 1u)])] >> kLabBits) != first;
+      found = ballot(d) != 0ull;
+    }
+    if (lane == L) {
+      diff = found;
+      want = found;
+    }
+  }
+  return diff;
+}
+
+template <class IdxT, class LabT, bool kList>
 __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
   const uint32_t lane = lane_id();
   const uint32_t m = (uint32_t)a.m, F = (uint32_t)a.F;
@@ -277,7 +335,8 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
     const uint32_t i = item;
     const FNode nd = a.front[i];
     const uint32_t n = nd.n;
-    const uint32_t nch = ceil_div(n, a.Cs);
+    // (list search: one task per feature of a node too large for one wave)
+    const uint32_t nch = kList ? (n > kListWave ? 2u : 1u) : ceil_div(n, a.Cs);
     Perm pm = make_perm(a.seed, a.tree_base + nd.tree, nd.depth, nd.start, F, a.identity != 0);
     // tasks: one per (feature, chunk) of a multi-chunk node; a single-chunk
     // node's features grouped about Cs positions per task.  A task's class is
@@ -286,8 +345,9 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
     // about kScanTaskTarget tasks to spread over the waves)
     const uint32_t fpt =
         (nch > 1) ? 1u : max(1u, (uint32_t)min<uint64_t>(a.Cs / n, (uint64_t)q * m / kScanTaskTarget));
-    const uint32_t wt = (nch > 1) ? nch : 1u;
+    const uint32_t wt = kList ? (nch > 1 ? 0u : 1u) : nch;
     const uint32_t K = (uint32_t)a.K;
+    const IdxT *list = kList ? rows_of(a, nd.src, nd.tree, 0) + nd.start : nullptr;
     uint32_t ncls = 0;
     uint32_t nf = 0;    // evaluated features with rows (they get scan tasks)
     uint32_t nsel = 0;  // evaluated features
@@ -333,7 +393,7 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
           const uint64_t nL = n - ones, nR = ones;
           const uint64_t SR = T2 + SL - 2 * Dd;
           cd = {SL * nR + SR * nL, nL * nR, (uint32_t)nL - 1u, (int32_t)f, 1u};
-        } else {
+        } else if constexpr (!kList) {
           const IdxT *row = (nd.src == 0 ? a.si0 + (size_t)f * a.N
                                          : (nd.src == 1 ? a.buf0 : a.buf1) +
                                                ((size_t)nd.tree * a.Fr + (uint32_t)slot) * a.N) +
@@ -349,6 +409,11 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
             nonconst = code_at(a.codes + fc_off(fc), kind, s0) != code_at(a.codes + fc_off(fc), kind, s1);
           }
         }
+      }
+      if constexpr (kList) {
+        const bool want = k < F && jr < 0;
+        const uint32_t *col = a.rank + (size_t)(want ? f : 0u) * (uint32_t)a.N;
+        nonconst |= list_varies(list, n, col, want, ballot(nonconst), m - nsel);
       }
       const uint64_t mk = ballot(nonconst);
       const uint32_t r = mbcnt(mk);
@@ -369,12 +434,13 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
       nsel += min((uint32_t)__popcll(mk), m - nsel);
     }
     rlb = wave_best(rlb);
-    const uint32_t ntask = (nf == 0) ? 0u : (nch > 1 ? nf * nch : ceil_div(nf, fpt));
+    const uint32_t ntask = (nf == 0) ? 0u : (nch > 1 ? (kList ? nf : nf * nch) : ceil_div(nf, fpt));
     if (lane < kXcd) a.vals[(size_t)i * kSelFields + 3 + lane] = ncls;
     if (lane == 0) {
       uint32_t *v = a.vals + (size_t)i * kSelFields;
       v[0] = ntask;
-      v[1] = (nch > 1) ? nf * nch * (uint32_t)a.K : 0u;
+      // class counts: at every chunk's start, or (list search) left of every feature's best split
+      v[1] = (nch > 1) ? ntask * (uint32_t)a.K : 0u;
       v[2] = ceil_div(n, a.Cf);
       NAux ax = {};
       ax.scan_ntask = ntask;
@@ -398,8 +464,10 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
   flush_bytes(a, kBytesScan, bytes);
 }
 
-// Writes the split-scan tasks of every node at its scanned offset.
-template <class IdxT, class LabT>
+// Writes the split-scan tasks of every node at its scanned offset (list
+// search: the tasks of the nodes too large for one wave go to the class lists
+// of the workgroup kernels, in any order: their results have fixed places).
+template <class IdxT, class LabT, bool kList>
 __global__ __launch_bounds__(kBlock) void k_select_emit(FitArgs<IdxT, LabT> a) {
   if (a.ctl->err) return;  // a list overflowed: the fit fails, nothing more is read
   const uint32_t lane = lane_id();
@@ -432,7 +500,29 @@ __global__ __launch_bounds__(kBlock) void k_select_emit(FitArgs<IdxT, LabT> a) {
     uint32_t cpos = lane < kXcd ? cls_base + o[3 + lane] : 0u;
     // items: features of a multi-chunk node (nch tasks each), else tasks
     const uint32_t nitem = nch > 1 ? nf : ntask;
-    for (uint32_t c0 = 0; c0 < nitem; c0 += kWave) {
+    if (kList && nch > 1) {
+      const int wg = a.front[i].n > kListWg[0] ? 1 : 0;
+      const uint32_t cap = a.cap_wg[wg];
+      bool over = false;
+      for (uint32_t c0 = 0; c0 < nf; c0 += kWave) {
+        const uint32_t it = c0 + lane;
+        const uint32_t c = it < nf ? scan_cls(a, (uint32_t)a.feats[(size_t)i * a.m + it], i) : kXcd;
+        for (uint32_t x = 0; x < kXcd; ++x) {
+          const uint64_t mk = ballot(c == x);
+          if (!mk) continue;
+          const uint32_t lead = (uint32_t)__ffsll((unsigned long long)mk) - 1u;
+          uint32_t p = 0;
+          if (lane == lead) p = atomicAdd(&a.ctl->n_wg[wg][x], (uint32_t)__popcll(mk));
+          p = readlane(p, lead) + mbcnt(mk);
+          if (c == x) {
+            if (p < cap) a.wg_tasks[wg][(size_t)x * cap + p] = Task{i, it | (1u << 16), 0u, 1u};
+            else over = true;
+          }
+        }
+      }
+      if (ballot(over) && lane == 0) atomicOr(&a.ctl->err, kErrCapacity);
+    }
+    for (uint32_t c0 = 0; c0 < nitem && !(kList && nch > 1); c0 += kWave) {
       const uint32_t it = c0 + lane;
       const bool valid = it < nitem;
       const uint32_t c = valid ? scan_cls(a, (uint32_t)a.feats[(size_t)i * a.m + (nch > 1 ? it : it * fpt)], i) : kXcd;
@@ -1162,7 +1252,37 @@ __device__ __forceinline__ uint32_t child_kind(const FitArgs<IdxT, LabT> &a, uin
   return 0u;
 }
 
+// Class counts of the samples of node i whose value index of feature f is at
+// most lo (list search, a node of one wave) into cntL; returns their sum.
 template <class IdxT, class LabT>
+__device__ uint32_t count_left_list(const FitArgs<IdxT, LabT> &a, uint32_t i, const FNode &nd, uint32_t f, uint32_t lo,
+                                uint32_t *h) {
+  const uint32_t lane = lane_id(), K = (uint32_t)a.K, n = nd.n;
+  const IdxT *list = rows_of(a, nd.src, nd.tree, 0) + nd.start;
+  const uint32_t *col = a.rank + (size_t)f * (uint32_t)a.N;
+  wave_sync();
+  for (uint32_t k = lane; k < K; k += kWave) h[k] = 0;
+  wave_sync();
+  for (uint32_t pb = 0; pb < n; pb += 4 * kWave) {
+    uint32_t e[4], w[4];
+    load_row_batch(list, pb, n, e);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) w[u] = col[sample_of((IdxT)e[u])];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (pb + (uint32_t)u * kWave + lane < n && (w[u] >> kLabBits) <= lo) atomicAdd(&h[w[u] & kLabMask], 1u);
+  }
+  wave_sync();
+  uint32_t sum = 0;
+  for (uint32_t k = lane; k < K; k += kWave) {
+    a.cntL[(size_t)i * K + k] = h[k];
+    sum += h[k];
+  }
+  wave_sync();
+  return wave_sum32(sum);
+}
+
+template <class IdxT, class LabT, bool kList>
 __global__ __launch_bounds__(kBlock) void k_decide(FitArgs<IdxT, LabT> a) {
   if (a.ctl->err) return;  // a list overflowed: the fit fails, nothing more is read
   extern __shared__ uint32_t smem[];
@@ -1174,12 +1294,22 @@ __global__ __launch_bounds__(kBlock) void k_decide(FitArgs<IdxT, LabT> a) {
     const FNode nd = a.front[i];
     NAux ax = a.aux[i];
     Cand best = {0, 1, 0, 0, 0};
+    uint32_t bt = 0;  // its task
     for (uint32_t t = lane; t < ax.scan_ntask; t += kWave) {
       const ScanRes r = a.res[ax.scan_base + t];
       Cand c = {r.num, r.den, r.pos, r.feat, r.ok};
-      if (cand_better(c, best)) best = c;
+      if (cand_better(c, best)) {
+        best = c;
+        bt = t;
+      }
     }
+    const int32_t own = best.ok ? best.feat : -1;
     best = wave_best(best);
+    if constexpr (kList) {
+      // a feature is scanned by one task here, so its lane is the winner's
+      const uint64_t mk = ballot(best.ok && own == best.feat);
+      if (mk) bt = readlane(bt, (uint32_t)__ffsll((unsigned long long)mk) - 1u);
+    }
     // the evaluated row-free features' best candidate, under the same order
     const Cand rlcand = {ax.rl_num, ax.rl_den, ax.rl_pos, ax.rl_feat, (a.Frl && ax.rl_feat >= 0) ? 1u : 0u};
     const bool rowfree = cand_better(rlcand, best);
@@ -1217,6 +1347,34 @@ __global__ __launch_bounds__(kBlock) void k_decide(FitArgs<IdxT, LabT> a) {
       ax.best_f = (int32_t)f;
       ax.best_p = p;
       ax.nL = p + 1;
+      ax.flags = kSplit | (2 * ax.nL > nd.n ? kInvert : 0u);
+      ax.dst = (nd.src == 2) ? 1u : 2u;
+    } else if (kList) {
+      // the side of a sample follows from its value index: the marks are
+      // made over the node's whole list
+      const uint32_t f = (uint32_t)best.feat, K = (uint32_t)a.K;
+      const ScanRes r = a.res[ax.scan_base + bt];
+      if (ax.nch_s > 1) {
+        const uint32_t *lc = a.hist + ax.hist_base + (size_t)bt * K;
+        for (uint32_t k = lane; k < K; k += kWave) a.cntL[(size_t)i * K + k] = lc[k];
+      } else {
+        // (the samples of a value index up to lo are those up to the position:
+        // the sides follow from the one, the children's sizes from the other)
+        if (count_left_list(a, i, nd, f, r.lo, h) != best.pos + 1u && lane == 0) atomicOr(&a.ctl->err, kErrBadNode);
+      }
+      nfill = nd.n;
+      if (lane == 0) {
+        const float *v = a.dval + a.voff[f];
+        // threshold midway in float, no contraction (bfs_module.cu:399-400)
+        a.arena.feat[id] = (int32_t)f;
+        a.arena.thr[id] = __fmul_rn(__fadd_rn(v[r.lo], v[r.hi]), 0.5f);
+        a.arena.value[id] = 0;
+        bytes += (unsigned long long)nd.n * (sizeof(IdxT) + 1);  // fill: n (b + 1)
+      }
+      ax.best_f = (int32_t)f;
+      ax.best_p = best.pos;
+      ax.lo = r.lo;
+      ax.nL = best.pos + 1;
       ax.flags = kSplit | (2 * ax.nL > nd.n ? kInvert : 0u);
       ax.dst = (nd.src == 2) ? 1u : 2u;
     } else {
@@ -1418,7 +1576,8 @@ __device__ __forceinline__ void rl_zero(uint32_t *cnt, uint32_t FK) {
 // wave's start) hold node `cur`'s counts: a task of another counting node
 // flushes them to rl_small first; the wave flushes the last node's at its
 // end.
-template <class IdxT, class LabT>
+// kList: the sides of a split on a feature follow from the value indices.
+template <bool kList, class IdxT, class LabT>
 __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, const Task &tk, uint32_t *bits,
                                                uint32_t *cnt, uint32_t &cur, bool &cur_whole) {
   const uint32_t lane = lane_id();
@@ -1432,12 +1591,15 @@ __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, con
     cur = tk.node;
     cur_whole = tk.nch == 1;
   }
-  if (jr >= 0) {
-    // row-free split: the samples holding the lower value, over feature 0's row
+  if (kList || jr >= 0) {
+    // row-free split: the samples holding the lower value, over feature 0's
+    // row; list search: those of a value index up to ax.lo
     const IdxT *row = rows_of(a, nd.src, nd.tree, 0) + nd.start;
     const uint32_t p0 = tk.chunk * a.Cf, p1 = min(nd.n, p0 + a.Cf);
+    const bool bycol = !kList || jr >= 0;
     // the feature's bit column (N / 8 bytes) rather than the signatures
-    const uint32_t *col = reinterpret_cast<const uint32_t *>(a.codes + fc_off(a.fcode[ax.best_f]));
+    const uint32_t *col = bycol ? reinterpret_cast<const uint32_t *>(a.codes + fc_off(a.fcode[ax.best_f]))
+                                : a.rank + (size_t)(uint32_t)ax.best_f * (uint32_t)a.N;
     for (uint32_t pb = p0; pb < p1; pb += kFillU * kWave) {
       uint32_t e[kFillU], low[kFillU];
 #pragma unroll
@@ -1448,7 +1610,9 @@ __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, con
 #pragma unroll
       for (int u = 0; u < kFillU; ++u) {
         const uint32_t s = sample_of((IdxT)e[u]);
-        low[u] = (e[u] != 0xFFFFFFFFu) ? !((col[s >> 5] >> (s & 31u)) & 1u) : 0u;
+        low[u] = 0u;
+        if (e[u] != 0xFFFFFFFFu)
+          low[u] = bycol ? !((col[s >> 5] >> (s & 31u)) & 1u) : (uint32_t)((col[s] >> kLabBits) <= ax.lo);
       }
       // the lower value goes left: the smaller side's samples are marked
       bool take[kFillU];
@@ -1500,7 +1664,7 @@ __device__ __forceinline__ uint32_t fill_groups(const FitArgs<IdxT, LabT> &a, ui
   return min(J, max(1u, ceil_div(fe - fb, kFillTasksPerGroup)));
 }
 
-template <class IdxT, class LabT>
+template <class IdxT, class LabT, bool kList>
 __global__ __launch_bounds__(kFillThreads) void k_fill_lds(FitArgs<IdxT, LabT> a, uint32_t J) {
   if (a.ctl->err) return;  // a list overflowed: the fit fails, nothing more is read
   extern __shared__ uint32_t lbits[];
@@ -1521,7 +1685,7 @@ __global__ __launch_bounds__(kFillThreads) void k_fill_lds(FitArgs<IdxT, LabT> a
   for (uint32_t k = fb + j * kFillWaves + wave; k < fe; k += Je * kFillWaves) {
     const Task tk = a.fill_tasks[k];
     if (tk.node == kLeaf || tk.chunk >= tk.nch) continue;
-    fill_task_bits(a, tk, lbits, cnt, cur, cur_whole);
+    fill_task_bits<kList>(a, tk, lbits, cnt, cur, cur_whole);
   }
   if (cur != kLeaf) rl_flush(a, cur, cnt, cur_whole);
   __syncthreads();
@@ -1536,7 +1700,7 @@ __global__ __launch_bounds__(kFillThreads) void k_fill_lds(FitArgs<IdxT, LabT> a
 
 // Bitmaps too large for LDS: global atomics into the bitmaps k_select
 // cleared (LDS: the waves' row-free counters).
-template <class IdxT, class LabT>
+template <class IdxT, class LabT, bool kList>
 __global__ __launch_bounds__(kBlock) void k_fill_global(FitArgs<IdxT, LabT> a) {
   if (a.ctl->err) return;  // a list overflowed: the fit fails, nothing more is read
   extern __shared__ uint32_t smem[];
@@ -1547,7 +1711,7 @@ __global__ __launch_bounds__(kBlock) void k_fill_global(FitArgs<IdxT, LabT> a) {
   WAVE_LOOP(a.ctl->n_fill) {
     const Task tk = a.fill_tasks[item];
     if (tk.node == kLeaf || tk.chunk >= tk.nch) continue;
-    fill_task_bits(a, tk, a.bits + (size_t)a.front[tk.node].tree * a.W, cnt, cur, cur_whole);
+    fill_task_bits<kList>(a, tk, a.bits + (size_t)a.front[tk.node].tree * a.W, cnt, cur, cur_whole);
   }
   if (cur != kLeaf) rl_flush(a, cur, cnt, cur_whole);
 }
@@ -1797,12 +1961,16 @@ __device__ __forceinline__ void ctl_next_body(Ctl *ctl, unsigned long long *bslo
   v = wave_sum64(v);
   if (slot == 0 && v) (&ctl->bytes_scan)[kind] += v;
   if (tid == 0) {
-    ctl->q = ctl->c_live;
+    if (ctl->bad) ctl->err |= kErrBadNode;
+    // (after an error no next frontier was written: the later levels stay empty)
+    ctl->q = ctl->err ? 0u : ctl->c_live;
     ctl->n_nodes += ctl->c_ids;
     ctl->n_sub += ctl->c_sub;
     ctl->c_live = 0;
     ctl->c_ids = 0;
     ctl->c_sub = 0;
+    for (uint32_t w = 0; w < 2; ++w)
+      for (uint32_t x = 0; x < kXcd; ++x) ctl->n_wg[w][x] = ctl->wg_next[w][x] = 0;
     // per-level record, so the host can read several levels at once
     const uint32_t d = (ctl->depth + 1) % kLevelRing;
     ctl->depth += 1;

@@ -40,7 +40,7 @@ struct NAux {
   uint32_t rl_pos;                             // best split of the evaluated row-free features:
   uint64_t rl_num, rl_den;                     //   position (zeros - 1), Q numerator / denominator,
   int32_t rl_feat;                             //   feature (-1: none)
-  uint32_t pad;
+  uint32_t lo;                                 // list search: samples of a value index up to lo go left
 };
 constexpr uint32_t kSplit = 1u, kLiveL = 2u, kLiveR = 4u;
 // Set by k_decide on a split node with a live child that stays in the levels
@@ -61,6 +61,7 @@ struct ScanRes {
   uint32_t pos;
   int32_t feat;
   uint32_t ok, pad;
+  uint32_t lo, hi;  // list search: value indices on both sides of the split
 };
 
 // Levels whose frontier size and id count are kept in Ctl.
@@ -86,7 +87,12 @@ struct Ctl {
       bytes_scan_skip;
   // small subtrees: nodes queued so far (whole levels), the next one a
   // subtree wave takes, and the deepest node depth the subtree waves made
-  uint32_t n_sub, sub_next, sub_depth, pad4;
+  uint32_t n_sub, sub_next, sub_depth;
+  uint32_t bad;  // a workgroup's split failed its check: an error at the level's end
+  // list search: tasks of this level's mid and large nodes per class
+  // (appended by the selection) and the next one a workgroup takes; both
+  // start every level at zero
+  uint32_t n_wg[2][kXcd], wg_next[2][kXcd];
   // after level `depth`: frontier size and ids in use, at depth % kLevelRing
   uint32_t lv_q[kLevelRing], lv_nodes[kLevelRing];
 };
@@ -143,6 +149,10 @@ struct Arena {
 // the sample id in the low kIdBits bits and its label in the high bits
 // (N < 2^22, K <= 1,024), so the split scan reads labels with the ids.
 constexpr uint32_t kIdBits = 22, kIdMask = (1u << kIdBits) - 1u;
+// Words of the list search: the sample's distinct-value index in the high
+// bits (below 2^22), its label in the low kLabBits, so that words sort by
+// value and carry the label along.
+constexpr uint32_t kLabBits = 32 - kIdBits, kLabMask = (1u << kLabBits) - 1u;
 
 // fcode[f]: byte offset of feature f's code column (a multiple of 256) and
 // the column kind (0: none, read X_T; 1: bits, 2: u8, 3: u16).
@@ -170,6 +180,16 @@ struct FitArgs {
   // for the children.
   uint32_t Frl, Wsig;       // row-free features, 32-bit signature words per sample
   uint32_t Fr;              // features with rows
+  // List search (a fit that keeps feature 0's row only): a node's samples are
+  // its segment of that row, and the words of an evaluated feature are
+  // gathered from its column of `rank` and sorted in the split search.
+  uint32_t Fc;              // features the split-scan classes are laid over
+  const uint32_t *rank;     // F x N words by sample: value index << kLabBits | label
+  const float *dval;        // distinct values of feature f in ascending order at voff[f]
+  const uint64_t *voff;     // [F]
+  const uint32_t *gapw;     // [F] indices this far apart always pass the candidate test
+  Task *wg_tasks[2];        // mid / large nodes' (node, feature) tasks, kXcd lists of cap_wg each
+  uint32_t cap_wg[2];
   const int32_t *rl_of;     // [F] row-free index of each feature, or -1
   const int32_t *slot_of;   // [F] row slot of each feature, or -1
   const int32_t *row_feat;  // [Fr] feature of each row slot

@@ -129,8 +129,15 @@ typedef struct {
                                 its whole subtree is grown by one wave, every such node of every tree in one
                                 launch after the levels (<= 0, the default: every node stays in the levels).
                                 The trees are identical */
-  int32_t reserved[1];
+  int32_t search;            /* how a batched fit finds its splits: CTA_SEARCH_AUTO (0), CTA_SEARCH_ROWS (1: over
+                                sorted rows of every feature, moved at every level) or CTA_SEARCH_LISTS (2: from
+                                the nodes' sample lists, sorting the features a node evaluates, where the sizes
+                                allow it, else rows); other values are taken as 0.  The trees are identical */
 } cta_fit_opts;
+
+#define CTA_SEARCH_AUTO 0
+#define CTA_SEARCH_ROWS 1
+#define CTA_SEARCH_LISTS 2
 
 #define CTA_HIST_AUTO 0
 #define CTA_HIST_REGS 1

@@ -457,12 +457,19 @@ constexpr uint32_t kLevelGroup = CTA_LEVEL_GROUP;
 constexpr uint32_t kScanChunk = 1024, kReshChunk = 4096, kFillChunk = CTA_FILL_CHUNK;
 
 
+// Workgroup kinds that the nodes of a training set of N samples can need.
+int list_kinds(int32_t N) {
+  const uint32_t n = (uint32_t)N;
+  return n <= kListWave ? 0 : n <= kListWg[0] ? 1 : n <= kListWg[1] ? 2 : 3;
+}
+
 // Whether a fit searches its splits from sample lists (list_kernels.hip)
 // instead of sorted rows; Fr: the rows it would keep.
 bool list_fits(const cta_ctx &ctx, const cta_dataset &ds, const cta_fit_opts &o, uint32_t Fr) {
   if (o.search == CTA_SEARCH_ROWS || o.mode != CTA_MODE_BATCHED || o.all_rows || o.subtree_max > 0) return false;
-  // every node must fit a workgroup's sort, and its class counts the LDS left
-  if ((uint32_t)ds.N > kListWg[1] || (size_t)list_wg_words(1, (uint32_t)ds.K) * 4 > ctx.lds_per_block) return false;
+  // the words or the sample set of a node and its class counts must fit the LDS
+  for (int w = 0; w < list_kinds(ds.N); ++w)
+    if ((size_t)list_wg_words(w, (uint32_t)ds.K, (uint32_t)ds.N) * 4 > ctx.lds_per_block) return false;
   if (o.search == CTA_SEARCH_LISTS) return true;
   // Rows move Fr rows per level where lists sort max_features of them, but a
   // node's sort takes one workgroup where rows split it into chunks.  Rows /
@@ -523,7 +530,7 @@ struct Fitter {
   uint32_t sub_max;  // small-subtree threshold of batched fits (0: none)
   bool list;         // list search: only feature 0's row is kept
   uint32_t Fc = 0;   // features the split-scan classes are laid over
-  uint32_t Glist = 0, Gwg[2] = {0, 0};  // blocks of k_list_scan and k_list_wg
+  uint32_t Glist = 0, Gwg[kWgKinds] = {};  // blocks of k_list_scan and k_list_wg
   hipStream_t st;
   uint32_t G;      // blocks of the wave-loop kernels
   uint32_t Gscan;  // blocks of k_scan: all resident at once, a multiple of kXcd
@@ -574,11 +581,13 @@ struct Fitter {
         HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k, threads, lds));
         return std::max<uint32_t>(kXcd, (uint32_t)(ctx->num_cu * std::max(b, 1)) / kXcd * kXcd);
       };
-      const void *wg[2] = {scan_regs ? (const void *)k_list_wg<IdxT, LabT, 0, true> : (const void *)k_list_wg<IdxT, LabT, 0, false>,
-                           scan_regs ? (const void *)k_list_wg<IdxT, LabT, 1, true> : (const void *)k_list_wg<IdxT, LabT, 1, false>};
-      for (int w = 0; w < 2; ++w) {
+      const void *wg[kWgKinds] = {
+          scan_regs ? (const void *)k_list_wg<IdxT, LabT, 0, true> : (const void *)k_list_wg<IdxT, LabT, 0, false>,
+          scan_regs ? (const void *)k_list_wg<IdxT, LabT, 1, true> : (const void *)k_list_wg<IdxT, LabT, 1, false>,
+          scan_regs ? (const void *)k_list_wg<IdxT, LabT, 2, true> : (const void *)k_list_wg<IdxT, LabT, 2, false>};
+      for (int w = 0; w < list_kinds(N); ++w) {
         HIPC(hipFuncSetAttribute(wg[w], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_per_block));
-        Gwg[w] = grid(wg[w], kListWaves[w] * kWave, list_wg_words(w, (uint32_t)K) * 4);
+        Gwg[w] = grid(wg[w], kListWaves[w] * kWave, wg_lds(w));
       }
       Glist = grid(scan_regs ? (const void *)k_list_scan<IdxT, LabT, true> : (const void *)k_list_scan<IdxT, LabT, false>,
                    kBlock, list_lds());
@@ -589,6 +598,8 @@ struct Fitter {
   // side bitmap, then each wave's row-free counters
   size_t fill_lds_bytes() const { return (((size_t)N + 31) / 32) * 4 + (size_t)kFillWaves * Frl * K * 4; }
 
+  // bytes of LDS of a list workgroup; the kinds a training set of N can need
+  size_t wg_lds(int w) const { return (size_t)list_wg_words(w, (uint32_t)K, (uint32_t)N) * 4; }
   size_t list_lds() const { return (size_t)kWavesPerBlock * list_wave_words((uint32_t)K, scan_regs) * 4; }
 
   size_t smem() const { return (size_t)kWavesPerBlock * 2 * K * sizeof(uint32_t); }
@@ -644,9 +655,10 @@ struct Fitter {
     const uint64_t cap_small = cap_q + 2ull * Fr * n_tot / Cr + 64;
     const uint64_t cap_fill = cap_q + n_tot / Cf + 64;
     const uint64_t cap_hist = (uint64_t)m * K * ((list ? n_tot / kListWave : 2 * n_tot / Cs) + 64);
-    // (node, feature) tasks of nodes of more than kListWave / kListWg[0] samples
-    const uint64_t cap_wg[2] = {list ? (uint64_t)m * (n_tot / kListWave) + 64 : 0,
-                                list ? (uint64_t)m * (n_tot / kListWg[0]) + 64 : 0};
+    // (node, feature) tasks of nodes of more than kListWave / kListWg[0] / kListWg[1] samples
+    const uint64_t cap_wg[kWgKinds] = {list ? (uint64_t)m * (n_tot / kListWave) + 64 : 0,
+                                       list ? (uint64_t)m * (n_tot / kListWg[0]) + 64 : 0,
+                                       list ? (uint64_t)m * (n_tot / kListWg[1]) + 64 : 0};
     if (cap_scan > 0xFFFFFFF0ull || cap_small > 0xFFFFFFF0ull || cap_big > 0xFFFFFFF0ull ||
         cap_nodes > 0xFFFFFFF0ull || cap_hist > 0xFFFFFFF0ull || cap_wg[0] > 0xFFFFFFF0ull)
       fail(CTA_EUNSUPPORTED, "batch of %d trees too large for 32-bit task indices", Tb);
@@ -705,8 +717,8 @@ struct Fitter {
       a.dval = ds->dval.as<float>();
       a.voff = ds->voff.as<uint64_t>();
       a.gapw = ds->gapw.as<uint32_t>();
-      for (int w = 0; w < 2; ++w) {
-        a.wg_tasks[w] = ctx->ws_as<Task>(w ? "wg_tasks1" : "wg_tasks0", cap_wg[w] * kXcd);
+      for (int w = 0; w < kWgKinds; ++w) {
+        a.wg_tasks[w] = ctx->ws_as<Task>("wg_tasks" + std::to_string(w), cap_wg[w] * kXcd);
         a.cap_wg[w] = (uint32_t)cap_wg[w];
       }
     }
@@ -1139,13 +1151,19 @@ struct Fitter {
   // The level's split scans from the nodes' sample lists, large nodes first.
   template <bool kRegs>
   void list_scan_k(const FitArgs<IdxT, LabT> &a) {
-    {
-      Timed tm(ctx, "k_list_big");
-      k_list_wg<IdxT, LabT, 1, kRegs><<<Gwg[1], kListWaves[1] * kWave, list_wg_words(1, (uint32_t)K) * 4, st>>>(a);
+    // (only the kinds that a node of this training set can need)
+    const int kinds = list_kinds(N);
+    if (kinds > 2) {
+      Timed tm(ctx, "k_list_filter");
+      k_list_wg<IdxT, LabT, 2, kRegs><<<Gwg[2], kListWaves[2] * kWave, wg_lds(2), st>>>(a);
     }
-    {
+    if (kinds > 1) {
+      Timed tm(ctx, "k_list_big");
+      k_list_wg<IdxT, LabT, 1, kRegs><<<Gwg[1], kListWaves[1] * kWave, wg_lds(1), st>>>(a);
+    }
+    if (kinds > 0) {
       Timed tm(ctx, "k_list_mid");
-      k_list_wg<IdxT, LabT, 0, kRegs><<<Gwg[0], kListWaves[0] * kWave, list_wg_words(0, (uint32_t)K) * 4, st>>>(a);
+      k_list_wg<IdxT, LabT, 0, kRegs><<<Gwg[0], kListWaves[0] * kWave, wg_lds(0), st>>>(a);
     }
     Timed tm(ctx, "k_scan");
     k_list_scan<IdxT, LabT, kRegs><<<Glist, kBlock, list_lds(), st>>>(a);

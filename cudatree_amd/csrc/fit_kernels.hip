@@ -258,10 +258,12 @@ __global__ __launch_bounds__(kOffThreads) void k_off_apply(const uint32_t *v, co
 }
 
 // Node sizes of the list search: up to kListWave samples one wave sorts a
-// feature's words, up to kListWg[0] / kListWg[1] a workgroup of 4 / 16 waves.
+// feature's words, up to kListWg[0] / kListWg[1] a workgroup of 4 / 16 waves;
+// larger nodes are filtered from the presorted row.
 constexpr uint32_t kListE = 16, kListWave = kWave * kListE;
 constexpr uint32_t kListWg[2] = {4096, 32768};
-constexpr int kListWaves[2] = {4, 16};
+constexpr int kListWaves[kWgKinds] = {4, 16, 16};
+__device__ __forceinline__ int list_kind(uint32_t n) { return n <= kListWg[0] ? 0 : n <= kListWg[1] ? 1 : 2; }
 
 // ------------------------------------------------------------------------
 // k_select: visiting order of every frontier node, its task and slot counts
@@ -501,8 +503,9 @@ __global__ __launch_bounds__(kBlock) void k_select_emit(FitArgs<IdxT, LabT> a) {
     // items: features of a multi-chunk node (nch tasks each), else tasks
     const uint32_t nitem = nch > 1 ? nf : ntask;
     if (kList && nch > 1) {
-      const int wg = a.front[i].n > kListWg[0] ? 1 : 0;
-      const uint32_t cap = a.cap_wg[wg];
+      const int wg = list_kind(a.front[i].n);
+      const uint32_t cap = wg == 0 ? a.cap_wg[0] : wg == 1 ? a.cap_wg[1] : a.cap_wg[2];
+      Task *tasks = wg == 0 ? a.wg_tasks[0] : wg == 1 ? a.wg_tasks[1] : a.wg_tasks[2];
       bool over = false;
       for (uint32_t c0 = 0; c0 < nf; c0 += kWave) {
         const uint32_t it = c0 + lane;
@@ -515,7 +518,7 @@ __global__ __launch_bounds__(kBlock) void k_select_emit(FitArgs<IdxT, LabT> a) {
           if (lane == lead) p = atomicAdd(&a.ctl->n_wg[wg][x], (uint32_t)__popcll(mk));
           p = readlane(p, lead) + mbcnt(mk);
           if (c == x) {
-            if (p < cap) a.wg_tasks[wg][(size_t)x * cap + p] = Task{i, it | (1u << 16), 0u, 1u};
+            if (p < cap) tasks[(size_t)x * cap + p] = Task{i, it | (1u << 16), 0u, 1u};
             else over = true;
           }
         }
@@ -1969,7 +1972,7 @@ __device__ __forceinline__ void ctl_next_body(Ctl *ctl, unsigned long long *bslo
     ctl->c_live = 0;
     ctl->c_ids = 0;
     ctl->c_sub = 0;
-    for (uint32_t w = 0; w < 2; ++w)
+    for (int w = 0; w < kWgKinds; ++w)
       for (uint32_t x = 0; x < kXcd; ++x) ctl->n_wg[w][x] = ctl->wg_next[w][x] = 0;
     // per-level record, so the host can read several levels at once
     const uint32_t d = (ctl->depth + 1) % kLevelRing;

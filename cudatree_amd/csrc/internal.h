@@ -72,6 +72,10 @@ constexpr uint32_t kLevelRing = 64;
 // on class b % 8, so the value gathers of a column hit few L2s.
 constexpr uint32_t kXcd = 8;
 
+// Kinds of workgroup tasks of the list search: by the node's size, sorted by 4
+// or 16 waves, or filtered from the presorted row.
+constexpr int kWgKinds = 3;
+
 // Counters of one level, in device memory.  Nothing is allocated with
 // atomics: the totals are written by the offset scans over the frontier.
 struct Ctl {
@@ -89,10 +93,10 @@ struct Ctl {
   // subtree wave takes, and the deepest node depth the subtree waves made
   uint32_t n_sub, sub_next, sub_depth;
   uint32_t bad;  // a workgroup's split failed its check: an error at the level's end
-  // list search: tasks of this level's mid and large nodes per class
+  // list search: workgroup tasks of this level per kind and class
   // (appended by the selection) and the next one a workgroup takes; both
   // start every level at zero
-  uint32_t n_wg[2][kXcd], wg_next[2][kXcd];
+  uint32_t n_wg[kWgKinds][kXcd], wg_next[kWgKinds][kXcd];
   // after level `depth`: frontier size and ids in use, at depth % kLevelRing
   uint32_t lv_q[kLevelRing], lv_nodes[kLevelRing];
 };
@@ -188,8 +192,8 @@ struct FitArgs {
   const float *dval;        // distinct values of feature f in ascending order at voff[f]
   const uint64_t *voff;     // [F]
   const uint32_t *gapw;     // [F] indices this far apart always pass the candidate test
-  Task *wg_tasks[2];        // mid / large nodes' (node, feature) tasks, kXcd lists of cap_wg each
-  uint32_t cap_wg[2];
+  Task *wg_tasks[kWgKinds];  // (node, feature) tasks by kind, kXcd lists of cap_wg each
+  uint32_t cap_wg[kWgKinds];
   const int32_t *rl_of;     // [F] row-free index of each feature, or -1
   const int32_t *slot_of;   // [F] row slot of each feature, or -1
   const int32_t *row_feat;  // [Fr] feature of each row slot

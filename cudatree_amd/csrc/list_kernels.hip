@@ -21,6 +21,9 @@
 //   up to kListWave           one wave, sorted in its registers   (k_list_scan)
 //   up to kListWg[0], [1]     one workgroup of 4 / 16 waves, sorted in
 //                             registers and LDS                   (k_list_wg)
+//   more                      one workgroup of 16 waves streams the feature's
+//                             presorted row of all N samples and keeps the
+//                             node's                              (k_list_wg)
 #include "device_util.h"
 #include "internal.h"
 
@@ -204,6 +207,8 @@ __device__ __forceinline__ void lane_masks(uint32_t (&M)[6]) {
 // the comparisons stay exact.
 struct Small {  // n <= 1,024: num < 2^31, den < 2^19, products in 64 bits
   using Num = uint32_t;
+  using Den = uint32_t;
+  using Sum = uint32_t;
   static __device__ __forceinline__ int cmp(uint32_t n1, uint32_t d1, uint32_t n2, uint32_t d2) {
     const uint64_t a = (uint64_t)n1 * d2, b = (uint64_t)n2 * d1;
     return a > b ? 1 : a < b ? -1 : 0;
@@ -211,6 +216,8 @@ struct Small {  // n <= 1,024: num < 2^31, den < 2^19, products in 64 bits
 };
 struct Mid {  // n <= 32,768: num < 2^46, den <= 2^28, products in 96 bits
   using Num = uint64_t;
+  using Den = uint32_t;
+  using Sum = uint32_t;
   static __device__ __forceinline__ int cmp(uint64_t n1, uint32_t d1, uint64_t n2, uint32_t d2) {
     const uint64_t al = (n1 & 0xFFFFFFFFull) * d2, bl = (n2 & 0xFFFFFFFFull) * d1;
     const uint64_t ah = (n1 >> 32) * d2 + (al >> 32), bh = (n2 >> 32) * d1 + (bl >> 32);
@@ -220,11 +227,21 @@ struct Mid {  // n <= 32,768: num < 2^46, den <= 2^28, products in 96 bits
   }
 };
 
+struct Large {  // any node: products in 128 bits
+  using Num = uint64_t;
+  using Den = uint64_t;
+  using Sum = uint64_t;
+  static __device__ __forceinline__ int cmp(uint64_t n1, uint64_t d1, uint64_t n2, uint64_t d2) {
+    return q_cmp(n1, d1, n2, d2);
+  }
+};
+
 // A lane's best split so far (num = 0: none; a split's num is positive).
 template <class A>
 struct Best {
   typename A::Num num = 0;
-  uint32_t den = 1, pos = 0;
+  typename A::Den den = 1;
+  uint32_t pos = 0;
   int32_t feat = 0x7FFFFFFF;
   uint32_t lo = 0, hi = 0;  // value indices on both sides
 };
@@ -237,14 +254,22 @@ __device__ __forceinline__ bool beats(const Best<A> &a, const Best<A> &b) {
   return a.pos < b.pos;
 }
 
+template <class T>
+__device__ __forceinline__ T readlane_of(T v, uint32_t lane) {
+  if constexpr (sizeof(T) == 8) return (uint64_t)readlane((uint32_t)(v >> 32), lane) << 32 | readlane((uint32_t)v, lane);
+  else return readlane(v, lane);
+}
+template <int kCtrl, int kRowMask, class T>
+__device__ __forceinline__ T dpp_of(T v) {
+  if constexpr (sizeof(T) == 8) return Move64{}.template operator()<kCtrl, kRowMask>(v);
+  else return dpp<kCtrl, kRowMask>(v);
+}
+
 template <class A>
 __device__ __forceinline__ Best<A> shfl_best(const Best<A> &b, uint32_t lane) {
   Best<A> r;
-  if constexpr (sizeof(typename A::Num) == 8)
-    r.num = (uint64_t)readlane((uint32_t)(b.num >> 32), lane) << 32 | readlane((uint32_t)b.num, lane);
-  else
-    r.num = readlane(b.num, lane);
-  r.den = readlane(b.den, lane);
+  r.num = readlane_of(b.num, lane);
+  r.den = readlane_of(b.den, lane);
   r.pos = readlane(b.pos, lane);
   r.feat = (int32_t)readlane((uint32_t)b.feat, lane);
   r.lo = readlane(b.lo, lane);
@@ -256,9 +281,8 @@ struct MoveBest {
   template <int kCtrl, int kRowMask, class A>
   static __device__ __forceinline__ Best<A> move(const Best<A> &b) {
     Best<A> r;
-    if constexpr (sizeof(typename A::Num) == 8) r.num = Move64{}.template operator()<kCtrl, kRowMask>(b.num);
-    else r.num = dpp<kCtrl, kRowMask>(b.num);
-    r.den = dpp<kCtrl, kRowMask>(b.den);  // a lane without a source reads num = 0: beaten by any split
+    r.num = dpp_of<kCtrl, kRowMask>(b.num);  // a lane without a source reads num = 0: beaten by any split
+    r.den = dpp_of<kCtrl, kRowMask>(b.den);
     r.pos = dpp<kCtrl, kRowMask>(b.pos);
     r.feat = (int32_t)dpp<kCtrl, kRowMask>((uint32_t)b.feat);
     r.lo = dpp<kCtrl, kRowMask>(b.lo);
@@ -282,6 +306,10 @@ __device__ __forceinline__ Best<A> wave_best_of(Best<A> b) {
   return shfl_best(b, kWave - 1);
 }
 
+__device__ __forceinline__ uint32_t label_bits(uint32_t K) {
+  return K > 1 ? 32u - (uint32_t)__builtin_clz(K - 1u) : 1u;
+}
+
 // What a feature's split scan needs besides its sorted words: adjacent words
 // are a candidate when their value indices differ by gapw or more, or differ
 // and the values pass the candidate test.
@@ -299,23 +327,25 @@ __device__ __forceinline__ bool splits(const FeatVals &fv, uint32_t i, uint32_t 
   return d >= fv.gapw || gap_ok(fv.v[i], fv.v[j]);
 }
 
-// Scan of the sorted words w[p0, p1) (LDS) of a node of n samples: the class
-// counts before p0 in cv (kRegs: lane k holds class k) or carry[] (LDS), the
-// class totals in tv / tot[], SL = sum c^2 and D = sum t c at p0, T2 = sum
-// t^2.  `after`: the word at p1, when p1 < n.  A node of at most 32,768
-// samples keeps these sums below 2^32.
+// The split scan of a node of n samples over one feature's words in ascending
+// order, 64 positions at a time: the class counts before the next position in
+// cv (kRegs: lane k holds class k) or carry[] (LDS), the class totals in tv /
+// tot[], SL = sum c^2 and D = sum t c before it, T2 = sum t^2.  (A node of at
+// most 32,768 samples keeps these sums below 2^32.)
 template <class A, bool kRegs>
-__device__ __forceinline__ void scan_words(const uint32_t *w, uint32_t p0, uint32_t p1, uint32_t n, uint32_t after,
-                                           uint32_t nbits, uint32_t &cv, uint32_t tv, uint32_t *carry,
-                                           const uint32_t *tot, uint32_t SL, uint32_t D, uint32_t T2, int32_t f,
-                                           const FeatVals &fv, Best<A> &best) {
-  using Num = typename A::Num;
-  const uint32_t lane = lane_id();
-  for (uint32_t pb = p0; pb < p1; pb += kWave) {
-    const uint32_t p = pb + lane;
-    const bool valid = p < p1;
-    const uint32_t x = w[min(p, p1 - 1u)];
-    uint32_t y = p + 1u < p1 ? w[p + 1u] : after;
+struct Scan {
+  using Sum = typename A::Sum;
+  uint32_t n, nbits;
+  uint32_t cv, tv;
+  uint32_t *carry;
+  const uint32_t *tot;
+  Sum SL, D, T2;
+  int32_t f;
+  FeatVals fv;
+
+  // Lane l's position p holds word x, the next one y (lanes with `valid` set).
+  __device__ __forceinline__ void tile(uint32_t x, uint32_t y, bool valid, uint32_t p, Best<A> &best) {
+    const uint32_t lane = lane_id();
     const uint32_t lab = x & kLabMask, i = x >> kLabBits, j = y >> kLabBits;
     // earlier lanes with the same label, and the label's total
     uint32_t cprev = 0, dD = 0;
@@ -349,15 +379,15 @@ __device__ __forceinline__ void scan_words(const uint32_t *w, uint32_t p0, uint3
     }
     const uint32_t iS = wave_incl_scan(valid ? 2u * cprev + 1u : 0u);
     const uint32_t iD = wave_incl_scan(dD);
-    const uint32_t SLp = SL + iS, Dp = D + iD;
+    const Sum SLp = SL + iS, Dp = D + iD;
     SL += readlane(iS, kWave - 1);
     D += readlane(iD, kWave - 1);
     if (valid && p + 1u < n && splits(fv, i, j)) {
-      const uint32_t nL = p + 1u, nR = n - nL, SR = T2 + SLp - 2u * Dp;
-      Num num;
-      if constexpr (sizeof(Num) == 4) num = SLp * nR + SR * nL;
-      else num = (uint64_t)SLp * nR + (uint64_t)SR * nL;
-      const uint32_t den = nL * nR;
+      const uint32_t nL = p + 1u, nR = n - nL;
+      const Sum SR = T2 + SLp - 2u * Dp;
+      using Num = typename A::Num;
+      const Num num = (Num)SLp * nR + (Num)SR * nL;
+      const typename A::Den den = (typename A::Den)nL * nR;
       const int c = A::cmp(num, den, best.num, best.den);
       // (positions rise within a feature, so an equal score stays with the
       // earlier one; another feature's wins with the lower id)
@@ -371,7 +401,17 @@ __device__ __forceinline__ void scan_words(const uint32_t *w, uint32_t p0, uint3
       }
     }
   }
-}
+
+  // Positions [p0, p1) of the sorted words w (LDS); `after`: the word at p1,
+  // when p1 < n.
+  __device__ __forceinline__ void words(const uint32_t *w, uint32_t p0, uint32_t p1, uint32_t after, Best<A> &best) {
+    for (uint32_t pb = p0; pb < p1; pb += kWave) {
+      const uint32_t p = pb + lane_id();
+      const uint32_t x = w[min(p, p1 - 1u)], y = p + 1u < p1 ? w[p + 1u] : after;
+      tile(x, y, p < p1, p, best);
+    }
+  }
+};
 
 template <class A>
 __device__ __forceinline__ ScanRes to_res(const Best<A> &b) {
@@ -385,10 +425,6 @@ __device__ __forceinline__ ScanRes to_res(const Best<A> &b) {
   r.lo = b.lo;
   r.hi = b.hi;
   return r;
-}
-
-__device__ __forceinline__ uint32_t label_bits(uint32_t K) {
-  return K > 1 ? 32u - (uint32_t)__builtin_clz(K - 1u) : 1u;
 }
 
 // ---- small nodes: one wave -------------------------------------------------------
@@ -432,8 +468,8 @@ __device__ __forceinline__ void list_features(const FitArgs<IdxT, LabT> &a, cons
     if constexpr (!kRegs)
       for (uint32_t c = lane; c < K; c += kWave) carry[c] = 0;
     wave_sync();
-    uint32_t cv = 0;
-    scan_words<Small, kRegs>(w, 0, n, n, 0u, nbits, cv, tv, carry, tot, 0u, 0u, T2, (int32_t)f, feat_vals(a, f), best);
+    Scan<Small, kRegs> sc = {n, nbits, 0u, tv, carry, tot, 0u, 0u, T2, (int32_t)f, feat_vals(a, f)};
+    sc.words(w, 0, n, 0u, best);
     f = fn;
   }
 }
@@ -482,12 +518,18 @@ __global__ __launch_bounds__(kBlock) void k_list_scan(FitArgs<IdxT, LabT> a) {
 }
 
 // ---- larger nodes: one workgroup -------------------------------------------------
-// kWg = 0: 4 waves, up to 4,096 samples; kWg = 1: 16 waves, up to 32,768.
-// LDS: the words, (W + 1) x K class counts (per wave, totals), then the
-// waves' best splits and first words.
-__host__ __device__ __forceinline__ uint32_t list_wg_words(int wg, uint32_t K) {
-  const uint32_t W = wg ? 16u : 4u;
-  return (wg ? 32768u : 4096u) + (W + 1u) * K + W * 8u + 8u;
+// kWg = 0: 4 waves, up to 4,096 samples; kWg = 1: 16 waves, up to 32,768;
+// kWg = 2: 16 waves, any size, from the presorted row.
+// LDS: the words (kWg = 2: the node's sample set as N bits, then a queue of
+// kQueue words per wave), (W + 1) x K class counts (per wave, totals), the
+// waves' results of 8 words each, the next task.
+constexpr uint32_t kQueue = 2 * kWave;
+__host__ __device__ __forceinline__ uint32_t list_body_words(int wg, uint32_t N) {
+  return wg == 0 ? kListWg[0] : wg == 1 ? kListWg[1] : (N + 31u) / 32u + (uint32_t)kListWaves[2] * kQueue;
+}
+__host__ __device__ __forceinline__ uint32_t list_wg_words(int wg, uint32_t K, uint32_t N) {
+  const uint32_t W = (uint32_t)kListWaves[wg];
+  return list_body_words(wg, N) + (W + 1u) * K + W * 8u + 8u;
 }
 
 // The words of the node's samples in ascending order into `w` (W x E x 64
@@ -538,6 +580,120 @@ __device__ __forceinline__ void wg_sort(const IdxT *list, uint32_t n, const uint
   __syncthreads();
 }
 
+// The waves' class counts in cnt[W][K] become each wave's starting counts.
+template <int W>
+__device__ __forceinline__ void wg_prefix(uint32_t *cnt, uint32_t K) {
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < K; k += W * kWave) {
+    uint32_t run = 0;
+    for (int v = 0; v < W; ++v) {
+      const uint32_t c = cnt[v * K + k];
+      cnt[v * K + k] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+}
+
+// Adds the labels of the lanes with `valid` set to the wave's counts (those
+// of one label by its last lane).
+__device__ __forceinline__ void count_labels(uint32_t *own, uint32_t lab, bool valid, uint32_t nbits) {
+  uint64_t same = ballot(valid);
+  for (uint32_t b = 0; b < nbits; ++b) {
+    const uint32_t bit = (lab >> b) & 1u;
+    const uint64_t mb = ballot(bit != 0u);
+    same &= bit ? mb : ~mb;
+  }
+  if (valid && (same >> lane_id()) == 1ull) own[lab] += (uint32_t)__popcll(same);
+  wave_sync();
+}
+
+// The wave's scan state at its starting counts `own`; returns the samples
+// before it.
+template <class A, bool kRegs>
+__device__ __forceinline__ uint32_t scan_start(Scan<A, kRegs> &sc, uint32_t *own, const uint32_t *tot, uint32_t K,
+                                               uint32_t n, uint32_t f, const FeatVals &fv) {
+  const uint32_t lane = lane_id();
+  uint64_t sl = 0, dd = 0, t2 = 0;
+  uint32_t before = 0, cv = 0, tv = 0;
+  for (uint32_t k = lane; k < K; k += kWave) {
+    const uint32_t c = own[k], t = tot[k];
+    if (kRegs) {
+      cv = c;
+      tv = t;
+    }
+    before += c;
+    sl += (uint64_t)c * c;
+    dd += (uint64_t)t * c;
+    t2 += (uint64_t)t * t;
+  }
+  using Sum = typename A::Sum;
+  if constexpr (sizeof(Sum) == 8) {
+    sc.SL = wave_sum64(sl);
+    sc.D = wave_sum64(dd);
+    sc.T2 = wave_sum64(t2);
+  } else {
+    sc.SL = wave_sum32((uint32_t)sl);
+    sc.D = wave_sum32((uint32_t)dd);
+    sc.T2 = wave_sum32((uint32_t)t2);
+  }
+  sc.n = n;
+  sc.nbits = label_bits(K);
+  sc.cv = cv;
+  sc.tv = tv;
+  sc.carry = own;
+  sc.tot = tot;
+  sc.f = (int32_t)f;
+  sc.fv = fv;
+  wave_sync();
+  return wave_sum32(before);
+}
+
+// Entry of a wave's best split in the waves' results: num, den, pos, lo, hi.
+template <class A>
+__device__ __forceinline__ void put_best(uint32_t *t, const Best<A> &b) {
+  t[0] = (uint32_t)b.num;
+  t[1] = (uint32_t)((uint64_t)b.num >> 32);
+  t[2] = (uint32_t)b.den;
+  t[3] = (uint32_t)((uint64_t)b.den >> 32);
+  t[4] = b.pos;
+  t[5] = b.lo;
+  t[6] = b.hi;
+}
+
+// The wave with the best entry (positions rise with the waves, so an equal
+// score stays with the earlier one); W: none.
+template <class A, int W>
+__device__ __forceinline__ uint32_t best_entry(const uint32_t *tail) {
+  uint32_t win = W;
+  uint64_t wnum = 0, wden = 1;
+#pragma unroll 1
+  for (uint32_t v = 0; v < (uint32_t)W; ++v) {
+    const uint64_t num = (uint64_t)tail[v * 8u + 1u] << 32 | tail[v * 8u];
+    const uint64_t den = (uint64_t)tail[v * 8u + 3u] << 32 | tail[v * 8u + 2u];
+    if (A::cmp((typename A::Num)num, (typename A::Den)den, (typename A::Num)wnum, (typename A::Den)wden) > 0) {
+      win = v;
+      wnum = num;
+      wden = den;
+    }
+  }
+  return uniform(win);
+}
+
+// Result entry of a task: the entry t of the winning wave, or none.
+__device__ __forceinline__ void put_res(ScanRes *res, const uint32_t *t, uint32_t f, bool found) {
+  ScanRes r;
+  r.num = found ? (uint64_t)t[1] << 32 | t[0] : 0ull;
+  r.den = found ? (uint64_t)t[3] << 32 | t[2] : 1ull;
+  r.pos = t[4];
+  r.feat = (int32_t)f;
+  r.ok = found ? 1u : 0u;
+  r.pad = 0;
+  r.lo = t[5];
+  r.hi = t[6];
+  *res = r;
+}
+
 // Split scan of the n sorted words in LDS: every wave takes 64 E of them, its
 // starting class counts from the counts of the waves before it.  Writes the
 // result entry and the left class counts of the best split (left[0, K)).
@@ -551,94 +707,30 @@ __device__ __forceinline__ void wg_scan(const FitArgs<IdxT, LabT> &a, uint32_t n
   uint32_t *own = cnt + wave * K;
   for (uint32_t c = threadIdx.x; c < W * K; c += W * kWave) cnt[c] = 0;
   __syncthreads();
-  // the wave's class counts: lanes with the same label added by the last of them
   for (uint32_t pb = p0; pb < p1; pb += kWave) {
-    const uint32_t p = pb + lane, lab = w[min(p, p1 - 1u)] & kLabMask;
-    uint64_t same = ballot(p < p1);
-    for (uint32_t b = 0; b < nbits; ++b) {
-      const uint32_t bit = (lab >> b) & 1u;
-      const uint64_t mb = ballot(bit != 0u);
-      same &= bit ? mb : ~mb;
-    }
-    if (p < p1 && (same >> lane) == 1ull) own[lab] += (uint32_t)__popcll(same);
-    wave_sync();
+    const uint32_t p = pb + lane;
+    count_labels(own, w[min(p, p1 - 1u)] & kLabMask, p < p1, nbits);
   }
-  __syncthreads();
-  for (uint32_t k = threadIdx.x; k < K; k += W * kWave) {
-    uint32_t run = 0;
-    for (int v = 0; v < W; ++v) {
-      const uint32_t c = cnt[v * K + k];
-      cnt[v * K + k] = run;
-      run += c;
-    }
-  }
-  __syncthreads();
-  uint32_t sl = 0, dd = 0, t2 = 0, cv = 0, tv = 0;
-  for (uint32_t k = lane; k < K; k += kWave) {
-    const uint32_t c = own[k], t = tot[k];
-    if (kRegs) {
-      cv = c;
-      tv = t;
-    }
-    sl += c * c;
-    dd += t * c;
-    t2 += t * t;
-  }
-  const uint32_t SL = wave_sum32(sl), D = wave_sum32(dd), T2 = wave_sum32(t2);
-  wave_sync();
+  wg_prefix<W>(cnt, K);
+  Scan<Mid, kRegs> sc;
+  scan_start(sc, own, tot, K, n, f, feat_vals(a, f));
   Best<Mid> best;
-  if (p0 < p1)
-    scan_words<Mid, kRegs>(w, p0, p1, n, p1 < n ? w[p1] : 0u, nbits, cv, tv, own, tot, SL, D, T2, (int32_t)f,
-                           feat_vals(a, f), best);
-  if (kRegs && lane < K) own[lane] = cv;  // the counts at the end of the chunk, as in LDS
+  if (p0 < p1) sc.words(w, p0, p1, p1 < n ? w[p1] : 0u, best);
+  if (kRegs && lane < K) own[lane] = sc.cv;  // the counts at the end of the chunk, as in LDS
   best = wave_best_of(best);
-  // tail: per wave {num lo, num hi, den, pos, lo, hi}
-  if (lane == 0) {
-    uint32_t *t = tail + wave * 8u;
-    t[0] = (uint32_t)best.num;
-    t[1] = (uint32_t)(best.num >> 32);
-    t[2] = best.den;
-    t[3] = best.pos;
-    t[4] = best.lo;
-    t[5] = best.hi;
-  }
+  if (lane == 0) put_best(tail + wave * 8u, best);
   __syncthreads();
-  // the winning wave (positions rise with the waves, so an equal score stays
-  // with the earlier one); its split's fields are then read from its entry
-  uint32_t win = W, wden = 1;
-  uint64_t wnum = 0;
-#pragma unroll 1
-  for (uint32_t v = 0; v < (uint32_t)W; ++v) {
-    const uint64_t num = (uint64_t)tail[v * 8u + 1u] << 32 | tail[v * 8u];
-    const uint32_t den = tail[v * 8u + 2u];
-    if (Mid::cmp(num, den, wnum, wden) > 0) {
-      win = v;
-      wnum = num;
-      wden = den;
-    }
-  }
-  win = uniform(win);
+  const uint32_t win = best_entry<Mid, W>(tail);
   bool found = win < (uint32_t)W;
   const uint32_t *t = tail + (found ? win : 0u) * 8u;
-  const uint32_t pos = t[3];
+  const uint32_t pos = t[4];
   if (found) {
     // the entry has to name the words at the split: the sides of the samples
     // follow from its indices, the children's sizes from its position
-    found = pos + 1u < n && w[min(pos, n - 1u)] >> kLabBits == t[4] && w[min(pos + 1u, n - 1u)] >> kLabBits == t[5];
+    found = pos + 1u < n && w[min(pos, n - 1u)] >> kLabBits == t[5] && w[min(pos + 1u, n - 1u)] >> kLabBits == t[6];
     if (!found && threadIdx.x == 0) a.ctl->bad = 1u;
   }
-  if (threadIdx.x == 0) {
-    ScanRes r;
-    r.num = found ? wnum : 0u;
-    r.den = wden;
-    r.pos = pos;
-    r.feat = (int32_t)f;
-    r.ok = found ? 1u : 0u;
-    r.pad = 0;
-    r.lo = t[4];
-    r.hi = t[5];
-    *res = r;
-  }
+  if (threadIdx.x == 0) put_res(res, t, f, found);
   if (!found) return;  // (the whole workgroup)
   // left class counts: those before the winning wave's chunk (where the wave
   // before it ended) and the chunk's words up to the split
@@ -648,6 +740,133 @@ __device__ __forceinline__ void wg_scan(const FitArgs<IdxT, LabT> &a, uint32_t n
   for (uint32_t p = win * C + threadIdx.x; p <= pos; p += W * kWave) atomicAdd(&acc[w[p] & kLabMask], 1u);
   __syncthreads();
   for (uint32_t k = threadIdx.x; k < K; k += W * kWave) left[k] = acc[k];
+}
+
+// Split scan of a node of any size: the waves stream equal shares of the
+// feature's presorted row of all N samples and keep the node's, whose set is
+// in LDS as N bits.  Twice: for the waves' class counts, then for the scan,
+// which takes 64 kept words at a time from a queue of the wave.  Streaming
+// costs about 50 VALU instructions per 64 row entries whether they are kept
+// or not, the scan about 250 per 64 kept, so it pays while a node holds more
+// than a small share of the samples: 200,000 x 256, 200 trees, nodes above
+// 32,768 samples (30% of the evaluated elements) 38 ms where moving their
+// rows took 60 and scanning them 30.
+template <int W, bool kRegs, class IdxT, class LabT>
+__device__ __forceinline__ void wg_filter(const FitArgs<IdxT, LabT> &a, const IdxT *list, uint32_t n, uint32_t f,
+                                          uint32_t *set, uint32_t *cnt, const uint32_t *tot, uint32_t *tail,
+                                          ScanRes *res, uint32_t *left) {
+  const uint32_t lane = lane_id(), wave = uniform(threadIdx.x / kWave), K = (uint32_t)a.K, N = (uint32_t)a.N;
+  const uint32_t nbits = label_bits(K), Wb = (N + 31u) / 32u;
+  const IdxT *row = a.si0 + (size_t)f * N;
+  const uint32_t *col = a.rank + (size_t)f * N;
+  uint32_t *q = set + Wb + wave * kQueue, *own = cnt + wave * K;
+  constexpr int U = 4;
+  for (uint32_t c = threadIdx.x; c < Wb; c += W * kWave) set[c] = 0;
+  for (uint32_t c = threadIdx.x; c < W * K; c += W * kWave) cnt[c] = 0;
+  __syncthreads();
+  for (uint32_t p = threadIdx.x; p < n; p += U * W * kWave) {
+    uint32_t s[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s[u] = sample_of(list[min(p + (uint32_t)u * (W * kWave), n - 1u)]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) atomicOr(&set[s[u] >> 5], 1u << (s[u] & 31u));  // (the last one again past the end)
+  }
+  __syncthreads();
+  // this wave's share of the row, whole tiles of U x 64
+  const uint32_t share = (N + W * U * kWave - 1u) / (W * U * kWave) * (U * kWave);
+  const uint32_t r0 = min(wave * share, N), r1 = min(r0 + share, N);
+  uint32_t firstw = 0xFFFFFFFFu;  // the wave's first kept word
+  for (uint32_t rb = r0; rb < r1; rb += U * kWave) {
+    uint32_t e[U];
+    load_row_batch(row, rb, r1, e);
+    uint32_t lab[U];
+    bool in[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) lab[u] = a.label((IdxT)e[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t s = sample_of((IdxT)e[u]);
+      in[u] = rb + (uint32_t)u * kWave + lane < r1 && (set[s >> 5] >> (s & 31u) & 1u) != 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint64_t mk = ballot(in[u]);
+      if (!mk) continue;
+      if (firstw == 0xFFFFFFFFu)
+        firstw = uniform(col[sample_of((IdxT)readlane(e[u], (uint32_t)__ffsll((unsigned long long)mk) - 1u))]);
+      count_labels(own, lab[u], in[u], nbits);
+    }
+  }
+  if (lane == 0) tail[wave * 8u + 7u] = firstw;
+  wg_prefix<W>(cnt, K);
+  uint32_t after = 0;  // the first kept word of the waves behind
+#pragma unroll 1
+  for (uint32_t v = W; v-- > wave + 1u;) {
+    const uint32_t x = tail[v * 8u + 7u];
+    if (x != 0xFFFFFFFFu) after = x;
+  }
+  Scan<Large, kRegs> sc;
+  const uint32_t p0 = scan_start(sc, own, tot, K, n, f, feat_vals(a, f));
+  Best<Large> best;
+  uint32_t qn = 0, qd = 0;  // words queued, words scanned
+  for (uint32_t rb = r0; rb < r1; rb += U * kWave) {
+    uint32_t e[U], x[U];
+    load_row_batch(row, rb, r1, e);
+    bool in[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t s = sample_of((IdxT)e[u]);
+      in[u] = rb + (uint32_t)u * kWave + lane < r1 && (set[s >> 5] >> (s & 31u) & 1u) != 0u;
+      x[u] = 0;
+      if (in[u]) x[u] = col[s];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint64_t mk = ballot(in[u]);
+      if (in[u]) q[(qn + mbcnt(mk)) % kQueue] = x[u];
+      qn += (uint32_t)__popcll(mk);
+      wave_sync();
+      if (qn - qd > kWave) {  // a whole tile and the word after it
+        sc.tile(q[(qd + lane) % kQueue], q[(qd + lane + 1u) % kQueue], true, p0 + qd + lane, best);
+        qd += kWave;
+        wave_sync();
+      }
+    }
+  }
+  if (qn != qd) {
+    const uint32_t m = qn - qd;  // at most 64
+    const uint32_t y = lane + 1u < m ? q[(qd + lane + 1u) % kQueue] : after;
+    sc.tile(q[(qd + lane) % kQueue], y, lane < m, p0 + qd + lane, best);
+  }
+  if (kRegs && lane < K) own[lane] = sc.cv;  // the counts at the end of the share, as in LDS
+  best = wave_best_of(best);
+  if (lane == 0) put_best(tail + wave * 8u, best);
+  __syncthreads();
+  const uint32_t win = best_entry<Large, W>(tail);
+  bool found = win < (uint32_t)W;
+  const uint32_t *t = tail + (found ? win : 0u) * 8u;
+  const uint32_t pos = t[4], lo = t[5];
+  if (found) {
+    // left class counts: those before the winning wave's share and its kept
+    // samples up to the split's value
+    uint32_t *acc = cnt + win * K;
+    for (uint32_t k = threadIdx.x; k < K; k += W * kWave) acc[k] = win ? cnt[(win - 1u) * K + k] : 0u;
+    __syncthreads();
+    for (uint32_t r = win * share + threadIdx.x; r < min((win + 1u) * share, N); r += W * kWave) {
+      const uint32_t s = sample_of(row[r]);
+      if (!(set[s >> 5] >> (s & 31u) & 1u)) continue;
+      const uint32_t x = col[s];
+      if (x >> kLabBits <= lo) atomicAdd(&acc[x & kLabMask], 1u);
+    }
+    __syncthreads();
+    uint32_t sum = 0;
+    for (uint32_t k = lane; k < K; k += kWave) sum += acc[k];
+    // (they have to be the samples up to the split's position)
+    found = wave_sum32(sum) == pos + 1u;
+    if (!found && threadIdx.x == 0) a.ctl->bad = 1u;
+    for (uint32_t k = threadIdx.x; k < K; k += W * kWave) left[k] = acc[k];
+  }
+  if (threadIdx.x == 0) put_res(res, t, f, found);
 }
 
 template <int kWg, int E, bool kRegs, class IdxT, class LabT>
@@ -671,7 +890,7 @@ __global__ __launch_bounds__(kListWaves[kWg] * kWave) void k_list_wg(FitArgs<Idx
   constexpr int W = kListWaves[kWg];
   extern __shared__ uint32_t smem[];
   const uint32_t K = (uint32_t)a.K;
-  uint32_t *w = smem, *cnt = w + kListWg[kWg], *tot = cnt + W * K, *tail = tot + K, *next = tail + W * 8u;
+  uint32_t *w = smem, *cnt = w + list_body_words(kWg, (uint32_t)a.N), *tot = cnt + W * K, *tail = tot + K, *next = tail + W * 8u;
   const uint32_t G = gridDim.x / kXcd;
   bool own = true;
   for (uint32_t turn = 0; turn < kXcd;) {
@@ -706,6 +925,8 @@ __global__ __launch_bounds__(kListWaves[kWg] * kWave) void k_list_wg(FitArgs<Idx
     if constexpr (kWg == 0) {
       if (n <= 2048) wg_task<kWg, 8, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
       else wg_task<kWg, 16, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
+    } else if constexpr (kWg == 2) {
+      wg_filter<W, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
     } else {
       if (n <= 8192) wg_task<kWg, 8, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
       else if (n <= 16384) wg_task<kWg, 16, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);

@@ -1,7 +1,7 @@
 """Split search from sample lists (needs an MI355X): forests grown with
 search=CTA_SEARCH_LISTS equal the oracle's bit for bit, with root sizes on
 both sides of every limit between the sorts (a wave's 64 to 1,024 samples, a
-workgroup's 4,096 and 32,768), for features with gaps below the candidate
+workgroup's 4,096 and 32,768, the filtered rows beyond), for features with gaps below the candidate
 test's, many ties, infinities, constants and two values, few and many
 classes, and both index widths."""
 import numpy as np
@@ -71,7 +71,8 @@ def test_tiny_cases(ctx, orc):
 
 @pytest.mark.parametrize("n,K", [(3, 2), (63, 2), (64, 4), (65, 5), (128, 3), (129, 7), (256, 2), (257, 20), (512, 4),
                                  (513, 300), (1024, 6), (1025, 3), (2048, 5), (2049, 9), (4096, 2), (4097, 4),
-                                 (8192, 7), (8193, 100), (16384, 3), (16385, 6), (32768, 2)])
+                                 (8192, 7), (8193, 100), (16384, 3), (16385, 6), (32768, 2),
+                                 (32769, 4), (40001, 7), (70001, 20), (131072, 2)])
 def test_sort_limits(ctx, orc, n, K):
     case = mixed(n, K, 1000 + n)
     print("list limits n=%d K=%d" % (n, K), flush=True)

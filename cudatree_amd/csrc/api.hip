@@ -260,8 +260,9 @@ struct cta_dataset {
   // list search, made by the first fit that uses it: words by sample, the
   // features' distinct values, and per feature where they start and the index
   // distance that needs no test
-  bool listed = false;
-  DevMem rank, dval, voff, gapw;
+  bool listed = false, hist_small = false;  // (hist_small: some feature suits the 4-wave count)
+  uint32_t hist_max = 0;                    // largest table of the features that suit the 16-wave count
+  DevMem rank, dval, voff, gapw, ndist;
   // row-free features (two-valued, other than feature 0): tables of the fits
   // that keep no rows for them, and identity tables for fits that keep all
   int32_t Frl = 0, Wsig = 0, Fr = 0;
@@ -464,19 +465,21 @@ int list_kinds(int32_t N) {
 }
 
 // Whether a fit searches its splits from sample lists (list_kernels.hip)
-// instead of sorted rows; Fr: the rows it would keep.
-bool list_fits(const cta_ctx &ctx, const cta_dataset &ds, const cta_fit_opts &o, uint32_t Fr) {
+// instead of sorted rows.
+bool list_search(const cta_ctx &ctx, const cta_dataset &ds, const cta_fit_opts &o) {
   if (o.search == CTA_SEARCH_ROWS || o.mode != CTA_MODE_BATCHED || o.all_rows || o.subtree_max > 0) return false;
   // the words or the sample set of a node and its class counts must fit the LDS
   for (int w = 0; w < list_kinds(ds.N); ++w)
-    if ((size_t)list_wg_words(w, (uint32_t)ds.K, (uint32_t)ds.N) * 4 > ctx.lds_per_block) return false;
+    if ((size_t)list_wg_words(w, (uint32_t)ds.K, (uint32_t)ds.N, 0) * 4 > ctx.lds_per_block) return false;
   if (o.search == CTA_SEARCH_LISTS) return true;
   // Rows move Fr rows per level where lists sort max_features of them, but a
   // node's sort takes one workgroup where rows split it into chunks.  Rows /
   // lists, ms: 20,000 x 4,096 (Fr / m = 64) 238 / 51; 7,490 x 233 (14) 7.5 /
-  // 5.3; 10,253 x 151, 6 trees (12) 3.8 / 3.8; 1,797 x 64 (8) 2.0 / 2.3;
-  // 29,894 x 48 (7) 3.5 / 4.5.
-  return (uint64_t)Fr >= 10ull * (uint64_t)o.max_features;
+  // 5.3; 10,253 x 151, 6 trees (12) 3.8 / 3.8; 1,000,000 x 64 of 256 levels
+  // (8) 656 / 415; 1,797 x 64 of 17 levels (8) 2.0 / 2.0 (a set that small is
+  // bound by launches); 29,894 x 48 (7) 3.5 / 4.5; 581,012 x 54 with 10 rows
+  // (1.4) 31 / 71.
+  return (uint64_t)ds.Fr >= ((uint32_t)ds.N > kListWg[1] ? 8ull : 10ull) * (uint64_t)o.max_features;
 }
 
 // The list search's tables of a training set (kept with it; built on the
@@ -490,23 +493,33 @@ void list_tables(cta_ctx *ctx, cta_dataset *ds) {
   const uint32_t ntiles = (N + kCodeTile - 1) / kCodeTile;
   uint32_t *pre = ctx->ws_as<uint32_t>("code_pre", (size_t)N * F);
   uint32_t *tsum = ctx->ws_as<uint32_t>("code_tsum", (size_t)ntiles * F);
-  uint32_t *db = ctx->ws_as<uint32_t>("code_meta", 2 * (size_t)F);  // distinct values, then the bad flags
+  uint32_t *bad = ctx->ws_as<uint32_t>("code_meta", 2 * (size_t)F);
+  ds->ndist.alloc((size_t)F * 4);
+  uint32_t *nd = ds->ndist.as<uint32_t>();
   const IdxT *rows = ds->si0.as<IdxT>();
   const float *XT = ds->XT.as<float>();
-  k_fill_u32<<<grid_for(2 * (size_t)F), 256, 0, st>>>(db, 2 * (size_t)F, 0u);
-  k_list_flags<IdxT><<<dim3(ntiles, F), kCodeThreads, 0, st>>>(rows, XT, N, ntiles, pre, tsum, db + F);
-  k_code_tscan<<<F, 1024, 0, st>>>(tsum, ntiles, db);
+  k_fill_u32<<<grid_for((size_t)F), 256, 0, st>>>(bad, (size_t)F, 0u);
+  k_list_flags<IdxT><<<dim3(ntiles, F), kCodeThreads, 0, st>>>(rows, XT, N, ntiles, pre, tsum, bad);
+  k_code_tscan<<<F, 1024, 0, st>>>(tsum, ntiles, nd);
   uint32_t *h = static_cast<uint32_t *>(ctx->host("code_meta", 2 * (size_t)F * 4));
-  HIPC(hipMemcpyAsync(h, db, (size_t)F * 4, hipMemcpyDeviceToHost, st));
+  HIPC(hipMemcpyAsync(h, nd, (size_t)F * 4, hipMemcpyDeviceToHost, st));
   ds->rank.alloc((size_t)N * F * 4);
   ds->voff.alloc((size_t)F * 8);
   ds->gapw.alloc((size_t)F * 4);
   uint64_t *hv = static_cast<uint64_t *>(ctx->host("list_voff", (size_t)F * 8));
   ctx->sync();
   uint64_t nval = 0;
+  const uint32_t K = (uint32_t)ds->K;
+  ds->hist_max = 0;
+  ds->hist_small = false;
   for (uint32_t f = 0; f < F; ++f) {
     hv[f] = nval;
     nval += h[f];
+    if (hist_small(h[f], K)) ds->hist_small = true;
+    const uint64_t words = (uint64_t)h[f] * hist_stride(K);
+    if (h[f] <= (uint32_t)(kListWaves[3] * kWave) && words > ds->hist_max &&
+        (uint64_t)list_wg_words(3, K, N, (uint32_t)words) * 4 <= ctx->lds_per_block)
+      ds->hist_max = (uint32_t)words;
   }
   ds->dval.alloc(nval * 4);
   HIPC(hipMemcpyAsync(ds->voff.p, hv, (size_t)F * 8, hipMemcpyHostToDevice, st));
@@ -515,7 +528,7 @@ void list_tables(cta_ctx *ctx, cta_dataset *ds) {
       rows, XT, ds->y.as<LabT>(), pre, tsum, N, ntiles, ds->voff.as<uint64_t>(), ds->rank.as<uint32_t>(),
       ds->dval.as<float>());
   k_list_gapw<<<dim3(std::min<uint32_t>(64, ntiles), F), kCodeThreads, 0, st>>>(
-      ds->dval.as<float>(), ds->voff.as<uint64_t>(), db, db + F, ds->gapw.as<uint32_t>());
+      ds->dval.as<float>(), ds->voff.as<uint64_t>(), nd, bad, ds->gapw.as<uint32_t>());
   HIPC(hipGetLastError());
   ds->listed = true;
 }
@@ -566,7 +579,7 @@ struct Fitter {
     slot_of_d = (rowfree ? d->slot_of : d->ident).as<int32_t>();
     row_feat_d = (rowfree ? d->row_feat : d->ident).as<int32_t>();
     Fc = Fr;
-    list = list_fits(*c, *d, opts, Fr);
+    list = list_search(*c, *d, opts);
     if (list) Fr = 1;  // (feature 0 has the first row slot)
     // a wave-loop grid larger than what stays resident leaves a tail of
     // late workgroups; k_scan's registers allow fewer than 8 per CU
@@ -584,8 +597,10 @@ struct Fitter {
       const void *wg[kWgKinds] = {
           scan_regs ? (const void *)k_list_wg<IdxT, LabT, 0, true> : (const void *)k_list_wg<IdxT, LabT, 0, false>,
           scan_regs ? (const void *)k_list_wg<IdxT, LabT, 1, true> : (const void *)k_list_wg<IdxT, LabT, 1, false>,
-          scan_regs ? (const void *)k_list_wg<IdxT, LabT, 2, true> : (const void *)k_list_wg<IdxT, LabT, 2, false>};
-      for (int w = 0; w < list_kinds(N); ++w) {
+          scan_regs ? (const void *)k_list_wg<IdxT, LabT, 2, true> : (const void *)k_list_wg<IdxT, LabT, 2, false>,
+          (const void *)k_list_wg<IdxT, LabT, 3, false>, (const void *)k_list_wg<IdxT, LabT, 4, false>};
+      for (int w = 0; w < kWgKinds; ++w) {
+        if (!wg_used(w)) continue;
         HIPC(hipFuncSetAttribute(wg[w], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ctx->lds_per_block));
         Gwg[w] = grid(wg[w], kListWaves[w] * kWave, wg_lds(w));
       }
@@ -598,8 +613,13 @@ struct Fitter {
   // side bitmap, then each wave's row-free counters
   size_t fill_lds_bytes() const { return (((size_t)N + 31) / 32) * 4 + (size_t)kFillWaves * Frl * K * 4; }
 
-  // bytes of LDS of a list workgroup; the kinds a training set of N can need
-  size_t wg_lds(int w) const { return (size_t)list_wg_words(w, (uint32_t)K, (uint32_t)N) * 4; }
+  // bytes of LDS of a list workgroup of kind w, and whether the training set has
+  // nodes and features for it
+  size_t wg_lds(int w) const { return (size_t)list_wg_words(w, (uint32_t)K, (uint32_t)N, ds->hist_max) * 4; }
+  bool wg_used(int w) const {
+    if (w < 3) return w < list_kinds(N);
+    return list_kinds(N) > 0 && (w == 3 ? ds->hist_max > 0 : ds->hist_small);
+  }
   size_t list_lds() const { return (size_t)kWavesPerBlock * list_wave_words((uint32_t)K, scan_regs) * 4; }
 
   size_t smem() const { return (size_t)kWavesPerBlock * 2 * K * sizeof(uint32_t); }
@@ -656,11 +676,11 @@ struct Fitter {
     const uint64_t cap_fill = cap_q + n_tot / Cf + 64;
     const uint64_t cap_hist = (uint64_t)m * K * ((list ? n_tot / kListWave : 2 * n_tot / Cs) + 64);
     // (node, feature) tasks of nodes of more than kListWave / kListWg[0] / kListWg[1] samples
-    const uint64_t cap_wg[kWgKinds] = {list ? (uint64_t)m * (n_tot / kListWave) + 64 : 0,
-                                       list ? (uint64_t)m * (n_tot / kListWg[0]) + 64 : 0,
-                                       list ? (uint64_t)m * (n_tot / kListWg[1]) + 64 : 0};
+    const uint64_t all_wg = (uint64_t)m * (n_tot / kListWave) + 64;
+    const uint64_t cap_wg[kWgKinds] = {all_wg, (uint64_t)m * (n_tot / kListWg[0]) + 64,
+                                       (uint64_t)m * (n_tot / kListWg[1]) + 64, all_wg, all_wg};
     if (cap_scan > 0xFFFFFFF0ull || cap_small > 0xFFFFFFF0ull || cap_big > 0xFFFFFFF0ull ||
-        cap_nodes > 0xFFFFFFF0ull || cap_hist > 0xFFFFFFF0ull || cap_wg[0] > 0xFFFFFFF0ull)
+        cap_nodes > 0xFFFFFFF0ull || cap_hist > 0xFFFFFFF0ull || (list && all_wg > 0xFFFFFFF0ull))
       fail(CTA_EUNSUPPORTED, "batch of %d trees too large for 32-bit task indices", Tb);
 
     IdxT *buf0 = ctx->ws_as<IdxT>("buf0", (size_t)Tb * Fr * N), *buf1 = ctx->ws_as<IdxT>("buf1", (size_t)Tb * Fr * N);
@@ -717,7 +737,10 @@ struct Fitter {
       a.dval = ds->dval.as<float>();
       a.voff = ds->voff.as<uint64_t>();
       a.gapw = ds->gapw.as<uint32_t>();
+      a.ndist = ds->ndist.as<uint32_t>();
+      a.hist_max = ds->hist_max;
       for (int w = 0; w < kWgKinds; ++w) {
+        if (!wg_used(w)) continue;
         a.wg_tasks[w] = ctx->ws_as<Task>("wg_tasks" + std::to_string(w), cap_wg[w] * kXcd);
         a.cap_wg[w] = (uint32_t)cap_wg[w];
       }
@@ -1151,17 +1174,23 @@ struct Fitter {
   // The level's split scans from the nodes' sample lists, large nodes first.
   template <bool kRegs>
   void list_scan_k(const FitArgs<IdxT, LabT> &a) {
-    // (only the kinds that a node of this training set can need)
-    const int kinds = list_kinds(N);
-    if (kinds > 2) {
+    if (wg_used(3)) {
+      Timed tm(ctx, "k_list_hist");
+      k_list_wg<IdxT, LabT, 3, false><<<Gwg[3], kListWaves[3] * kWave, wg_lds(3), st>>>(a);
+    }
+    if (wg_used(2)) {
       Timed tm(ctx, "k_list_filter");
       k_list_wg<IdxT, LabT, 2, kRegs><<<Gwg[2], kListWaves[2] * kWave, wg_lds(2), st>>>(a);
     }
-    if (kinds > 1) {
+    if (wg_used(1)) {
       Timed tm(ctx, "k_list_big");
       k_list_wg<IdxT, LabT, 1, kRegs><<<Gwg[1], kListWaves[1] * kWave, wg_lds(1), st>>>(a);
     }
-    if (kinds > 0) {
+    if (wg_used(4)) {
+      Timed tm(ctx, "k_list_hist4");
+      k_list_wg<IdxT, LabT, 4, false><<<Gwg[4], kListWaves[4] * kWave, wg_lds(4), st>>>(a);
+    }
+    if (wg_used(0)) {
       Timed tm(ctx, "k_list_mid");
       k_list_wg<IdxT, LabT, 0, kRegs><<<Gwg[0], kListWaves[0] * kWave, wg_lds(0), st>>>(a);
     }
@@ -1399,11 +1428,11 @@ void append_trees(cta_forest *dst, const cta_forest *src, int32_t t, int32_t n) 
 template <class IdxT, class LabT>
 void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, const int64_t *off,
               const cta_fit_opts &o, cta_forest *out) {
-  Fitter<IdxT, LabT> fz(ctx, ds, o);
-  if (fz.list) {
+  if (list_search(*ctx, *ds, o)) {
     list_tables<IdxT, LabT>(ctx, ds);
     if (o.lanes == 2) ctx->sync();  // (the other lane's stream reads them too)
   }
+  Fitter<IdxT, LabT> fz(ctx, ds, o);
   // trees resident at once on one stream: as asked, else what 60% of the
   // free memory holds (workspaces are reused by this fit)
   int32_t per = o.trees_per_batch;

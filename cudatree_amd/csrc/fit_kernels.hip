@@ -262,25 +262,65 @@ __global__ __launch_bounds__(kOffThreads) void k_off_apply(const uint32_t *v, co
 // larger nodes are filtered from the presorted row.
 constexpr uint32_t kListE = 16, kListWave = kWave * kListE;
 constexpr uint32_t kListWg[2] = {4096, 32768};
-constexpr int kListWaves[kWgKinds] = {4, 16, 16};
-__device__ __forceinline__ int list_kind(uint32_t n) { return n <= kListWg[0] ? 0 : n <= kListWg[1] ? 1 : 2; }
+#ifndef CTA_HIST_WORTH
+#define CTA_HIST_WORTH 4
+#endif
+constexpr uint32_t kHistWorth = CTA_HIST_WORTH;  // table words that one sample is worth clearing and scanning
+constexpr int kListWaves[kWgKinds] = {4, 16, 16, 16, 4};
+// Features of few values are counted instead of sorted: a table of D values x
+// hist_stride(K) words in LDS (an odd stride spreads a class's counts over
+// the banks), 64 values a wave.  The 4-wave count takes tables of up to
+// kHistSmall words at nodes of up to kHistSmallN samples (beyond, 16 waves
+// count faster); the 16-wave count tables of up to kHistWorth words a sample
+// (1,000,000 x 64 of 256 levels, 100 classes, per fit: 4 words 156 ms for all
+// large nodes, 8 words 156 ms, 16 words 183 ms).
+constexpr uint32_t kHistSmall = 4096, kHistSmallN = 16384;
+__host__ __device__ __forceinline__ uint32_t hist_stride(uint32_t K) { return K | 1u; }
+__host__ __device__ __forceinline__ bool hist_small(uint32_t D, uint32_t K) {
+  return D <= 4u * kWave && D * hist_stride(K) <= kHistSmall;
+}
+__device__ __forceinline__ int list_kind(uint32_t n, uint32_t D, uint32_t K, uint32_t hist_max) {
+  const uint32_t words = D * hist_stride(K);
+  if (hist_small(D, K) && n <= kHistSmallN) return 4;
+  if (D <= 16u * kWave && words <= hist_max && words <= kHistWorth * n) return 3;
+  return n <= kListWg[0] ? 0 : n <= kListWg[1] ? 1 : 2;
+}
 
 // ------------------------------------------------------------------------
 // k_select: visiting order of every frontier node, its task and slot counts
 // (scan tasks, histogram words, fill-task slots) and the frontier range of
 // each tree.
 // ------------------------------------------------------------------------
+// List search: a feature's value indices by sample, from its code column
+// where it has one of 8 or 16 bits (a quarter or half the cache lines of the
+// words), else from its words.
+struct IndexCol {
+  const uint8_t *p;
+  uint32_t kind;
+  __device__ __forceinline__ uint32_t at(uint32_t s) const {
+    if (kind == 2) return p[s];
+    if (kind == 3) return reinterpret_cast<const uint16_t *>(p)[s];
+    return reinterpret_cast<const uint32_t *>(p)[s] >> kLabBits;
+  }
+};
+template <class IdxT, class LabT>
+__device__ __forceinline__ IndexCol index_col(const FitArgs<IdxT, LabT> &a, uint32_t f) {
+  const uint64_t fc = a.fcode[f];
+  if (fc_kind(fc) >= 2) return {a.codes + fc_off(fc), fc_kind(fc)};
+  return {reinterpret_cast<const uint8_t *>(a.rank + (size_t)f * (uint32_t)a.N), 0u};
+}
+
 // List search: the node's order of a feature is not at hand, so the constant
 // test compares the value indices of its samples with the first sample's.
 // True in the lanes with `want` set whose column (col) differs somewhere over
 // the node's samples list[0, n), as far as it takes to know the first `need`
 // features that are not constant, `known` being those already known.
 template <class IdxT>
-__device__ __forceinline__ bool list_varies(const IdxT *list, uint32_t n, const uint32_t *col, bool want,
+__device__ __forceinline__ bool list_varies(const IdxT *list, uint32_t n, const IndexCol &col, bool want,
                                             uint64_t known, uint32_t need) {
   const uint32_t lane = lane_id();
   bool diff = false;
-  const uint32_t w0 = want ? col[sample_of(list[0])] >> kLabBits : 0u;
+  const uint32_t w0 = want ? col.at(sample_of(list[0])) : 0u;
   // the lanes still to be decided, none once the need-th known one comes
   // before all of them
   auto open = [&]() -> uint64_t {
@@ -295,23 +335,24 @@ __device__ __forceinline__ bool list_varies(const IdxT *list, uint32_t n, const 
     if (!open()) return diff;
     uint32_t x[U];
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) x[u] = want && !diff ? col[sample_of(list[min(j + u, n - 1u)])] >> kLabBits : w0;
+    for (uint32_t u = 0; u < U; ++u) x[u] = want && !diff ? col.at(sample_of(list[min(j + u, n - 1u)])) : w0;
 #pragma unroll
     for (uint32_t u = 0; u < U; ++u) diff |= x[u] != w0;
   }
   // rarely further: the wave reads one lane's column 64 U samples at a time
   for (uint64_t und = n > near ? open() : 0ull; und; und = open()) {
     const uint32_t L = (uint32_t)__ffsll((unsigned long long)und) - 1u;
-    const uint64_t cp = reinterpret_cast<uint64_t>(col);
-    const uint32_t *c = reinterpret_cast<const uint32_t *>((uint64_t)readlane((uint32_t)(cp >> 32), L) << 32 |
-                                                           readlane((uint32_t)cp, L));
+    const uint64_t cp = reinterpret_cast<uint64_t>(col.p);
+    const IndexCol c = {reinterpret_cast<const uint8_t *>((uint64_t)readlane((uint32_t)(cp >> 32), L) << 32 |
+                                                          readlane((uint32_t)cp, L)),
+                        readlane(col.kind, L)};
     const uint32_t first = readlane(w0, L);
     bool found = false;
     for (uint32_t pb = near; pb < n && !found; pb += U * kWave) {
       bool d = false;
 #pragma unroll
       for (uint32_t u = 0; u < U; ++u)
-        d |= (c[sample_of(list[min(pb + u * kWave + lane, n - 1u)])] >> kLabBits) != first;
+        d |= c.at(sample_of(list[min(pb + u * kWave + lane, n - 1u)])) != first;
       found = ballot(d) != 0ull;
     }
     if (lane == L) {
@@ -414,8 +455,7 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
       }
       if constexpr (kList) {
         const bool want = k < F && jr < 0;
-        const uint32_t *col = a.rank + (size_t)(want ? f : 0u) * (uint32_t)a.N;
-        nonconst |= list_varies(list, n, col, want, ballot(nonconst), m - nsel);
+        nonconst |= list_varies(list, n, index_col(a, want ? f : 0u), want, ballot(nonconst), m - nsel);
       }
       const uint64_t mk = ballot(nonconst);
       const uint32_t r = mbcnt(mk);
@@ -503,24 +543,37 @@ __global__ __launch_bounds__(kBlock) void k_select_emit(FitArgs<IdxT, LabT> a) {
     // items: features of a multi-chunk node (nch tasks each), else tasks
     const uint32_t nitem = nch > 1 ? nf : ntask;
     if (kList && nch > 1) {
-      const int wg = list_kind(a.front[i].n);
-      const uint32_t cap = wg == 0 ? a.cap_wg[0] : wg == 1 ? a.cap_wg[1] : a.cap_wg[2];
-      Task *tasks = wg == 0 ? a.wg_tasks[0] : wg == 1 ? a.wg_tasks[1] : a.wg_tasks[2];
+      const uint32_t n = a.front[i].n;
       bool over = false;
       for (uint32_t c0 = 0; c0 < nf; c0 += kWave) {
         const uint32_t it = c0 + lane;
-        const uint32_t c = it < nf ? scan_cls(a, (uint32_t)a.feats[(size_t)i * a.m + it], i) : kXcd;
-        for (uint32_t x = 0; x < kXcd; ++x) {
+        // the list of the lane's task: kind * kXcd + class
+        uint32_t c = kWgKinds * kXcd;
+        if (it < nf) {
+          const uint32_t f = (uint32_t)a.feats[(size_t)i * a.m + it];
+          c = (uint32_t)list_kind(n, a.ndist[f], (uint32_t)a.K, a.hist_max) * kXcd + scan_cls(a, f, i);
+        }
+        // one atomic per list that the lanes name
+        for (uint64_t rem = ballot(it < nf); rem;) {
+          const uint32_t lead = (uint32_t)__ffsll((unsigned long long)rem) - 1u;
+          const uint32_t x = readlane(c, lead);
           const uint64_t mk = ballot(c == x);
-          if (!mk) continue;
-          const uint32_t lead = (uint32_t)__ffsll((unsigned long long)mk) - 1u;
           uint32_t p = 0;
-          if (lane == lead) p = atomicAdd(&a.ctl->n_wg[wg][x], (uint32_t)__popcll(mk));
+          if (lane == lead) p = atomicAdd(&a.ctl->n_wg[0][0] + x, (uint32_t)__popcll(mk));
           p = readlane(p, lead) + mbcnt(mk);
+          const uint32_t kind = x / kXcd;
+          Task *tasks = a.wg_tasks[0];
+          uint32_t cap = a.cap_wg[0];
+#pragma unroll
+          for (uint32_t k = 1; k < (uint32_t)kWgKinds; ++k) {
+            tasks = kind == k ? a.wg_tasks[k] : tasks;
+            cap = kind == k ? a.cap_wg[k] : cap;
+          }
           if (c == x) {
-            if (p < cap) tasks[(size_t)x * cap + p] = Task{i, it | (1u << 16), 0u, 1u};
+            if (p < cap) tasks[(size_t)(x % kXcd) * cap + p] = Task{i, it | (1u << 16), 0u, 1u};
             else over = true;
           }
+          rem &= ~mk;
         }
       }
       if (ballot(over) && lane == 0) atomicOr(&a.ctl->err, kErrCapacity);
@@ -1601,8 +1654,9 @@ __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, con
     const uint32_t p0 = tk.chunk * a.Cf, p1 = min(nd.n, p0 + a.Cf);
     const bool bycol = !kList || jr >= 0;
     // the feature's bit column (N / 8 bytes) rather than the signatures
-    const uint32_t *col = bycol ? reinterpret_cast<const uint32_t *>(a.codes + fc_off(a.fcode[ax.best_f]))
-                                : a.rank + (size_t)(uint32_t)ax.best_f * (uint32_t)a.N;
+    const uint32_t *col = reinterpret_cast<const uint32_t *>(a.codes + fc_off(a.fcode[ax.best_f]));
+    IndexCol ic = {nullptr, 0u};
+    if (kList && !bycol) ic = index_col(a, (uint32_t)ax.best_f);
     for (uint32_t pb = p0; pb < p1; pb += kFillU * kWave) {
       uint32_t e[kFillU], low[kFillU];
 #pragma unroll
@@ -1615,7 +1669,7 @@ __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, con
         const uint32_t s = sample_of((IdxT)e[u]);
         low[u] = 0u;
         if (e[u] != 0xFFFFFFFFu)
-          low[u] = bycol ? !((col[s >> 5] >> (s & 31u)) & 1u) : (uint32_t)((col[s] >> kLabBits) <= ax.lo);
+          low[u] = bycol ? !((col[s >> 5] >> (s & 31u)) & 1u) : (uint32_t)(ic.at(s) <= ax.lo);
       }
       // the lower value goes left: the smaller side's samples are marked
       bool take[kFillU];

@@ -73,8 +73,9 @@ constexpr uint32_t kLevelRing = 64;
 constexpr uint32_t kXcd = 8;
 
 // Kinds of workgroup tasks of the list search: by the node's size, sorted by 4
-// or 16 waves, or filtered from the presorted row.
-constexpr int kWgKinds = 3;
+// or 16 waves, or filtered from the presorted row; for a feature of few
+// values, counted by value and class by 16 or 4 waves.
+constexpr int kWgKinds = 5;
 
 // Counters of one level, in device memory.  Nothing is allocated with
 // atomics: the totals are written by the offset scans over the frontier.
@@ -192,6 +193,8 @@ struct FitArgs {
   const float *dval;        // distinct values of feature f in ascending order at voff[f]
   const uint64_t *voff;     // [F]
   const uint32_t *gapw;     // [F] indices this far apart always pass the candidate test
+  const uint32_t *ndist;    // [F] distinct values
+  uint32_t hist_max;        // most words of a (value, class) table the 16-wave count takes
   Task *wg_tasks[kWgKinds];  // (node, feature) tasks by kind, kXcd lists of cap_wg each
   uint32_t cap_wg[kWgKinds];
   const int32_t *rl_of;     // [F] row-free index of each feature, or -1

@@ -24,6 +24,8 @@
 //   more                      one workgroup of 16 waves streams the feature's
 //                             presorted row of all N samples and keeps the
 //                             node's                              (k_list_wg)
+//   a feature of few values   above kListWave: one workgroup counts the
+//                             node's samples by value and class   (k_list_wg)
 #include "device_util.h"
 #include "internal.h"
 
@@ -519,17 +521,22 @@ __global__ __launch_bounds__(kBlock) void k_list_scan(FitArgs<IdxT, LabT> a) {
 
 // ---- larger nodes: one workgroup -------------------------------------------------
 // kWg = 0: 4 waves, up to 4,096 samples; kWg = 1: 16 waves, up to 32,768;
-// kWg = 2: 16 waves, any size, from the presorted row.
+// kWg = 2: 16 waves, any size, from the presorted row; kWg = 3 / 4: 16 / 4
+// waves, counted by value and class.
 // LDS: the words (kWg = 2: the node's sample set as N bits, then a queue of
-// kQueue words per wave), (W + 1) x K class counts (per wave, totals), the
-// waves' results of 8 words each, the next task.
+// kQueue words per wave; kWg = 3, 4: the table), (W + 1) x K class counts (per
+// wave, totals), the waves' results of 8 words each, the next task.
 constexpr uint32_t kQueue = 2 * kWave;
-__host__ __device__ __forceinline__ uint32_t list_body_words(int wg, uint32_t N) {
-  return wg == 0 ? kListWg[0] : wg == 1 ? kListWg[1] : (N + 31u) / 32u + (uint32_t)kListWaves[2] * kQueue;
+__host__ __device__ __forceinline__ uint32_t list_body_words(int wg, uint32_t N, uint32_t hist_max) {
+  return wg == 0   ? kListWg[0]
+         : wg == 1 ? kListWg[1]
+         : wg == 2 ? (N + 31u) / 32u + (uint32_t)kListWaves[2] * kQueue
+         : wg == 3 ? hist_max
+                   : kHistSmall;
 }
-__host__ __device__ __forceinline__ uint32_t list_wg_words(int wg, uint32_t K, uint32_t N) {
+__host__ __device__ __forceinline__ uint32_t list_wg_words(int wg, uint32_t K, uint32_t N, uint32_t hist_max) {
   const uint32_t W = (uint32_t)kListWaves[wg];
-  return list_body_words(wg, N) + (W + 1u) * K + W * 8u + 8u;
+  return list_body_words(wg, N, hist_max) + (W + 1u) * K + W * 8u + 8u;
 }
 
 // The words of the node's samples in ascending order into `w` (W x E x 64
@@ -869,6 +876,106 @@ __device__ __forceinline__ void wg_filter(const FitArgs<IdxT, LabT> &a, const Id
   if (threadIdx.x == 0) put_res(res, t, f, found);
 }
 
+// Split scan of a node over a feature of D <= 64 W values: the samples counted
+// by value and class in LDS (table h, hist_stride(K) words a value), then the
+// candidates between adjacent present values scored from the running class
+// counts, a lane a value.  No order of the samples is needed: per sample it
+// takes the value's code, the label and one LDS atomic.
+template <int W, class IdxT, class LabT>
+__device__ __forceinline__ void wg_hist(const FitArgs<IdxT, LabT> &a, const IdxT *list, uint32_t n, uint32_t f,
+                                        uint32_t *h, uint32_t *cnt, const uint32_t *tot, uint32_t *tail, ScanRes *res,
+                                        uint32_t *left) {
+  const uint32_t lane = lane_id(), wave = uniform(threadIdx.x / kWave), K = (uint32_t)a.K;
+  const uint32_t Kp = hist_stride(K), D = uniform(a.ndist[f]);
+  for (uint32_t c = threadIdx.x; c < D * Kp; c += W * kWave) h[c] = 0;
+  __syncthreads();
+  IndexCol col = index_col(a, f);
+  col.kind = uniform(col.kind);
+  constexpr int U = 8;
+  for (uint32_t p = threadIdx.x; p < n; p += U * W * kWave) {
+    uint32_t e[U], x[U], l[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) e[u] = (uint32_t)list[min(p + (uint32_t)u * (W * kWave), n - 1u)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t s = sample_of((IdxT)e[u]);
+      l[u] = a.label((IdxT)e[u]);
+      x[u] = col.at(s);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (p + (uint32_t)u * (W * kWave) < n) atomicAdd(&h[x[u] * Kp + l[u]], 1u);
+  }
+  __syncthreads();
+  // class counts of the wave's 64 values, then those before them
+  const uint32_t v0 = min(wave * kWave, D), v1 = min(v0 + kWave, D);
+  uint32_t *own = cnt + wave * K;
+  for (uint32_t k = lane; k < K; k += kWave) {
+    uint32_t s = 0;
+    for (uint32_t v = v0; v < v1; ++v) s += h[v * Kp + k];
+    own[k] = s;
+  }
+  wg_prefix<W>(cnt, K);
+  const uint32_t v = v0 + lane;
+  const bool valid = v < v1;
+  uint64_t SL = 0, Dd = 0, T2 = 0;
+  uint32_t here = 0, nL = 0;
+  if (v0 < v1)
+    for (uint32_t k = 0; k < K; ++k) {
+      const uint32_t x = valid ? h[v * Kp + k] : 0u, t = tot[k];
+      const uint32_t c = own[k] + wave_incl_scan(x);
+      here += x;
+      nL += c;
+      SL += (uint64_t)c * c;
+      Dd += (uint64_t)t * c;
+      T2 += (uint64_t)t * t;
+    }
+  const uint64_t present = ballot(here != 0u);
+  if (lane == 0) tail[wave * 8u + 7u] = present ? v0 + (uint32_t)__ffsll((unsigned long long)present) - 1u : 0xFFFFFFFFu;
+  __syncthreads();
+  // the next present value: in the wave's, else the first of the waves behind
+  uint32_t nx = 0xFFFFFFFFu;
+#pragma unroll 1
+  for (uint32_t w = W; w-- > wave + 1u;) {
+    const uint32_t x = tail[w * 8u + 7u];
+    if (x != 0xFFFFFFFFu) nx = x;
+  }
+  const uint64_t later = lane == kWave - 1 ? 0ull : present >> (lane + 1u);
+  if (later) nx = v + (uint32_t)__ffsll((unsigned long long)later);
+  const FeatVals fv = feat_vals(a, f);
+  Best<Large> best;
+  if (here != 0u && nx != 0xFFFFFFFFu && splits(fv, v, nx)) {
+    const uint64_t l = nL, r = (uint64_t)n - nL, SR = T2 + SL - 2 * Dd;
+    best.num = SL * r + SR * l;
+    best.den = l * r;
+    best.pos = nL - 1u;
+    best.feat = (int32_t)f;
+    best.lo = v;
+    best.hi = nx;
+  }
+  best = wave_best_of(best);
+  if (lane == 0) put_best(tail + wave * 8u, best);
+  __syncthreads();
+  const uint32_t win = best_entry<Large, W>(tail);
+  bool found = win < (uint32_t)W;
+  const uint32_t *t = tail + (found ? win : 0u) * 8u;
+  if (found) {
+    // left class counts: those before the winning wave's values and theirs up
+    // to the split (they have to be the samples up to the split's position)
+    const uint32_t lo = t[5];
+    uint32_t sum = 0;
+    for (uint32_t k = lane; k < K; k += kWave) {
+      uint32_t s = cnt[win * K + k];
+      for (uint32_t x = win * kWave; x <= min(lo, D - 1u); ++x) s += h[x * Kp + k];
+      if (wave == 0) left[k] = s;
+      sum += s;
+    }
+    found = wave_sum32(sum) == t[4] + 1u;
+    if (!found && threadIdx.x == 0) a.ctl->bad = 1u;
+  }
+  if (threadIdx.x == 0) put_res(res, t, f, found);
+}
+
 template <int kWg, int E, bool kRegs, class IdxT, class LabT>
 __device__ __forceinline__ void wg_task(const FitArgs<IdxT, LabT> &a, const IdxT *list, uint32_t n, uint32_t f,
                                         uint32_t *w, uint32_t *cnt, const uint32_t *tot, uint32_t *tail, ScanRes *res,
@@ -890,7 +997,7 @@ __global__ __launch_bounds__(kListWaves[kWg] * kWave) void k_list_wg(FitArgs<Idx
   constexpr int W = kListWaves[kWg];
   extern __shared__ uint32_t smem[];
   const uint32_t K = (uint32_t)a.K;
-  uint32_t *w = smem, *cnt = w + list_body_words(kWg, (uint32_t)a.N), *tot = cnt + W * K, *tail = tot + K, *next = tail + W * 8u;
+  uint32_t *w = smem, *cnt = w + list_body_words(kWg, (uint32_t)a.N, a.hist_max), *tot = cnt + W * K, *tail = tot + K, *next = tail + W * 8u;
   const uint32_t G = gridDim.x / kXcd;
   bool own = true;
   for (uint32_t turn = 0; turn < kXcd;) {
@@ -925,6 +1032,8 @@ __global__ __launch_bounds__(kListWaves[kWg] * kWave) void k_list_wg(FitArgs<Idx
     if constexpr (kWg == 0) {
       if (n <= 2048) wg_task<kWg, 8, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
       else wg_task<kWg, 16, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
+    } else if constexpr (kWg >= 3) {
+      wg_hist<W>(a, list, n, f, w, cnt, tot, tail, res, left);
     } else if constexpr (kWg == 2) {
       wg_filter<W, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
     } else {

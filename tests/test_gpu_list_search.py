@@ -41,7 +41,8 @@ def fit(ctx, case, search, idx_bits=0, **opts):
 def mixed(n, K, seed, F=10, m=4, n_trees=1, max_depth=4, mss=1):
     """Features: continuous; distinct values mostly closer than 1e-5; three of
     every four equal; 6 levels; 300 levels; infinities at both ends; constant;
-    two-valued; nearly constant (one other value); continuous."""
+    two-valued; nearly constant (two other values); a few hundred levels closer
+    than 1e-5."""
     rng = np.random.Generator(np.random.PCG64(seed))
     y = rng.integers(0, K, size=n)
     y[:min(K, n)] = np.arange(min(K, n))
@@ -57,6 +58,7 @@ def mixed(n, K, seed, F=10, m=4, n_trees=1, max_depth=4, mss=1):
     X[:, 8] = 0.0
     X[n - 1, 8] = 1.0 if n % 2 else -1.0
     X[n // 2, 8] = 3.0
+    X[:, 9] = np.floor(X[:, 9] * 40) * np.float32(4e-6)
     return {"X": X, "y": y, "K": K, "m": m, "mss": mss, "max_depth": max_depth, "identity": False, "seed": seed,
             "boot": False, "n_trees": n_trees}
 

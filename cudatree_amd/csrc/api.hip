@@ -262,7 +262,7 @@ struct cta_dataset {
   // distance that needs no test
   bool listed = false, hist_small = false;  // (hist_small: some feature suits the 4-wave count)
   uint32_t hist_max = 0;                    // largest table of the features that suit the 16-wave count
-  DevMem rank, dval, voff, gapw, ndist;
+  DevMem rank, dval, voff, gapw, ndist, all;  // (all: the list of every sample)
   // row-free features (two-valued, other than feature 0): tables of the fits
   // that keep no rows for them, and identity tables for fits that keep all
   int32_t Frl = 0, Wsig = 0, Fr = 0;
@@ -504,6 +504,8 @@ void list_tables(cta_ctx *ctx, cta_dataset *ds) {
   uint32_t *h = static_cast<uint32_t *>(ctx->host("code_meta", 2 * (size_t)F * 4));
   HIPC(hipMemcpyAsync(h, nd, (size_t)F * 4, hipMemcpyDeviceToHost, st));
   ds->rank.alloc((size_t)N * F * 4);
+  ds->all.alloc((size_t)N * sizeof(IdxT));
+  k_list_all<IdxT, LabT><<<grid_for(N), 256, 0, st>>>(ds->y.as<LabT>(), N, ds->all.as<IdxT>());
   ds->voff.alloc((size_t)F * 8);
   ds->gapw.alloc((size_t)F * 4);
   uint64_t *hv = static_cast<uint64_t *>(ctx->host("list_voff", (size_t)F * 8));
@@ -733,6 +735,8 @@ struct Fitter {
     a.Fr = Fr;
     a.Fc = Fc;
     if (list) {
+      a.presorted = a.si0;
+      a.si0 = ds->all.as<IdxT>();
       a.rank = ds->rank.as<uint32_t>();
       a.dval = ds->dval.as<float>();
       a.voff = ds->voff.as<uint64_t>();
@@ -2344,7 +2348,7 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
     // plus the copies of host X and y while it is built
     // and the list search's words and distinct values
     *dataset_bytes = nf * 4 + n * lab + nf * b + 2 * nf + 256 * f + 4 * n * ((f + 31) / 32) + 64 * f + 4096 +
-                     nf * 4 + n * 4 + nf * 8 + 16 * f;
+                     nf * 4 + n * 4 + nf * 8 + n * b + 20 * f;
     // the context's workspaces: radix-sort and code-column temporaries of the
     // build, then per resident tree (every feature keeping rows), the node
     // arena and canonical export of at most two nodes per in-bag sample, and

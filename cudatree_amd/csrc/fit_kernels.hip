@@ -1308,6 +1308,23 @@ __device__ __forceinline__ uint32_t child_kind(const FitArgs<IdxT, LabT> &a, uin
   return 0u;
 }
 
+// List search: label of the first of the list's samples in feature 0's
+// presorted order -- the lowest value, then the lowest id -- among those that
+// take(entry) keeps (0xFFFFFFFF: none of them).
+template <class IdxT, class LabT, class Take>
+__device__ __forceinline__ uint32_t first_label(const FitArgs<IdxT, LabT> &a, const IdxT *list, uint32_t n,
+                                                const Take &take) {
+  uint64_t best = ~0ull;  // value index, sample, label
+  for (uint32_t p = lane_id(); p < n; p += kWave) {
+    const IdxT e = list[p];
+    const uint32_t s = sample_of(e), w = a.rank[s];
+    if (take(e)) best = min(best, (uint64_t)(w >> kLabBits) << 32 | (uint64_t)s << kLabBits | (w & kLabMask));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) best = min(best, (uint64_t)__shfl_xor((unsigned long long)best, o, kWave));
+  return best == ~0ull ? 0xFFFFFFFFu : (uint32_t)best & kLabMask;
+}
+
 // Class counts of the samples of node i whose value index of feature f is at
 // most lo (list search, a node of one wave) into cntL; returns their sum.
 template <class IdxT, class LabT>
@@ -1375,13 +1392,15 @@ __global__ __launch_bounds__(kBlock) void k_decide(FitArgs<IdxT, LabT> a) {
     if (!best.ok) {
       // no candidate position: leaf labelled by the first sample of the
       // segment in feature 0's row (random_tree.py:628-634, 50-63)
+      const IdxT *row0 = rows_of(a, nd.src, nd.tree, 0) + nd.start;
+      uint32_t lab = 0;
+      if constexpr (kList) lab = first_label(a, row0, nd.n, [](IdxT) { return true; });
       if (lane == 0) {
-        const IdxT *row0 = rows_of(a, nd.src, nd.tree, 0) + nd.start;
         a.arena.feat[id] = -1;
         a.arena.thr[id] = 0.f;
         a.arena.left[id] = kLeaf;
         a.arena.right[id] = kLeaf;
-        a.arena.value[id] = a.label(row0[0]);
+        a.arena.value[id] = kList ? lab : a.label(row0[0]);
       }
       ax.best_f = -1;
       ax.flags = 0;
@@ -1837,6 +1856,15 @@ __global__ __launch_bounds__(kBlock) void k_children_emit(FitArgs<IdxT, LabT> a)
       const uint32_t *bits = a.bits + (size_t)nd.tree * a.W;
       const uint32_t inv = (ax.flags & kInvert) ? 1u : 0u;  // the marks are on the right
       bool needl = lab[0] == kFirstSample, needr = lab[1] == kFirstSample;
+      if (a.rank) {  // (list search)
+        auto side = [&](IdxT e, uint32_t want) {
+          const uint32_t s = sample_of(e);
+          return (((bits[s >> 5] >> (s & 31u)) & 1u) ^ inv) == want;
+        };
+        if (needl) lab[0] = first_label(a, row0, nd.n, [&](IdxT e) { return side(e, 1u); });
+        if (needr) lab[1] = first_label(a, row0, nd.n, [&](IdxT e) { return side(e, 0u); });
+        needl = needr = false;
+      }
       for (uint32_t pb = 0; pb < nd.n && (needl || needr); pb += kWave) {
         const uint32_t p = pb + lane;
         uint32_t e = 0, side = 2;
@@ -2604,7 +2632,22 @@ __global__ __launch_bounds__(kPlanThreads) void k_roots(FitArgs<IdxT, LabT> a, c
       // a positive max_depth never caps the root.
       uint32_t leaf_label = kLeaf;
       if (nz <= 1) leaf_label = only;
-      else if ((int64_t)n < (int64_t)a.mss) leaf_label = a.label(rows_of(a, src, t, 0)[0]);
+      else if ((int64_t)n < (int64_t)a.mss) {
+        if (a.rank) {
+          // list search: the first in-bag sample of the presorted row (src 0:
+          // every sample is; the bitmaps still hold the in-bag marks)
+          const uint32_t *bits = a.bits + (size_t)t * a.W;
+          uint32_t p = 0;
+          while (src != 0 && p + 1 < (uint32_t)a.N) {
+            const uint32_t s = sample_of(a.presorted[p]);
+            if ((bits[s >> 5] >> (s & 31u)) & 1u) break;
+            ++p;
+          }
+          leaf_label = a.label(a.presorted[p]);
+        } else {
+          leaf_label = a.label(rows_of(a, src, t, 0)[0]);
+        }
+      }
       if (leaf_label != kLeaf) {
         a.arena.feat[t] = -1;
         a.arena.thr[t] = 0.f;

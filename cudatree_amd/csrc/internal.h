@@ -185,9 +185,11 @@ struct FitArgs {
   // for the children.
   uint32_t Frl, Wsig;       // row-free features, 32-bit signature words per sample
   uint32_t Fr;              // features with rows
-  // List search (a fit that keeps feature 0's row only): a node's samples are
-  // its segment of that row, and the words of an evaluated feature are
-  // gathered from its column of `rank` and sorted in the split search.
+  // List search (a fit that keeps one row): a node's samples are its segment
+  // of that row, which holds them in ascending order (si0 is the list of all
+  // samples then), and the words of an evaluated feature are gathered from its
+  // column of `rank` and ordered in the split search.
+  const IdxT *presorted;    // F x N presorted rows
   uint32_t Fc;              // features the split-scan classes are laid over
   const uint32_t *rank;     // F x N words by sample: value index << kLabBits | label
   const float *dval;        // distinct values of feature f in ascending order at voff[f]

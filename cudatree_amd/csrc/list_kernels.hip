@@ -2,8 +2,8 @@
 //
 // A node evaluates max_features of the F features, yet a schedule over sorted
 // rows moves all F rows at every level to have the few it will read in order.
-// Here a node keeps one row, its segment of feature 0's row, as the list of
-// its samples, and the order of an evaluated feature is made when it is
+// Here a node keeps one row, the list of its samples in ascending order, and
+// the order of an evaluated feature is made when it is
 // needed: the words (value index << kLabBits | label) of the node's samples
 // are gathered from the feature's column and sorted on the chip.  Samples of
 // equal value may leave the sort in any order: a split lies between two
@@ -16,6 +16,10 @@
 // classes keep in L2; against that, sorted rows cost 9 bytes of HBM traffic a
 // sample and kept row.  20,000 x 4,096, 100 trees, 64 of 4,096 features a
 // node: reshuffle 170 -> 0.6 ms, split search 39 -> 35 ms, fit 239 -> 53 ms.
+//
+// Ascending lists make the gathers of a large node walk its columns in order,
+// several samples a cache line (with the lists in feature 0's order the counts
+// of 1,000,000 x 64 took 105 ms a fit, ascending 56; the marks 33 and 23).
 //
 // Per (node, feature), by the node's size n:
 //   up to kListWave           one wave, sorted in its registers   (k_list_scan)
@@ -104,6 +108,16 @@ __global__ __launch_bounds__(kCodeThreads) void k_list_tables(const IdxT *rows, 
     // position it is the position's own flag)
     const bool first = r == 0 || p != (r % kCodeTile ? pf[r - 1] : 0u);
     if (first) v[base + p] = XT[(size_t)f * N + s];
+  }
+}
+
+// Row entries of all samples in ascending order (the list of a node that
+// holds every sample).
+template <class IdxT, class LabT>
+__global__ void k_list_all(const LabT *y, uint32_t N, IdxT *out) {
+  for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < N; s += gridDim.x * blockDim.x) {
+    if constexpr (sizeof(IdxT) == 4) out[s] = (IdxT)(s | ((uint32_t)y[s] << kIdBits));
+    else out[s] = (IdxT)s;
   }
 }
 
@@ -764,7 +778,7 @@ __device__ __forceinline__ void wg_filter(const FitArgs<IdxT, LabT> &a, const Id
                                           ScanRes *res, uint32_t *left) {
   const uint32_t lane = lane_id(), wave = uniform(threadIdx.x / kWave), K = (uint32_t)a.K, N = (uint32_t)a.N;
   const uint32_t nbits = label_bits(K), Wb = (N + 31u) / 32u;
-  const IdxT *row = a.si0 + (size_t)f * N;
+  const IdxT *row = a.presorted + (size_t)f * N;
   const uint32_t *col = a.rank + (size_t)f * N;
   uint32_t *q = set + Wb + wave * kQueue, *own = cnt + wave * K;
   constexpr int U = 4;

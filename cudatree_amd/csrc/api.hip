@@ -622,7 +622,7 @@ struct Fitter {
     if (w < 3) return w < list_kinds(N);
     return list_kinds(N) > 0 && (w == 3 ? ds->hist_max > 0 : ds->hist_small);
   }
-  size_t list_lds() const { return (size_t)kWavesPerBlock * list_wave_words((uint32_t)K, scan_regs) * 4; }
+  size_t list_lds() const { return (size_t)kWavesPerBlock * list_wave_words((uint32_t)K) * 4; }
 
   size_t smem() const { return (size_t)kWavesPerBlock * 2 * K * sizeof(uint32_t); }
 

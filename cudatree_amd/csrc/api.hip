@@ -262,10 +262,12 @@ struct cta_dataset {
   // distance that needs no test
   bool listed = false, hist_small = false;  // (hist_small: some feature suits the 4-wave count)
   uint32_t hist_max = 0;                    // largest table of the features that suit the 16-wave count
+  int few = -1;                             // few_valued, -1 before it was asked
   DevMem rank, dval, voff, gapw, ndist, all;  // (all: the list of every sample)
   // row-free features (two-valued, other than feature 0): tables of the fits
   // that keep no rows for them, and identity tables for fits that keep all
   int32_t Frl = 0, Wsig = 0, Fr = 0;
+  int32_t two = 0;  // two-valued features that keep rows all the same
   DevMem rl_of, slot_of, row_feat, rl_thr, sig;
   DevMem ident, rl_none;
 };
@@ -464,22 +466,59 @@ int list_kinds(int32_t N) {
   return n <= kListWave ? 0 : n <= kListWg[0] ? 1 : n <= kListWg[1] ? 2 : 3;
 }
 
-// Whether a fit searches its splits from sample lists (list_kernels.hip)
-// instead of sorted rows.
-bool list_search(const cta_ctx &ctx, const cta_dataset &ds, const cta_fit_opts &o) {
+// Whether most features that keep rows have few enough values to be counted by
+// value and class (from a sample of each presorted row; asked once of a set).
+template <class IdxT>
+bool few_valued(cta_ctx *ctx, cta_dataset *ds) {
+  if (ds->few < 0) {
+    uint32_t most = 0;
+    while (most < (uint32_t)(kListWaves[3] * kWave) &&
+           (size_t)list_wg_words(3, (uint32_t)ds->K, (uint32_t)ds->N, (most + 1u) * hist_stride((uint32_t)ds->K)) * 4 <=
+               ctx->lds_per_block)
+      ++most;
+    uint32_t *many = ctx->ws_as<uint32_t>("few_many", 1);
+    uint32_t *h = static_cast<uint32_t *>(ctx->host("few_many", 4));
+    k_fill_u32<<<1, 64, 0, ctx->stream>>>(many, 1, 0u);
+    k_list_many<IdxT><<<ds->F, 256, 0, ctx->stream>>>(ds->si0.as<IdxT>(), ds->XT.as<float>(), (uint32_t)ds->N, most, many);
+    HIPC(hipGetLastError());
+    HIPC(hipMemcpyAsync(h, many, 4, hipMemcpyDeviceToHost, ctx->stream));
+    ctx->sync();
+    ds->few = 4ull * h[0] <= (uint64_t)ds->Fr;
+  }
+  return ds->few != 0;
+}
+
+// Whether a fit of T trees searches its splits from sample lists
+// (list_kernels.hip) instead of sorted rows.
+template <class IdxT>
+bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T) {
   if (o.search == CTA_SEARCH_ROWS || o.mode != CTA_MODE_BATCHED || o.all_rows || o.subtree_max > 0) return false;
   // the words or the sample set of a node and its class counts must fit the LDS
-  for (int w = 0; w < list_kinds(ds.N); ++w)
-    if ((size_t)list_wg_words(w, (uint32_t)ds.K, (uint32_t)ds.N, 0) * 4 > ctx.lds_per_block) return false;
+  for (int w = 0; w < list_kinds(ds->N); ++w)
+    if ((size_t)list_wg_words(w, (uint32_t)ds->K, (uint32_t)ds->N, 0) * 4 > ctx->lds_per_block) return false;
   if (o.search == CTA_SEARCH_LISTS) return true;
-  // Rows move Fr rows per level where lists sort max_features of them, but a
-  // node's sort takes one workgroup where rows split it into chunks.  Rows /
-  // lists, ms: 20,000 x 4,096 (Fr / m = 64) 238 / 51; 7,490 x 233 (14) 7.5 /
-  // 5.3; 10,253 x 151, 6 trees (12) 3.8 / 3.8; 1,000,000 x 64 of 256 levels
-  // (8) 656 / 415; 1,797 x 64 of 17 levels (8) 2.0 / 2.0 (a set that small is
-  // bound by launches); 29,894 x 48 (7) 3.5 / 4.5; 581,012 x 54 with 10 rows
-  // (1.4) 31 / 71.
-  return (uint64_t)ds.Fr >= ((uint32_t)ds.N > kListWg[1] ? 8ull : 10ull) * (uint64_t)o.max_features;
+  // (a workspace limit that holds the rows may not hold the tables' scratch)
+  if (ctx->ws_limit && !ds->listed && ctx->ws_limit < ctx->ws_bytes() + (uint64_t)ds->N * ds->F * 4) return false;
+  // Rows move Fr rows of every tree per level where lists sort max_features of
+  // them, but a node's feature takes one workgroup where rows split it into
+  // chunks, and the tables cost about a presort: lists need enough trees.
+  // Rows / lists, ms, by samples x features, trees:
+  // - up to 4,096 samples, features >= 10 max_features: 3,000 x 128, 20: 2.5 /
+  //   2.2; 3,000 x 2,000, 20: 10.2 / 4.6; 600 x 400, 3: 2.7 / 1.8 (3,000 x 64
+  //   of 17 levels, 20: 1.8 / 1.8)
+  // - few-valued features: 600,000 x 49, 100: 78 / 30; 600,000 x 30, 20: 17 /
+  //   12; 200,000 x 36, 20: 8.2 / 7.3; but 600,000 x 49, 3: 8.2 / 8.8; 30,000 x
+  //   128, 20: 3.8 / 4.1
+  // - others: 230,000 x 256, 40: 74 / 54; 300,000 x 196, 40: 79 / 67; 30,000 x
+  //   256, 100: 17 / 13; 30,000 x 160, 100: 13 / 12; but 40,000 x 200, 40: 10.3
+  //   / 10.4; 370,000 x 160, 40: 93 / 104; 230,000 x 256, 3: 16 / 21
+  // A two-valued feature counts half: a rare value's list is read through in
+  // the constant test, where its row shows both ends (of 201 features 140
+  // such, 2,500 samples, 5 trees: 3.6 / 4.3; 990 of 1,000, 3,000: 12.5 / 10.0).
+  const int64_t Fr = ds->Fr - ds->two / 2, m = o.max_features;
+  if (ds->N <= (int32_t)kListWg[0]) return Fr >= 10 * m;
+  if ((Fr - 8 * m) * T >= 4000) return true;
+  return Fr >= 6 * m && Fr * T * ds->N >= (1ll << 27) && few_valued<IdxT>(ctx, ds);
 }
 
 // The list search's tables of a training set (kept with it; built on the
@@ -559,7 +598,7 @@ struct Fitter {
   uint32_t Jcap = 1;       // most fill workgroups per tree
   uint32_t *bsum = nullptr;
 
-  Fitter(cta_ctx *c, cta_dataset *d, const cta_fit_opts &opts) : ctx(c), ds(d), o(opts) {
+  Fitter(cta_ctx *c, cta_dataset *d, const cta_fit_opts &opts, bool lists) : ctx(c), ds(d), o(opts), list(lists) {
     N = d->N;
     F = d->F;
     K = d->K;
@@ -581,7 +620,6 @@ struct Fitter {
     slot_of_d = (rowfree ? d->slot_of : d->ident).as<int32_t>();
     row_feat_d = (rowfree ? d->row_feat : d->ident).as<int32_t>();
     Fc = Fr;
-    list = list_search(*c, *d, opts);
     if (list) Fr = 1;  // (feature 0 has the first row slot)
     // a wave-loop grid larger than what stays resident leaves a tail of
     // late workgroups; k_scan's registers allow fewer than 8 per CU
@@ -1432,11 +1470,12 @@ void append_trees(cta_forest *dst, const cta_forest *src, int32_t t, int32_t n) 
 template <class IdxT, class LabT>
 void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, const int64_t *off,
               const cta_fit_opts &o, cta_forest *out) {
-  if (list_search(*ctx, *ds, o)) {
+  const bool lists = list_search<IdxT>(ctx, ds, o, T);
+  if (lists) {
     list_tables<IdxT, LabT>(ctx, ds);
     if (o.lanes == 2) ctx->sync();  // (the other lane's stream reads them too)
   }
-  Fitter<IdxT, LabT> fz(ctx, ds, o);
+  Fitter<IdxT, LabT> fz(ctx, ds, o, lists);
   // trees resident at once on one stream: as asked, else what 60% of the
   // free memory holds (workspaces are reused by this fit)
   int32_t per = o.trees_per_batch;
@@ -1486,7 +1525,7 @@ void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, con
   std::thread th([&] {
     try {
       HIPC(hipSetDevice(lc->device));
-      Fitter<IdxT, LabT> fz1(lc, ds, o);
+      Fitter<IdxT, LabT> fz1(lc, ds, o, lists);
       for (size_t k = 1; k < b0.size(); k += 2) fz1.run_batch(b0[k], bsize(k), T, ids, off, &part[1]);
     } catch (...) {
       lane_err = std::current_exception();
@@ -1682,6 +1721,7 @@ void build_codes(cta_ctx *ctx, cta_dataset *ds, const uint32_t *keys, const uint
     } else {
       slot_of[f] = (int32_t)row_feat.size();
       row_feat.push_back((int32_t)f);
+      ds->two += fc_kind(fc[f]) == 1;
     }
   }
   ds->Frl = (int32_t)rl_feat.size();

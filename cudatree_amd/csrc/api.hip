@@ -783,9 +783,12 @@ struct Fitter {
       a.hist_max = ds->hist_max;
       for (int w = 0; w < kWgKinds; ++w) {
         if (!wg_used(w)) continue;
-        a.wg_tasks[w] = ctx->ws_as<Task>("wg_tasks" + std::to_string(w), cap_wg[w] * kXcd);
+        a.wg_tasks[w] = ctx->ws_as<Task>("wg_tasks" + std::to_string(w), cap_wg[w]);
         a.cap_wg[w] = (uint32_t)cap_wg[w];
       }
+      a.wg_cnt = ctx->ws_as<uint32_t>("wg_cnt", (size_t)kWgKinds * F);
+      a.wg_cur = ctx->ws_as<uint32_t>("wg_cur", (size_t)kWgKinds * F);
+      k_fill_u32<<<grid_for((size_t)kWgKinds * F), 256, 0, st>>>(a.wg_cnt, (size_t)kWgKinds * F, 0u);
     }
     a.rl_of = rl_of_d;
     a.slot_of = slot_of_d;
@@ -1256,6 +1259,12 @@ struct Fitter {
       if (list) k_select<IdxT, LabT, true><<<G, kBlock, 0, st>>>(a);
       else k_select<IdxT, LabT, false><<<G, kBlock, 0, st>>>(a);
       offsets<kSelFields>(a, q, &a.ctl->n_scan);
+      if (list && list_kinds(N) > 0) {
+        uint32_t kinds = 0;
+        for (int w = 0; w < kWgKinds; ++w) kinds |= wg_used(w) ? 1u << w : 0u;
+        if (F <= 256) k_wg_bins<1><<<1, kWave, 0, st>>>(a.ctl, a.wg_cnt, a.wg_cur, (uint32_t)F, kinds);
+        else k_wg_bins<16><<<1, 16 * kWave, 0, st>>>(a.ctl, a.wg_cnt, a.wg_cur, (uint32_t)F, kinds);
+      }
       if (list) k_select_emit<IdxT, LabT, true><<<G, kBlock, 0, st>>>(a);
       else k_select_emit<IdxT, LabT, false><<<G, kBlock, 0, st>>>(a);
     }

@@ -94,10 +94,9 @@ struct Ctl {
   // subtree wave takes, and the deepest node depth the subtree waves made
   uint32_t n_sub, sub_next, sub_depth;
   uint32_t bad;  // a workgroup's split failed its check: an error at the level's end
-  // list search: workgroup tasks of this level per kind and class
-  // (appended by the selection) and the next one a workgroup takes; both
-  // start every level at zero
-  uint32_t n_wg[kWgKinds][kXcd], wg_next[kWgKinds][kXcd];
+  // list search: workgroup tasks of this level per kind, and the next one of
+  // a class that a workgroup takes, zero at the start of every level
+  uint32_t n_wg[kWgKinds], wg_next[kWgKinds][kXcd];
   // after level `depth`: frontier size and ids in use, at depth % kLevelRing
   uint32_t lv_q[kLevelRing], lv_nodes[kLevelRing];
 };
@@ -197,8 +196,11 @@ struct FitArgs {
   const uint32_t *gapw;     // [F] indices this far apart always pass the candidate test
   const uint32_t *ndist;    // [F] distinct values
   uint32_t hist_max;        // most words of a (value, class) table the 16-wave count takes
-  Task *wg_tasks[kWgKinds];  // (node, feature) tasks by kind, kXcd lists of cap_wg each
+  Task *wg_tasks[kWgKinds];  // (node, feature) tasks by kind, in feature order
   uint32_t cap_wg[kWgKinds];
+  // [kWgKinds x F] tasks of a kind and feature: counted by the selection (zero
+  // at the start of every level), then where the next one is written
+  uint32_t *wg_cnt, *wg_cur;
   const int32_t *rl_of;     // [F] row-free index of each feature, or -1
   const int32_t *slot_of;   // [F] row slot of each feature, or -1
   const int32_t *row_feat;  // [Fr] feature of each row slot

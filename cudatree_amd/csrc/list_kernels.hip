@@ -1092,8 +1092,9 @@ __device__ __forceinline__ void wg_task(const FitArgs<IdxT, LabT> &a, const IdxT
   wg_scan<W, E, kRegs>(a, n, f, w, cnt, tot, tail, res, left);
 }
 
-// A workgroup per (node, feature).  The tasks of class c belong to the G
-// workgroups of XCD c (its L2 holds their columns): each starts with the task
+// A workgroup per (node, feature).  The tasks are in feature order; the c-th
+// eighth of them (class c) belongs to the G workgroups of XCD c, so that the
+// ones in flight share few columns in its L2: each starts with the task
 // of its own number, and any beyond the G-th are taken one at a time by
 // whoever is free, workgroups of other classes too -- nodes differ in size by
 // orders of magnitude, so no fixed split would be even.  A level with few
@@ -1105,11 +1106,12 @@ __global__ __launch_bounds__(kListWaves[kWg] * kWave) void k_list_wg(FitArgs<Idx
   extern __shared__ uint32_t smem[];
   const uint32_t K = (uint32_t)a.K;
   uint32_t *w = smem, *cnt = w + list_body_words(kWg, (uint32_t)a.N, a.hist_max), *tot = cnt + W * K, *tail = tot + K, *next = tail + W * 8u;
-  const uint32_t G = gridDim.x / kXcd;
+  const uint32_t G = gridDim.x / kXcd, total = min(uniform(a.ctl->n_wg[kWg]), a.cap_wg[kWg]);
   bool own = true;
   for (uint32_t turn = 0; turn < kXcd;) {
     const uint32_t cls = (blockIdx.x + turn) % kXcd;
-    const uint32_t count = min(uniform(a.ctl->n_wg[kWg][cls]), a.cap_wg[kWg]);
+    const uint32_t first = (uint32_t)((uint64_t)total * cls / kXcd);
+    const uint32_t count = (uint32_t)((uint64_t)total * (cls + 1u) / kXcd) - first;
     uint32_t item = blockIdx.x / kXcd;
     if (!own) {
       if (count <= G) {
@@ -1127,7 +1129,7 @@ __global__ __launch_bounds__(kListWaves[kWg] * kWave) void k_list_wg(FitArgs<Idx
       continue;
     }
     __syncthreads();  // (the last task's LDS is free)
-    const Task tk = a.wg_tasks[kWg][(size_t)cls * a.cap_wg[kWg] + item];
+    const Task tk = a.wg_tasks[kWg][first + item];
     const uint32_t i = uniform(tk.node), j = uniform(tk.first_count & 0xFFFFu);
     const FNode nd = a.front[i];
     const uint32_t n = uniform(nd.n);

@@ -1390,18 +1390,26 @@ struct Fitter {
     }
     k_canon_scatter<<<grid_for(n), 256, 0, st>>>(n, ar, size, pos, tr, toff, co);
     HIPC(hipGetLastError());
-    // copy out through pinned staging: each array is appended to the forest
-    // once its own copy has landed (an event per copy), the seven appends on
-    // threads of their own, so they overlap the copies and each other
+    // copy out through pinned staging, a piece of each of the seven arrays at a
+    // time.  The arrays are appended on threads of their own, which take the
+    // pages of the new part while the device still works and then copy each
+    // piece once it has landed (14 M nodes: 33 -> 24 ms).
     uint32_t *stage = static_cast<uint32_t *>(ctx->host("export", (size_t)n * 4 * 7 + ((size_t)Tb + 1) * 4));
     uint32_t *htoff = stage + (size_t)7 * n;
     HIPC(hipMemcpyAsync(htoff, toff, ((size_t)Tb + 1) * 4, hipMemcpyDeviceToHost, st));
     const void *srcs[7] = {co.feat, co.thr, co.left, co.right, co.value, co.nsamp, co.depth};
-    hipEvent_t evs[7];
-    for (int k = 0; k < 7; ++k) {
-      HIPC(hipMemcpyAsync(stage + (size_t)k * n, srcs[k], (size_t)n * 4, hipMemcpyDeviceToHost, st));
-      evs[k] = ctx->ev();
-      HIPC(hipEventRecord(evs[k], st));
+    constexpr uint32_t kPieces = 8, kPiece = 1u << 18;  // at most so many, of at least so many nodes
+    const uint32_t pieces = std::max(1u, std::min(kPieces, n / kPiece));
+    auto piece_at = [&](uint32_t c) { return (size_t)((uint64_t)n * c / pieces); };
+    hipEvent_t evs[kPieces * 7];
+    for (uint32_t c = 0; c < pieces; ++c) {
+      const size_t p0 = piece_at(c), np = piece_at(c + 1) - p0;
+      for (int k = 0; k < 7; ++k) {
+        HIPC(hipMemcpyAsync(stage + (size_t)k * n + p0, static_cast<const uint32_t *>(srcs[k]) + p0, np * 4,
+                            hipMemcpyDeviceToHost, st));
+        evs[c * 7 + k] = ctx->ev();
+        HIPC(hipEventRecord(evs[c * 7 + k], st));
+      }
     }
     if (only_batch) {
       out->nodes.alloc((size_t)n * sizeof(PNode));
@@ -1412,24 +1420,27 @@ struct Fitter {
     struct Done {  // returns the events to the context's pool
       cta_ctx *c;
       hipEvent_t *e;
+      uint32_t n;
       ~Done() {
-        for (int k = 0; k < 7; ++k) c->pool.push_back(e[k]);
+        for (uint32_t k = 0; k < n; ++k) c->pool.push_back(e[k]);
       }
-    } done{ctx, evs};
-    HIPC(hipEventSynchronize(evs[0]));  // the tree offsets landed before the first array
-    if (htoff[Tb] != n) fail(CTA_EINTERNAL, "canonical export counted %u of %u nodes", htoff[Tb], n);
+    } done{ctx, evs, pieces * 7};
     std::atomic<bool> ok{true};
     auto app = [&](auto &vec, int k) {
-      using V = typename std::decay_t<decltype(vec)>::value_type;
-      if (hipEventSynchronize(evs[k]) != hipSuccess) {
+      const size_t base = vec.size();
+      try {
+        vec.resize(base + n);
+      } catch (...) {
         ok = false;
         return;
       }
-      const V *p = reinterpret_cast<const V *>(stage + (size_t)k * n);
-      try {
-        vec.insert(vec.end(), p, p + n);
-      } catch (...) {
-        ok = false;
+      for (uint32_t c = 0; c < pieces; ++c) {
+        if (hipEventSynchronize(evs[c * 7 + (uint32_t)k]) != hipSuccess) {
+          ok = false;
+          return;
+        }
+        const size_t p0 = piece_at(c);
+        std::memcpy(vec.data() + base + p0, stage + (size_t)k * n + p0, (piece_at(c + 1) - p0) * 4);
       }
     };
     {
@@ -1449,6 +1460,7 @@ struct Fitter {
     }
     ctx->sync();
     if (!ok) fail(CTA_EINTERNAL, "copying the trees to host memory failed");
+    if (htoff[Tb] != n) fail(CTA_EINTERNAL, "canonical export counted %u of %u nodes", htoff[Tb], n);
     const int64_t base = out->tree_off.back();
     for (int32_t t = 1; t <= Tb; ++t) out->tree_off.push_back(base + htoff[t]);
     out->T += Tb;

@@ -263,7 +263,7 @@ __global__ __launch_bounds__(kOffThreads) void k_off_apply(const uint32_t *v, co
 constexpr uint32_t kListE = 16, kListWave = kWave * kListE;
 constexpr uint32_t kListWg[2] = {4096, 32768};
 #ifndef CTA_HIST_WORTH
-#define CTA_HIST_WORTH 4
+#define CTA_HIST_WORTH 8
 #endif
 constexpr uint32_t kHistWorth = CTA_HIST_WORTH;  // table words that one sample is worth clearing and scanning
 constexpr int kListWaves[kWgKinds] = {4, 16, 16, 16, 4};
@@ -272,8 +272,8 @@ constexpr int kListWaves[kWgKinds] = {4, 16, 16, 16, 4};
 // the banks), 64 values a wave.  The 4-wave count takes tables of up to
 // kHistSmall words at nodes of up to kHistSmallN samples (beyond, 16 waves
 // count faster); the 16-wave count tables of up to kHistWorth words a sample
-// (1,000,000 x 64 of 256 levels, 100 classes, per fit: 4 words 156 ms for all
-// large nodes, 8 words 156 ms, 16 words 183 ms).
+// (1,000,000 x 64 of 256 levels, 100 classes, per fit: 4 words 86 ms for all
+// large nodes, 8 words 79 ms, 12 words 86 ms).
 constexpr uint32_t kHistSmall = 4096, kHistSmallN = 16384;
 __host__ __device__ __forceinline__ uint32_t hist_stride(uint32_t K) { return K | 1u; }
 __host__ __device__ __forceinline__ bool hist_small(uint32_t D, uint32_t K) {

@@ -983,12 +983,29 @@ __device__ __forceinline__ void wg_filter(const FitArgs<IdxT, LabT> &a, const Id
   if (threadIdx.x == 0) put_res(res, t, f, found);
 }
 
+// Inclusive prefix sums over groups of V = 16, 32 or 64 lanes.
+template <int V>
+__device__ __forceinline__ uint32_t group_incl_scan(uint32_t v) {
+  if constexpr (V == 64) return wave_incl_scan(v);
+  v += dpp<kDppRowShr + 1>(v);
+  v += dpp<kDppRowShr + 2>(v);
+  v += dpp<kDppRowShr + 4>(v);
+  v += dpp<kDppRowShr + 8>(v);
+  if constexpr (V == 32) v += dpp<kDppBcast15, 0xA>(v);
+  return v;
+}
+
 // Split scan of a node over a feature of D <= 64 W values: the samples counted
 // by value and class in LDS (table h, hist_stride(K) words a value), then the
 // candidates between adjacent present values scored from the running class
 // counts, a lane a value.  No order of the samples is needed: per sample it
-// takes the value's code, the label and one LDS atomic.
-template <int W, class IdxT, class LabT>
+// takes the value's code, the label and one LDS atomic.  The table's part is
+// as long as the samples' at small nodes (at 1,000,000 x 64 of 256 levels, 100
+// classes, 9,300 samples a task), so all waves share it: V = 16, 32 or 64
+// values a wave, the wave's lanes over 64 / V classes at a time, and the left
+// counts summed by every wave (64 values a wave and the left counts by one
+// thread a class 52 ms, this way 39).
+template <int W, int V, class IdxT, class LabT>
 __device__ __forceinline__ void wg_hist(const FitArgs<IdxT, LabT> &a, const IdxT *list, uint32_t n, uint32_t f,
                                         uint32_t *h, uint32_t *cnt, const uint32_t *tot, uint32_t *tail, ScanRes *res,
                                         uint32_t *left) {
@@ -1014,8 +1031,9 @@ __device__ __forceinline__ void wg_hist(const FitArgs<IdxT, LabT> &a, const IdxT
       if (p + (uint32_t)u * (W * kWave) < n) atomicAdd(&h[x[u] * Kp + l[u]], 1u);
   }
   __syncthreads();
-  // class counts of the wave's 64 values, then those before them
-  const uint32_t v0 = min(wave * kWave, D), v1 = min(v0 + kWave, D);
+  // class counts of the wave's V values, then those before them
+  constexpr uint32_t G = kWave / V;
+  const uint32_t v0 = min(wave * V, D), v1 = min(v0 + V, D);
   uint32_t *own = cnt + wave * K;
   for (uint32_t k = lane; k < K; k += kWave) {
     uint32_t s = 0;
@@ -1023,20 +1041,31 @@ __device__ __forceinline__ void wg_hist(const FitArgs<IdxT, LabT> &a, const IdxT
     own[k] = s;
   }
   wg_prefix<W>(cnt, K);
-  const uint32_t v = v0 + lane;
+  // a lane a value and every G-th class, summed over the G groups of V lanes
+  const uint32_t g = lane / V, v = v0 + lane % V;
   const bool valid = v < v1;
   uint64_t SL = 0, Dd = 0, T2 = 0;
   uint32_t here = 0, nL = 0;
   if (v0 < v1)
-    for (uint32_t k = 0; k < K; ++k) {
-      const uint32_t x = valid ? h[v * Kp + k] : 0u, t = tot[k];
-      const uint32_t c = own[k] + wave_incl_scan(x);
+    for (uint32_t k0 = 0; k0 < K; k0 += G) {
+      const uint32_t k = k0 + g;
+      const uint32_t x = valid && k < K ? h[v * Kp + k] : 0u, t = k < K ? tot[k] : 0u;
+      const uint32_t c = (k < K ? own[k] : 0u) + group_incl_scan<V>(x);
       here += x;
       nL += c;
       SL += (uint64_t)c * c;
       Dd += (uint64_t)t * c;
       T2 += (uint64_t)t * t;
     }
+#pragma unroll
+  for (int o = V; o < kWave; o <<= 1) {
+    here += (uint32_t)__shfl_xor((int)here, o, kWave);
+    nL += (uint32_t)__shfl_xor((int)nL, o, kWave);
+    SL += (uint64_t)__shfl_xor((unsigned long long)SL, o, kWave);
+    Dd += (uint64_t)__shfl_xor((unsigned long long)Dd, o, kWave);
+    T2 += (uint64_t)__shfl_xor((unsigned long long)T2, o, kWave);
+  }
+  here = g == 0 ? here : 0u;  // (the first group goes on)
   const uint64_t present = ballot(here != 0u);
   if (lane == 0) tail[wave * 8u + 7u] = present ? v0 + (uint32_t)__ffsll((unsigned long long)present) - 1u : 0xFFFFFFFFu;
   __syncthreads();
@@ -1069,16 +1098,23 @@ __device__ __forceinline__ void wg_hist(const FitArgs<IdxT, LabT> &a, const IdxT
   if (found) {
     // left class counts: those before the winning wave's values and theirs up
     // to the split (they have to be the samples up to the split's position)
-    const uint32_t lo = t[5];
-    uint32_t sum = 0;
+    const uint32_t last = min(t[5], D - 1u);
+    uint32_t *acc = cnt + win * K;
     for (uint32_t k = lane; k < K; k += kWave) {
-      uint32_t s = cnt[win * K + k];
-      for (uint32_t x = win * kWave; x <= min(lo, D - 1u); ++x) s += h[x * Kp + k];
-      if (wave == 0) left[k] = s;
-      sum += s;
+      uint32_t s = 0;
+      for (uint32_t x = win * V + wave; x <= last; x += W) s += h[x * Kp + k];
+      if (s) atomicAdd(&acc[k], s);
     }
-    found = wave_sum32(sum) == t[4] + 1u;
-    if (!found && threadIdx.x == 0) a.ctl->bad = 1u;
+    __syncthreads();
+    if (wave == 0) {
+      uint32_t sum = 0;
+      for (uint32_t k = lane; k < K; k += kWave) {
+        left[k] = acc[k];
+        sum += acc[k];
+      }
+      found = wave_sum32(sum) == t[4] + 1u;
+      if (!found && lane == 0) a.ctl->bad = 1u;
+    }
   }
   if (threadIdx.x == 0) put_res(res, t, f, found);
 }
@@ -1142,7 +1178,10 @@ __global__ __launch_bounds__(kListWaves[kWg] * kWave) void k_list_wg(FitArgs<Idx
       if (n <= 2048) wg_task<kWg, 8, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
       else wg_task<kWg, 16, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
     } else if constexpr (kWg >= 3) {
-      wg_hist<W>(a, list, n, f, w, cnt, tot, tail, res, left);
+      const uint32_t D = uniform(a.ndist[f]);
+      if (D <= W * 16u) wg_hist<W, 16>(a, list, n, f, w, cnt, tot, tail, res, left);
+      else if (D <= W * 32u) wg_hist<W, 32>(a, list, n, f, w, cnt, tot, tail, res, left);
+      else wg_hist<W, 64>(a, list, n, f, w, cnt, tot, tail, res, left);
     } else if constexpr (kWg == 2) {
       wg_filter<W, kRegs>(a, list, n, f, w, cnt, tot, tail, res, left);
     } else {

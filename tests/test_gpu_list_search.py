@@ -1,9 +1,11 @@
 """Split search from sample lists (needs an MI355X): forests grown with
 search=CTA_SEARCH_LISTS equal the oracle's bit for bit, with root sizes on
 both sides of every limit between the sorts (a wave's 64 to 1,024 samples, a
-workgroup's 4,096 and 32,768, the filtered rows beyond), for features with gaps below the candidate
-test's, many ties, infinities, constants and two values, few and many
-classes, and both index widths."""
+workgroup's 4,096 and 32,768, the filtered rows beyond), for features with gaps
+below the candidate test's, many ties, infinities, constants and two values,
+few and many classes, both index widths, and numbers of distinct values on both
+sides of every limit of the counted features; and the fit's own choice grows
+the forest of either search."""
 import numpy as np
 import pytest
 
@@ -93,3 +95,37 @@ def test_full_depth(ctx, orc, idx_bits, opts):
     d = helpers.forest_diff(fit(ctx, case, _lib.CTA_SEARCH_LISTS, idx_bits=idx_bits, **opts),
                             helpers.oracle_forest(case, orc))
     assert d is None, d
+
+
+@pytest.mark.parametrize("D,K", [(64, 3), (65, 3), (128, 10), (129, 10), (256, 9), (256, 20), (257, 20), (512, 20),
+                                 (513, 3), (1024, 20), (1025, 3)])
+def test_counted_values(ctx, orc, D, K):
+    rng = np.random.Generator(np.random.PCG64(D))
+    n = 12001
+    y = rng.integers(0, K, size=n)
+    X = rng.integers(0, D, size=(n, 3)).astype(np.float32)
+    X[:, 1] = np.minimum(np.abs(rng.standard_normal(n) * D / 8 + y * D / (2 * K)).astype(np.int64), D - 1)
+    X[:D, :] = np.arange(D)[:, None]
+    case = {"X": X, "y": y, "K": K, "m": 3, "mss": 1, "max_depth": 4, "identity": False, "seed": D, "boot": False,
+            "n_trees": 2}
+    print("list counted D=%d K=%d" % (D, K), flush=True)
+    d = helpers.forest_diff(fit(ctx, case, _lib.CTA_SEARCH_LISTS), helpers.oracle_forest(case, orc))
+    assert d is None, d
+
+
+@pytest.mark.parametrize("n,F,m,T,levels", [(4096, 40, 4, 3, 0), (4097, 40, 4, 400, 0), (4097, 80, 6, 126, 0),
+                                            (40000, 48, 4, 70, 10), (40000, 48, 4, 69, 10), (40000, 48, 4, 70, 2)])
+def test_choice(ctx, n, F, m, T, levels):
+    """Both sides of the size rule, few and many values (levels = 0)."""
+    rng = np.random.Generator(np.random.PCG64(n + T))
+    y = rng.integers(0, 3, size=n)
+    X = (rng.standard_normal((n, F)) + y[:, None] * 0.3).astype(np.float32)
+    if levels:
+        X = np.clip(np.floor(X + levels / 2), 0, levels - 1).astype(np.float32)
+    case = {"X": X, "y": y, "K": 3, "m": m, "mss": 1, "max_depth": 5, "identity": False, "seed": 3, "boot": False,
+            "n_trees": T}
+    print("list choice", n, F, m, T, levels, flush=True)
+    auto = fit(ctx, case, _lib.CTA_SEARCH_AUTO)
+    for search in (_lib.CTA_SEARCH_ROWS, _lib.CTA_SEARCH_LISTS):
+        d = helpers.forest_diff(auto, fit(ctx, case, search))
+        assert d is None, d

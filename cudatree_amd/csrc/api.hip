@@ -1398,7 +1398,7 @@ struct Fitter {
     uint32_t *htoff = stage + (size_t)7 * n;
     HIPC(hipMemcpyAsync(htoff, toff, ((size_t)Tb + 1) * 4, hipMemcpyDeviceToHost, st));
     const void *srcs[7] = {co.feat, co.thr, co.left, co.right, co.value, co.nsamp, co.depth};
-    constexpr uint32_t kPieces = 8, kPiece = 1u << 18;  // at most so many, of at least so many nodes
+    constexpr uint32_t kPieces = 8, kPiece = 1u << 20;  // at most so many, of at least so many nodes
     const uint32_t pieces = std::max(1u, std::min(kPieces, n / kPiece));
     auto piece_at = [&](uint32_t c) { return (size_t)((uint64_t)n * c / pieces); };
     hipEvent_t evs[kPieces * 7];

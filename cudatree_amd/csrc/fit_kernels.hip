@@ -2096,6 +2096,7 @@ __device__ __forceinline__ void ctl_next_body(Ctl *ctl, unsigned long long *bslo
   }
   v = wave_sum64(v);
   if (slot == 0 && v) (&ctl->bytes_scan)[kind] += v;
+  if (tid < (uint32_t)kWgKinds * kXcd) (&ctl->wg_next[0][0])[tid] = 0;
   if (tid == 0) {
     if (ctl->bad) ctl->err |= kErrBadNode;
     // (after an error no next frontier was written: the later levels stay empty)
@@ -2105,8 +2106,6 @@ __device__ __forceinline__ void ctl_next_body(Ctl *ctl, unsigned long long *bslo
     ctl->c_live = 0;
     ctl->c_ids = 0;
     ctl->c_sub = 0;
-    for (int w = 0; w < kWgKinds; ++w)
-      for (uint32_t x = 0; x < kXcd; ++x) ctl->wg_next[w][x] = 0;
     // per-level record, so the host can read several levels at once
     const uint32_t d = (ctl->depth + 1) % kLevelRing;
     ctl->depth += 1;

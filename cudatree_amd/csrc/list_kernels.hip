@@ -12,14 +12,17 @@
 //
 // What bounds it: the sort's and the scan's VALU work (a bitonic network of
 // two instructions a step, about 120 a 64-sample tile at n = 1,024) and the
-// gathers of the words, one 4-byte word a sample from columns that the XCD
-// classes keep in L2; against that, sorted rows cost 9 bytes of HBM traffic a
-// sample and kept row.  20,000 x 4,096, 100 trees, 64 of 4,096 features a
-// node: reshuffle 170 -> 0.6 ms, split search 39 -> 35 ms, fit 239 -> 53 ms.
+// gathers of the words, a cache line a sample at sparse nodes, from columns
+// that the workgroup kernels' feature order keeps in L2; against that, sorted
+// rows cost 9 bytes of HBM traffic a sample and kept row.  Fits, rows / lists:
+// 20,000 x 4,096, 100 trees, 64 of 4,096 features a node 233 / 47 ms (reshuffle
+// 170 / 0.6); 200,000 x 256, 200 trees 299 / 138; 1,000,000 x 64 of 256
+// levels, 100 classes, 100 trees 690 / 273.
 //
 // Ascending lists make the gathers of a large node walk its columns in order,
 // several samples a cache line (with the lists in feature 0's order the counts
-// of 1,000,000 x 64 took 105 ms a fit, ascending 56; the marks 33 and 23).
+// of 1,000,000 x 64 took 105 ms a fit, ascending 56, when this came in; the marks
+// 33 and 23).
 //
 // Per (node, feature), by the node's size n:
 //   up to kListWave           one wave, sorted in its registers   (k_list_scan)

@@ -460,6 +460,9 @@ constexpr uint32_t kLevelGroup = CTA_LEVEL_GROUP;
 constexpr uint32_t kScanChunk = 1024, kReshChunk = 4096, kFillChunk = CTA_FILL_CHUNK;
 
 
+// LDS of a workgroup on this device (what a context reads back).
+constexpr size_t kMaxLds = 160 * 1024;
+
 // Workgroup kinds that the nodes of a training set of N samples can need.
 int list_kinds(int32_t N) {
   const uint32_t n = (uint32_t)N;
@@ -488,37 +491,51 @@ bool few_valued(cta_ctx *ctx, cta_dataset *ds) {
   return ds->few != 0;
 }
 
-// Whether a fit of T trees searches its splits from sample lists
-// (list_kernels.hip) instead of sorted rows.
-template <class IdxT>
-bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T) {
+// Whether a fit on N samples and K classes can search its splits from sample
+// lists (list_kernels.hip) at all.
+bool list_possible(int32_t N, int32_t K, const cta_fit_opts &o, size_t lds_per_block) {
   if (o.search == CTA_SEARCH_ROWS || o.mode != CTA_MODE_BATCHED || o.all_rows || o.subtree_max > 0) return false;
   // the words or the sample set of a node and its class counts must fit the LDS
-  for (int w = 0; w < list_kinds(ds->N); ++w)
-    if ((size_t)list_wg_words(w, (uint32_t)ds->K, (uint32_t)ds->N, 0) * 4 > ctx->lds_per_block) return false;
+  for (int w = 0; w < list_kinds(N); ++w)
+    if ((size_t)list_wg_words(w, (uint32_t)K, (uint32_t)N, 0) * 4 > lds_per_block) return false;
+  return true;
+}
+
+// The sizes from which lists are the faster search, in a fit of T trees on N
+// samples and Fr features with rows, m of them evaluated at a node; `few`: asked
+// when the answer depends on whether most of them have few values.
+// Rows move Fr rows of every tree per level where lists sort max_features of
+// them, but a node's feature takes one workgroup where rows split it into
+// chunks, and the tables cost about a presort: lists need enough trees.
+// Rows / lists, ms, by samples x features, trees:
+// - up to 4,096 samples, features >= 10 max_features: 3,000 x 128, 20: 2.5 /
+//   2.2; 3,000 x 2,000, 20: 10.2 / 4.6; 600 x 400, 3: 2.7 / 1.8 (3,000 x 64
+//   of 17 levels, 20: 1.8 / 1.8)
+// - few-valued features: 600,000 x 49, 100: 78 / 30; 600,000 x 30, 20: 17 /
+//   12; 200,000 x 36, 20: 8.2 / 7.3; but 600,000 x 49, 3: 8.2 / 8.8; 30,000 x
+//   128, 20: 3.8 / 4.1
+// - others: 230,000 x 256, 40: 74 / 54; 300,000 x 196, 40: 79 / 67; 30,000 x
+//   256, 100: 17 / 13; 30,000 x 160, 100: 13 / 12; but 40,000 x 200, 40: 10.3
+//   / 10.4; 370,000 x 160, 40: 93 / 104; 230,000 x 256, 3: 16 / 21
+template <class Few>
+bool list_worth(int32_t N, int64_t Fr, int64_t m, int64_t T, const Few &few) {
+  if (N <= (int32_t)kListWg[0]) return Fr >= 10 * m;
+  if ((Fr - 8 * m) * T >= 4000) return true;
+  return Fr >= 6 * m && Fr * T * N >= (1ll << 27) && few();
+}
+
+// Whether a fit of T trees searches its splits from sample lists instead of
+// sorted rows.
+template <class IdxT>
+bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T) {
+  if (!list_possible(ds->N, ds->K, o, ctx->lds_per_block)) return false;
   if (o.search == CTA_SEARCH_LISTS) return true;
   // (a workspace limit that holds the rows may not hold the tables' scratch)
   if (ctx->ws_limit && !ds->listed && ctx->ws_limit < ctx->ws_bytes() + (uint64_t)ds->N * ds->F * 4) return false;
-  // Rows move Fr rows of every tree per level where lists sort max_features of
-  // them, but a node's feature takes one workgroup where rows split it into
-  // chunks, and the tables cost about a presort: lists need enough trees.
-  // Rows / lists, ms, by samples x features, trees:
-  // - up to 4,096 samples, features >= 10 max_features: 3,000 x 128, 20: 2.5 /
-  //   2.2; 3,000 x 2,000, 20: 10.2 / 4.6; 600 x 400, 3: 2.7 / 1.8 (3,000 x 64
-  //   of 17 levels, 20: 1.8 / 1.8)
-  // - few-valued features: 600,000 x 49, 100: 78 / 30; 600,000 x 30, 20: 17 /
-  //   12; 200,000 x 36, 20: 8.2 / 7.3; but 600,000 x 49, 3: 8.2 / 8.8; 30,000 x
-  //   128, 20: 3.8 / 4.1
-  // - others: 230,000 x 256, 40: 74 / 54; 300,000 x 196, 40: 79 / 67; 30,000 x
-  //   256, 100: 17 / 13; 30,000 x 160, 100: 13 / 12; but 40,000 x 200, 40: 10.3
-  //   / 10.4; 370,000 x 160, 40: 93 / 104; 230,000 x 256, 3: 16 / 21
   // A two-valued feature counts half: a rare value's list is read through in
   // the constant test, where its row shows both ends (of 201 features 140
   // such, 2,500 samples, 5 trees: 3.6 / 4.3; 990 of 1,000, 3,000: 12.5 / 10.0).
-  const int64_t Fr = ds->Fr - ds->two / 2, m = o.max_features;
-  if (ds->N <= (int32_t)kListWg[0]) return Fr >= 10 * m;
-  if ((Fr - 8 * m) * T >= 4000) return true;
-  return Fr >= 6 * m && Fr * T * ds->N >= (1ll << 27) && few_valued<IdxT>(ctx, ds);
+  return list_worth(ds->N, ds->Fr - ds->two / 2, o.max_features, T, [&] { return few_valued<IdxT>(ctx, ds); });
 }
 
 // The list search's tables of a training set (kept with it; built on the
@@ -2404,19 +2421,23 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
     const uint64_t n = (uint64_t)N, f = (uint64_t)F, nf = n * f;
     const size_t b = N <= 65535 ? 2 : 4;
     const uint64_t lab = K <= 255 ? 1 : 2;
+    const int32_t m = opts->max_features > 0 ? opts->max_features : (int32_t)std::ceil(std::sqrt((double)F));
     // the dataset's own buffers: X_T, labels, presorted rows, code columns
     // (at most 16 bits per value), row-free signatures and feature tables,
     // plus the copies of host X and y while it is built
-    // and the list search's words and distinct values
     *dataset_bytes = nf * 4 + n * lab + nf * b + 2 * nf + 256 * f + 4 * n * ((f + 31) / 32) + 64 * f + 4096 +
-                     nf * 4 + n * 4 + nf * 8 + n * b + 20 * f;
+                     nf * 4 + n * 4;
+    // and the list search's words and distinct values, where the fit may choose
+    // it for data that suit it best (every feature with a row and few values)
+    if (list_possible(N, K, *opts, kMaxLds) &&
+        (opts->search == CTA_SEARCH_LISTS || list_worth(N, F, m, T, [] { return true; })))
+      *dataset_bytes += nf * 8 + n * b + 20 * f;
     // the context's workspaces: radix-sort and code-column temporaries of the
     // build, then per resident tree (every feature keeping rows), the node
     // arena and canonical export of at most two nodes per in-bag sample, and
     // the device predict table
     const uint64_t ntiles = (n + kSortTile - 1) / kSortTile;
     const uint64_t build = 6 * nf * 4 + f * kDigits * ntiles * 4 + 64 * f + ((n + kCodeTile - 1) / kCodeTile) * f * 4;
-    const int32_t m = opts->max_features > 0 ? opts->max_features : (int32_t)std::ceil(std::sqrt((double)F));
     const int64_t Tb = opts->mode != CTA_MODE_BATCHED ? 1
                        : opts->trees_per_batch > 0 ? std::min(opts->trees_per_batch, T)
                                                    : T;

@@ -1421,7 +1421,7 @@ __global__ __launch_bounds__(kBlock) void k_decide(FitArgs<IdxT, LabT> a) {
     uint32_t bt = 0;  // its task
     for (uint32_t t = lane; t < ax.scan_ntask; t += kWave) {
       const ScanRes r = a.res[ax.scan_base + t];
-      Cand c = {r.num, r.den, r.pos, r.feat, r.ok};
+      Cand c = {r.num, r.den, r.pos, r.feat, kList ? (r.num != 0 ? 1u : 0u) : r.ok};
       if (cand_better(c, best)) {
         best = c;
         bt = t;

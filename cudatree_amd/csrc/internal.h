@@ -56,13 +56,20 @@ struct Task {
   uint32_t node, first_count, chunk, nch;
 };
 
+// Over sorted rows `ok` says whether there is a split; the list search keeps the
+// value indices on both sides of it instead and has num = 0 for none.
 struct ScanRes {
   uint64_t num, den;
   uint32_t pos;
   int32_t feat;
-  uint32_t ok, pad;
-  uint32_t lo, hi;  // list search: value indices on both sides of the split
+  union {
+    uint32_t ok, lo;
+  };
+  union {
+    uint32_t pad, hi;
+  };
 };
+static_assert(sizeof(ScanRes) == 32, "a fit's result lists are sized by it");
 
 // Levels whose frontier size and id count are kept in Ctl.
 constexpr uint32_t kLevelRing = 64;

@@ -458,8 +458,6 @@ __device__ __forceinline__ ScanRes to_res(const Best<A> &b) {
   r.den = b.den;
   r.pos = b.pos;
   r.feat = b.feat;
-  r.ok = b.num != 0 ? 1u : 0u;
-  r.pad = 0;
   r.lo = b.lo;
   r.hi = b.hi;
   return r;
@@ -804,8 +802,6 @@ __device__ __forceinline__ void put_res(ScanRes *res, const uint32_t *t, uint32_
   r.den = found ? (uint64_t)t[3] << 32 | t[2] : 1ull;
   r.pos = t[4];
   r.feat = (int32_t)f;
-  r.ok = found ? 1u : 0u;
-  r.pad = 0;
   r.lo = t[5];
   r.hi = t[6];
   *res = r;

@@ -240,7 +240,9 @@ int cta_ctx_set_workspace_limit(cta_ctx *ctx, uint64_t bytes);
  * transient copies of host X and y) and a bound on the context workspaces a
  * fit of T trees with these options holds (the build's sort temporaries,
  * every resident tree's rows and level state, the node arena, the canonical
- * export and the predict table).  Computed on the host; no device is needed.
+ * export and the predict table).  A fit that may search from sample lists is
+ * charged their tables with the dataset; CTA_SEARCH_ROWS is not.  Computed on
+ * the host; no device is needed.
  * No counterpart in the reference (which allocates per tree without
  * accounting, random_forest.py:146-174, random_tree.py:255-282); the
  * serving loop admits fit jobs with it. */

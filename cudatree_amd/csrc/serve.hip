@@ -103,6 +103,7 @@ struct FitJob {
   int32_t N, F, K, T;
   cta_fit_opts opts;
   uint64_t est;     // admitted device bytes (dataset + workspace cap)
+  uint64_t est_rows;  // the same for a search over sorted rows (est where the job leaves no choice)
   uint64_t ws_cap;  // workspace cap of the fit context
 };
 
@@ -324,7 +325,7 @@ struct cta_server {
           if (stop && fq.empty()) return;
           if (!fq.empty()) {
             FitJob &h = fq.front();
-            if (h.est > budget) {  // can never fit: reject
+            if (std::min(h.est, h.est_rows) > budget) {  // can never fit: reject
               const uint64_t t = h.ticket;
               fq.pop_front();
               fit_rejected += 1;
@@ -332,6 +333,12 @@ struct cta_server {
               continue;
             }
             if (in_use + h.est <= budget) break;  // admit
+            if (in_use + h.est_rows <= budget) {
+              // no room for the list search's tables: the same trees from sorted rows
+              h.opts.search = CTA_SEARCH_ROWS;
+              h.est = h.est_rows;
+              break;
+            }
           }
           cv_fit.wait(lk);
         }
@@ -559,6 +566,14 @@ int cta_server_submit_fit(cta_server *s, const float *X, const uint32_t *y, int3
     uint64_t dsb = 0;
     fit_estimate(N, F, K, T, j.opts, &dsb, &j.ws_cap);
     j.est = dsb + j.ws_cap;
+    j.est_rows = j.est;
+    if (j.opts.search != CTA_SEARCH_LISTS) {
+      cta_fit_opts rows = j.opts;
+      rows.search = CTA_SEARCH_ROWS;
+      uint64_t ws = 0;
+      fit_estimate(N, F, K, T, rows, &dsb, &ws);
+      j.est_rows = dsb + ws;
+    }
     std::lock_guard<std::mutex> lk(s->mu);
     j.ticket = s->new_ticket_locked();
     *ticket = j.ticket;

@@ -256,7 +256,8 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
  * the rows of queued predict requests for one forest into one traversal
  * launch (requests arriving while a batch runs join the next batch), and
  * admits fit jobs only when their estimated device footprint fits the HBM
- * budget (a job larger than the whole budget fails with CTA_ENOMEM). */
+ * budget (a job larger than the whole budget fails with CTA_ENOMEM; one that
+ * fits only without the list search's tables runs with CTA_SEARCH_ROWS). */
 typedef struct cta_server cta_server;
 
 typedef struct {

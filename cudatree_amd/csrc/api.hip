@@ -264,6 +264,10 @@ struct cta_dataset {
   uint32_t hist_max = 0;                    // largest table of the features that suit the 16-wave count
   int few = -1;                             // few_valued, -1 before it was asked
   DevMem rank, dval, voff, gapw, ndist, all;  // (all: the list of every sample)
+  void drop_lists() {
+    for (DevMem *m : {&rank, &dval, &voff, &gapw, &ndist, &all}) m->release();
+    listed = false;
+  }
   // row-free features (two-valued, other than feature 0): tables of the fits
   // that keep no rows for them, and identity tables for fits that keep all
   int32_t Frl = 0, Wsig = 0, Fr = 0;
@@ -283,6 +287,15 @@ struct cta_forest {
   DevMem nodes, roots;     // pre-order predict table (PNode) and the trees' first nodes: the blocked table's source
   DevMem blocks, broots;   // blocked predict table (BNode) and each tree's root block
   bool device_ready = false;
+  void clear() {  // no trees
+    T = 0;
+    tree_off.assign(1, 0);
+    for (auto *v : {&left, &right, &value, &nsamp, &depth}) v->clear();
+    feature.clear();
+    threshold.clear();
+    for (DevMem *m : {&nodes, &roots, &blocks, &broots}) m->release();
+    device_ready = false;
+  }
 };
 
 // ---- allocation-free predict ---------------------------------------------------
@@ -479,7 +492,7 @@ bool few_valued(cta_ctx *ctx, cta_dataset *ds) {
            (size_t)list_wg_words(3, (uint32_t)ds->K, (uint32_t)ds->N, (most + 1u) * hist_stride((uint32_t)ds->K)) * 4 <=
                ctx->lds_per_block)
       ++most;
-    uint32_t *many = ctx->ws_as<uint32_t>("few_many", 1);
+    uint32_t *many = ctx->ws_as<uint32_t>("ds_err", 1);  // (the build's: no growth under a limit)
     uint32_t *h = static_cast<uint32_t *>(ctx->host("few_many", 4));
     k_fill_u32<<<1, 64, 0, ctx->stream>>>(many, 1, 0u);
     k_list_many<IdxT><<<ds->F, 256, 0, ctx->stream>>>(ds->si0.as<IdxT>(), ds->XT.as<float>(), (uint32_t)ds->N, most, many);
@@ -1505,14 +1518,10 @@ void append_trees(cta_forest *dst, const cta_forest *src, int32_t t, int32_t n) 
   dst->T += n;
 }
 
+// Grows the forest with the search decided on.
 template <class IdxT, class LabT>
-void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, const int64_t *off,
-              const cta_fit_opts &o, cta_forest *out) {
-  const bool lists = list_search<IdxT>(ctx, ds, o, T);
-  if (lists) {
-    list_tables<IdxT, LabT>(ctx, ds);
-    if (o.lanes == 2) ctx->sync();  // (the other lane's stream reads them too)
-  }
+void fit_grow(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, const int64_t *off,
+              const cta_fit_opts &o, bool lists, cta_forest *out) {
   Fitter<IdxT, LabT> fz(ctx, ds, o, lists);
   // trees resident at once on one stream: as asked, else what 60% of the
   // free memory holds (workspaces are reused by this fit)
@@ -1621,6 +1630,39 @@ void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, con
     build_blocks(ctx, out, dep);
     out->device_ready = true;
   }
+}
+
+// Grows the forest.  The list search needs tables, and task lists of other
+// sizes than the rows': where they cannot be had the rows are searched, and
+// rows that lack the memory the tables of an earlier fit hold take it.
+template <class IdxT, class LabT>
+void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, const int64_t *off,
+              const cta_fit_opts &o, cta_forest *out) {
+  auto start_over = [&] {  // nothing of the attempt stays
+    ctx->sync();
+    if (ctx->lane) ctx->lane->sync();
+    ds->drop_lists();
+    ctx->ws_release();
+    if (ctx->lane) ctx->lane->ws_release();
+    out->clear();
+  };
+  if (list_search<IdxT>(ctx, ds, o, T)) {
+    try {
+      list_tables<IdxT, LabT>(ctx, ds);
+      if (o.lanes == 2) ctx->sync();  // (the other lane's stream reads them too)
+      return fit_grow<IdxT, LabT>(ctx, ds, T, ids, off, o, true, out);
+    } catch (const Error &e) {
+      if (e.code != CTA_ENOMEM && e.code != CTA_EUNSUPPORTED) throw;
+    }
+    start_over();
+  }
+  try {
+    return fit_grow<IdxT, LabT>(ctx, ds, T, ids, off, o, false, out);
+  } catch (const Error &e) {
+    if (e.code != CTA_ENOMEM || !ds->listed) throw;
+  }
+  start_over();
+  fit_grow<IdxT, LabT>(ctx, ds, T, ids, off, o, false, out);
 }
 
 void build_codes(cta_ctx *ctx, cta_dataset *ds, const uint32_t *keys, const uint32_t *ids);

@@ -132,7 +132,8 @@ typedef struct {
   int32_t search;            /* how a batched fit finds its splits: CTA_SEARCH_AUTO (0), CTA_SEARCH_ROWS (1: over
                                 sorted rows of every feature, moved at every level) or CTA_SEARCH_LISTS (2: from
                                 the nodes' sample lists, sorting the features a node evaluates, where the sizes
-                                allow it, else rows); other values are taken as 0.  The trees are identical */
+                                and the memory for its tables allow it, else rows); other values are taken as 0.
+                                The trees are identical */
 } cta_fit_opts;
 
 #define CTA_SEARCH_AUTO 0

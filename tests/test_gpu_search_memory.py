@@ -48,3 +48,90 @@ def test_server_admits_what_sorted_rows_need(spare):
         assert s["fit_rejected"] == 0 and s["hbm_peak"] <= rows + spare and s["fit_mem_ratio_max"] <= 1.0, s
     finally:
         srv.close()
+
+
+class Hog:
+    """Device memory taken until about `leave` bytes are free."""
+
+    def __init__(self, ctx, leave):
+        self.held = []
+        chunk = 16 << 30
+        while chunk >= 1 << 20:
+            if ctx.mem_info()[0] <= leave + chunk:
+                chunk >>= 1
+                continue
+            self.held.append(helpers.DeviceArray(chunk, np.uint8))
+
+    def free(self):
+        for d in self.held:
+            d.free()
+
+
+def searches(ctx, fit):
+    """fit()'s result and whether rows were searched, and lists, in it."""
+    ctx.reset_stats()
+    ctx.set_profiling(True)
+    try:
+        out = fit()
+    finally:
+        ctx.set_profiling(False)
+    st = ctx.kernel_stats()
+    return out, "k_scan_hist" in st, "k_select" in st and "k_scan_hist" not in st
+
+
+def test_rows_where_the_list_tables_do_not_fit():
+    """60,000 x 1,000, one tree's rows 240 MB, the tables 480 MB and their
+    scratch 240 MB: with 600 MB free the fit's own choice is lists, and the
+    trees come from rows.  Then the other way round: tables of an earlier fit
+    make way for rows that need their memory."""
+    N, F, K, T, m = 60000, 1000, 5, 5, 10
+    X, y = gauss(N, F, K, 2)
+    ctx = _lib.Context(0)
+    ds = _lib.Dataset(ctx, X, y, K)
+    assert ds.idx_bits == 16
+
+    def fit(**kw):
+        return _lib.Forest.fit(ctx, ds, T, opts(m, **kw), None).export()
+
+    want = fit(search=_lib.CTA_SEARCH_ROWS)
+    ctx.release_workspace()
+    print("tables that do not fit", flush=True)
+    free0 = ctx.mem_info()[0]
+    hog = Hog(ctx, 600 << 20)
+    try:
+        got, rows, lists = searches(ctx, fit)
+    finally:
+        hog.free()
+    assert rows and helpers.forest_diff(got, want) is None
+    ctx.release_workspace()
+    assert ctx.mem_info()[0] >= free0 - (32 << 20)  # nothing of the tables stayed
+    got, rows, lists = searches(ctx, fit)
+    assert lists and not rows and helpers.forest_diff(got, want) is None
+    ctx.release_workspace()
+    print("tables that make way", flush=True)
+    hog = Hog(ctx, 200 << 20)
+    try:
+        got, rows, lists = searches(ctx, lambda: fit(search=_lib.CTA_SEARCH_ROWS))
+    finally:
+        hog.free()
+    assert rows and helpers.forest_diff(got, want) is None
+    ds.close()
+    ctx.close()
+
+
+def test_rows_where_the_list_tasks_do_not_fit_their_indices():
+    """1,100 x 65,535 with every feature evaluated at 1,024 classes: the class
+    counts of the list search's workgroup tasks pass 32 bits, those of the rows
+    (one chunk a node) do not."""
+    N, F, K = 1100, 65535, 1024
+    rng = np.random.Generator(np.random.PCG64(3))
+    y = rng.permutation(np.arange(N) % K)
+    X = rng.integers(0, 3, size=(N, F)).astype(np.float32)
+    ctx = _lib.Context(0)
+    ds = _lib.Dataset(ctx, X, y, K)
+    print("task indices", flush=True)
+    trees = [_lib.Forest.fit(ctx, ds, 1, opts(F, search=s, bootstrap=0, max_depth=1, scan_chunk=1 << 20), None).export()
+             for s in (_lib.CTA_SEARCH_ROWS, _lib.CTA_SEARCH_LISTS)]
+    assert len(trees[0]["feature"]) == 3 and helpers.forest_diff(*trees) is None
+    ds.close()
+    ctx.close()

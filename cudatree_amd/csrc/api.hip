@@ -165,6 +165,13 @@ struct cta_ctx {
     for (auto &kv : wspace) b += kv.second ? kv.second->bytes : 0;
     return b;
   }
+  // Bytes by which a workspace would grow to hold `bytes`.
+  size_t ws_growth(const std::string &key, size_t bytes) const {
+    const auto it = wspace.find(key);
+    const size_t held = it != wspace.end() && it->second ? it->second->bytes : 0;
+    return bytes > held ? bytes - held : 0;
+  }
+  void ws_drop(const std::string &key) { wspace.erase(key); }
   void ws_release() { wspace.clear(); }
   // Pinned host memory the device writes directly (mapped, coherent): the
   // host pointer; *dev receives the device's address for it.
@@ -543,8 +550,15 @@ template <class IdxT>
 bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T) {
   if (!list_possible(ds->N, ds->K, o, ctx->lds_per_block)) return false;
   if (o.search == CTA_SEARCH_LISTS) return true;
-  // (a workspace limit that holds the rows may not hold the tables' scratch)
-  if (ctx->ws_limit && !ds->listed && ctx->ws_limit < ctx->ws_bytes() + (uint64_t)ds->N * ds->F * 4) return false;
+  // (a workspace limit that holds the rows may not hold the tables' scratch,
+  // as far as the dataset's build has not left it)
+  if (ctx->ws_limit && !ds->listed) {
+    const size_t NF = (size_t)ds->N * ds->F, tiles = ((size_t)ds->N + kCodeTile - 1) / kCodeTile;
+    if (ctx->ws_bytes() + ctx->ws_growth("code_pre", NF * 4) + ctx->ws_growth("code_tsum", tiles * ds->F * 4) +
+            ctx->ws_growth("code_meta", 8 * (size_t)ds->F) >
+        ctx->ws_limit)
+      return false;
+  }
   // A two-valued feature counts half: a rare value's list is read through in
   // the constant test, where its row shows both ends (of 201 features 140
   // such, 2,500 samples, 5 trees: 3.6 / 4.3; 990 of 1,000, 3,000: 12.5 / 10.0).
@@ -560,6 +574,7 @@ void list_tables(cta_ctx *ctx, cta_dataset *ds) {
   hipStream_t st = ctx->stream;
   Timed tm(ctx, "k_list_tables");
   const uint32_t ntiles = (N + kCodeTile - 1) / kCodeTile;
+  const bool grown = ctx->ws_growth("code_pre", (size_t)N * F * 4) != 0;
   uint32_t *pre = ctx->ws_as<uint32_t>("code_pre", (size_t)N * F);
   uint32_t *tsum = ctx->ws_as<uint32_t>("code_tsum", (size_t)ntiles * F);
   uint32_t *bad = ctx->ws_as<uint32_t>("code_meta", 2 * (size_t)F);
@@ -601,6 +616,10 @@ void list_tables(cta_ctx *ctx, cta_dataset *ds) {
   k_list_gapw<<<dim3(std::min<uint32_t>(64, ntiles), F), kCodeThreads, 0, st>>>(
       ds->dval.as<float>(), ds->voff.as<uint64_t>(), nd, bad, ds->gapw.as<uint32_t>());
   HIPC(hipGetLastError());
+  if (ctx->ws_limit && grown) {  // what the limit leaves is for the trees
+    ctx->sync();
+    ctx->ws_drop("code_pre");
+  }
   ds->listed = true;
 }
 

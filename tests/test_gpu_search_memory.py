@@ -1,6 +1,8 @@
 """Memory and the choice of search (needs an MI355X): the list search's tables
 take device memory that sorted rows do not, so a fit that may use either goes
 back to rows where they do not fit, and grows the same trees."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -133,5 +135,42 @@ def test_rows_where_the_list_tasks_do_not_fit_their_indices():
     trees = [_lib.Forest.fit(ctx, ds, 1, opts(F, search=s, bootstrap=0, max_depth=1, scan_chunk=1 << 20), None).export()
              for s in (_lib.CTA_SEARCH_ROWS, _lib.CTA_SEARCH_LISTS)]
     assert len(trees[0]["feature"]) == 3 and helpers.forest_diff(*trees) is None
+    ds.close()
+    ctx.close()
+
+
+def limited(ctx, spare=None):
+    """Sets the context's workspace limit to what it holds and `spare` bytes."""
+    held = ctypes.c_uint64()
+    _lib.check(ctx.lib.cta_ctx_workspace_bytes(ctx.h, ctypes.byref(held)))
+    _lib.check(ctx.lib.cta_ctx_set_workspace_limit(ctx.h, held.value + spare if spare is not None else 0))
+    return held.value
+
+
+def test_limited_context_builds_tables_in_the_scratch_it_holds():
+    """3,000 x 2,000: the scratch of the tables (24 MB) is what the dataset's
+    build left, so lists need next to nothing more; and after a release a limit
+    that one tree's rows fit holds the tables' scratch as well."""
+    N, F, K, T, m = 3000, 2000, 5, 3, 45
+    X, y = gauss(N, F, K, 4)
+    ctx = _lib.Context(0)
+    ds = _lib.Dataset(ctx, X, y, K)
+
+    def fit(**kw):
+        return _lib.Forest.fit(ctx, ds, T, opts(m, **kw), None).export()
+
+    want = fit(search=_lib.CTA_SEARCH_ROWS)
+    print("limited context", flush=True)
+    limited(ctx, 1 << 20)
+    got, rows, lists = searches(ctx, fit)
+    assert lists and not rows and helpers.forest_diff(got, want) is None
+    ds.close()
+    limited(ctx)
+    ds = _lib.Dataset(ctx, X, y, K)
+    ctx.release_workspace()
+    limited(ctx, 28 << 20)
+    got, rows, lists = searches(ctx, fit)
+    assert lists and not rows and helpers.forest_diff(got, want) is None
+    assert limited(ctx) <= 20 << 20  # the scratch was given back
     ds.close()
     ctx.close()

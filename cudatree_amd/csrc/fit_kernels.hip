@@ -472,7 +472,8 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
         }
       }
       if constexpr (kList) {
-        const bool want = k < F && jr < 0;
+        // (a feature of one value over the whole set is not read at all)
+        const bool want = k < F && jr < 0 && a.ndist[f] > 1u;
         nonconst |= list_varies(list, n, index_col(a, want ? f : 0u), want, ballot(nonconst), m - nsel);
       }
       const uint64_t mk = ballot(nonconst);

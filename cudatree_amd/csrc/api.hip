@@ -259,6 +259,15 @@ struct Timed {
 };
 
 // ---- dataset -------------------------------------------------------------------
+// How the values of a training set's features are spread, as the choice of search
+// takes it.  A feature's rare share is the share of samples that do not hold its
+// middle value: next to nothing for a column of zeros with a few counts in it.
+struct Spread {
+  bool few = true;     // most features with rows have few enough values to be counted by value and class
+  double rare = 1.0;   // mean rare share of the features of more than one value
+  double drag = 0.0;   // mean cost of the constant tests per feature with a row (see spread_of)
+};
+
 struct cta_dataset {
   cta_ctx *ctx = nullptr;
   int32_t N = 0, F = 0, K = 0, idx_bits = 32, lab_bits = 8;
@@ -269,7 +278,7 @@ struct cta_dataset {
   // distance that needs no test
   bool listed = false, hist_small = false;  // (hist_small: some feature suits the 4-wave count)
   uint32_t hist_max = 0;                    // largest table of the features that suit the 16-wave count
-  int few = -1;                             // few_valued, -1 before it was asked
+  Spread spread;                            // of its features' values
   DevMem rank, dval, voff, gapw, ndist, all;  // (all: the list of every sample)
   void drop_lists() {
     for (DevMem *m : {&rank, &dval, &voff, &gapw, &ndist, &all}) m->release();
@@ -489,28 +498,6 @@ int list_kinds(int32_t N) {
   return n <= kListWave ? 0 : n <= kListWg[0] ? 1 : n <= kListWg[1] ? 2 : 3;
 }
 
-// Whether most features that keep rows have few enough values to be counted by
-// value and class (from a sample of each presorted row; asked once of a set).
-template <class IdxT>
-bool few_valued(cta_ctx *ctx, cta_dataset *ds) {
-  if (ds->few < 0) {
-    uint32_t most = 0;
-    while (most < (uint32_t)(kListWaves[3] * kWave) &&
-           (size_t)list_wg_words(3, (uint32_t)ds->K, (uint32_t)ds->N, (most + 1u) * hist_stride((uint32_t)ds->K)) * 4 <=
-               ctx->lds_per_block)
-      ++most;
-    uint32_t *many = ctx->ws_as<uint32_t>("ds_err", 1);  // (the build's: no growth under a limit)
-    uint32_t *h = static_cast<uint32_t *>(ctx->host("few_many", 4));
-    k_fill_u32<<<1, 64, 0, ctx->stream>>>(many, 1, 0u);
-    k_list_many<IdxT><<<ds->F, 256, 0, ctx->stream>>>(ds->si0.as<IdxT>(), ds->XT.as<float>(), (uint32_t)ds->N, most, many);
-    HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(h, many, 4, hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    ds->few = 4ull * h[0] <= (uint64_t)ds->Fr;
-  }
-  return ds->few != 0;
-}
-
 // Whether a fit on N samples and K classes can search its splits from sample
 // lists (list_kernels.hip) at all.
 bool list_possible(int32_t N, int32_t K, const cta_fit_opts &o, size_t lds_per_block) {
@@ -521,9 +508,41 @@ bool list_possible(int32_t N, int32_t K, const cta_fit_opts &o, size_t lds_per_b
   return true;
 }
 
+// The spread of a training set's values from the samples of k_spread.  Where a
+// feature is constant in a node, rows see it at both ends of a segment, but a
+// list has to be read through, by one wave if it is long: that cost per feature
+// goes with about one over the square root of its rare share.  A mean of the
+// measured slowdown (300 and 1,000 features, 30 and 60% of them of a rare share
+// of 0.0003 to 0.03) is 1.04, 0.57, 0.33, 0.18, 0.10 of what rows spend to move
+// the feature at 0.0003, 0.001, 0.003, 0.01, 0.03; row-free and constant
+// features cost nothing.
+Spread spread_of(const uint32_t *sampled, const int32_t *rl_of, const cta_dataset *ds, size_t lds_per_block) {
+  const uint32_t F = (uint32_t)ds->F, K = (uint32_t)ds->K;
+  uint32_t most = 0;  // values whose table fits the 16-wave count
+  while (most < (uint32_t)(kListWaves[3] * kWave) &&
+         (size_t)list_wg_words(3, K, (uint32_t)ds->N, (most + 1u) * hist_stride(K)) * 4 <= lds_per_block)
+    ++most;
+  double rare = 0, drag = 0;
+  uint64_t vary = 0, many = 0;
+  for (uint32_t f = 0; f < F; ++f) {
+    const uint32_t changes = sampled[f] & 0xFFFFu;
+    if (!changes) continue;
+    // (one of the two ends is always another value)
+    const double r = std::max(0.0, kSpreadSamples - (double)(sampled[f] >> 16)) / kSpreadSamples;
+    ++vary;
+    rare += r;
+    many += changes >= most;
+    if (rl_of[f] < 0) drag += std::min(1.3, std::max(0.0, 0.018 / std::sqrt(std::max(r, 1e-6)) - 0.03));
+  }
+  Spread sp;
+  sp.few = 4 * many <= (uint64_t)ds->Fr;
+  if (vary) sp.rare = rare / (double)vary;
+  sp.drag = drag / (double)ds->Fr;
+  return sp;
+}
+
 // The sizes from which lists are the faster search, in a fit of T trees on N
-// samples and Fr features with rows, m of them evaluated at a node; `few`: asked
-// when the answer depends on whether most of them have few values.
+// samples and Fr features with rows, m of them evaluated at a node.
 // Rows move Fr rows of every tree per level where lists sort max_features of
 // them, but a node's feature takes one workgroup where rows split it into
 // chunks, and the tables cost about a presort: lists need enough trees.
@@ -537,16 +556,26 @@ bool list_possible(int32_t N, int32_t K, const cta_fit_opts &o, size_t lds_per_b
 // - others: 230,000 x 256, 40: 74 / 54; 300,000 x 196, 40: 79 / 67; 30,000 x
 //   256, 100: 17 / 13; 30,000 x 160, 100: 13 / 12; but 40,000 x 200, 40: 10.3
 //   / 10.4; 370,000 x 160, 40: 93 / 104; 230,000 x 256, 3: 16 / 21
-template <class Few>
-bool list_worth(int32_t N, int64_t Fr, int64_t m, int64_t T, const Few &few) {
-  if (N <= (int32_t)kListWg[0]) return Fr >= 10 * m;
-  if ((Fr - 8 * m) * T >= 4000) return true;
-  return Fr >= 6 * m && Fr * T * N >= (1ll << 27) && few();
+// Where the m features of a node hold few rare values between them, its splits
+// cut off a few samples each, the trees become long chains of large nodes and
+// most features are constant in them: 20,000 x 300, 40 trees, every feature of
+// a rare share of 0.001 / 0.01 / 0.03 / 0.1: 234 / 2,310, 155 / 398, 70 / 66,
+// 28 / 18; 100,000 x 300 of 0.01, 30 trees: 372 / 1,411; 20,000 x 1,000 of
+// 0.01, 20 trees: 224 / 219.  Beside dense features rare values only drag the
+// constant tests: 20,000 x 1,000, 20 trees, 60% of the features of a rare share
+// of 0.0003 / 0.001 / 0.01: 13.1 / 16.0, 13.1 / 11.3, 13.9 / 8.4; small sets,
+// where the tests weigh more, 3,000 x 300, 20 trees, 30% of 0.003: 2.7 / 3.1.
+bool list_worth(int64_t N, double Fr, int64_t m, int64_t T, const Spread &sp) {
+  if ((double)m * sp.rare < 0.5) return false;
+  if (N <= (int64_t)kListWg[0]) return Fr * (1.0 - 5.0 * sp.drag) >= 10.0 * (double)m;
+  if ((Fr - 8.0 * (double)m) * (double)T >= 4000.0 && (Fr * (1.0 - sp.drag) - 8.0 * (double)m) * (double)T >= 2700.0)
+    return true;
+  const double Fc = Fr * (1.0 - 2.0 * sp.drag);  // (20,000 x 1,000, 95% two-valued of 0.003, 20 trees: 23 / 27)
+  return sp.few && Fc >= 6.0 * (double)m && Fc * (double)T * (double)N >= 0x1p27;
 }
 
 // Whether a fit of T trees searches its splits from sample lists instead of
 // sorted rows.
-template <class IdxT>
 bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T) {
   if (!list_possible(ds->N, ds->K, o, ctx->lds_per_block)) return false;
   if (o.search == CTA_SEARCH_LISTS) return true;
@@ -562,7 +591,7 @@ bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T
   // A two-valued feature counts half: a rare value's list is read through in
   // the constant test, where its row shows both ends (of 201 features 140
   // such, 2,500 samples, 5 trees: 3.6 / 4.3; 990 of 1,000, 3,000: 12.5 / 10.0).
-  return list_worth(ds->N, ds->Fr - ds->two / 2, o.max_features, T, [&] { return few_valued<IdxT>(ctx, ds); });
+  return list_worth(ds->N, (double)(ds->Fr - ds->two / 2), o.max_features, T, ds->spread);
 }
 
 // The list search's tables of a training set (kept with it; built on the
@@ -1665,7 +1694,7 @@ void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, con
     if (ctx->lane) ctx->lane->ws_release();
     out->clear();
   };
-  if (list_search<IdxT>(ctx, ds, o, T)) {
+  if (list_search(ctx, ds, o, T)) {
     try {
       list_tables<IdxT, LabT>(ctx, ds);
       if (o.lanes == 2) ctx->sync();  // (the other lane's stream reads them too)
@@ -1776,8 +1805,10 @@ void build_codes(cta_ctx *ctx, cta_dataset *ds, const uint32_t *keys, const uint
   k_code_flags<<<dim3(ntiles, F), kCodeThreads, 0, st>>>(keys, N, ntiles, pre, tsum, db + F);
   k_code_tscan<<<F, 1024, 0, st>>>(tsum, ntiles, db);
   k_code_scatter<<<dim3(ntiles, F), kCodeThreads, 0, st>>>(ids, pre, tsum, N, ntiles, d);
-  uint32_t *h = static_cast<uint32_t *>(ctx->host("code_meta", 2 * (size_t)F * 4));
+  k_spread<<<F, 256, 0, st>>>(keys, N, tsum);  // (the tile totals are no longer needed)
+  uint32_t *h = static_cast<uint32_t *>(ctx->host("code_meta", 3 * (size_t)F * 4));
   HIPC(hipMemcpyAsync(h, db, 2 * (size_t)F * 4, hipMemcpyDeviceToHost, st));
+  HIPC(hipMemcpyAsync(h + 2 * (size_t)F, tsum, (size_t)F * 4, hipMemcpyDeviceToHost, st));
   ctx->sync();
   std::vector<uint64_t> fc(F);
   uint64_t off = 0;
@@ -1826,6 +1857,7 @@ void build_codes(cta_ctx *ctx, cta_dataset *ds, const uint32_t *keys, const uint
   ds->Frl = (int32_t)rl_feat.size();
   ds->Wsig = (ds->Frl + 31) / 32;
   ds->Fr = (int32_t)row_feat.size();
+  ds->spread = spread_of(h + 2 * (size_t)F, rl_of, ds, ctx->lds_per_block);
   int32_t *ht = static_cast<int32_t *>(ctx->host("rl_tables", ((size_t)6 * F + 2) * 4));
   std::memcpy(ht, tab.data(), (size_t)4 * F * 4);
   std::memcpy(ht + 4 * F, row_feat.data(), row_feat.size() * 4);
@@ -2489,9 +2521,9 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
     *dataset_bytes = nf * 4 + n * lab + nf * b + 2 * nf + 256 * f + 4 * n * ((f + 31) / 32) + 64 * f + 4096 +
                      nf * 4 + n * 4;
     // and the list search's words and distinct values, where the fit may choose
-    // it for data that suit it best (every feature with a row and few values)
+    // it for data that suit it best (every feature with a row, dense, of few values)
     if (list_possible(N, K, *opts, kMaxLds) &&
-        (opts->search == CTA_SEARCH_LISTS || list_worth(N, F, m, T, [] { return true; })))
+        (opts->search == CTA_SEARCH_LISTS || list_worth(N, F, m, T, Spread{})))
       *dataset_bytes += nf * 8 + n * b + 20 * f;
     // the context's workspaces: radix-sort and code-column temporaries of the
     // build, then per resident tree (every feature keeping rows), the node

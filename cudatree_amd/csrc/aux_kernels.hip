@@ -455,6 +455,29 @@ __global__ __launch_bounds__(kCodeThreads) void k_code_flags(const uint32_t *key
   if (tid == kCodeThreads - 1) tsum[(size_t)f * ntiles + blockIdx.x] = run;
 }
 
+// How a feature's values are spread (a workgroup each), from kSpreadSamples + 1
+// evenly spaced positions of its sorted keys, both ends among them: out[f] = the
+// value changes between neighbours (none: the feature has one value), and in
+// the high half how many positions hold the middle one's value.
+constexpr uint32_t kSpreadSamples = 2048;
+__global__ __launch_bounds__(256) void k_spread(const uint32_t *keys, uint32_t N, uint32_t *out) {
+  __shared__ uint32_t sum;
+  if (threadIdx.x == 0) sum = 0;
+  __syncthreads();
+  const uint32_t *k = keys + (size_t)blockIdx.x * N;
+  auto key = [&](uint32_t i) { return k[(uint64_t)i * (N - 1u) / kSpreadSamples]; };
+  const uint32_t mid = key(kSpreadSamples / 2);
+  uint32_t mine = 0;
+  for (uint32_t i = threadIdx.x; i <= kSpreadSamples; i += blockDim.x) {
+    const uint32_t v = key(i);
+    mine += v == mid ? 1u << 16 : 0u;
+    mine += i < kSpreadSamples && v != key(i + 1u) ? 1u : 0u;
+  }
+  atomicAdd(&sum, mine);
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = sum;
+}
+
 // Exclusive scan of feature f's tile totals (one workgroup per feature);
 // D[f] = total + 1.
 __global__ __launch_bounds__(1024) void k_code_tscan(uint32_t *tsum, uint32_t ntiles, uint32_t *D) {

@@ -114,25 +114,6 @@ __global__ __launch_bounds__(kCodeThreads) void k_list_tables(const IdxT *rows, 
   }
 }
 
-// many[0] += the features (a workgroup each) with more than `most` values,
-// judged by the value changes between kManySamples evenly spaced positions of
-// the presorted row.
-constexpr uint32_t kManySamples = 2048;
-template <class IdxT>
-__global__ __launch_bounds__(256) void k_list_many(const IdxT *rows, const float *XT, uint32_t N, uint32_t most,
-                                                    uint32_t *many) {
-  __shared__ uint32_t changes;
-  if (threadIdx.x == 0) changes = 0;
-  __syncthreads();
-  const IdxT *row = rows + (size_t)blockIdx.x * N;
-  const float *x = XT + (size_t)blockIdx.x * N;
-  auto value = [&](uint32_t i) { return x[sample_of(row[(uint64_t)i * (N - 1u) / kManySamples])]; };
-  for (uint32_t i = threadIdx.x; i < kManySamples; i += blockDim.x)
-    if (value(i) != value(i + 1u)) atomicAdd(&changes, 1u);
-  __syncthreads();
-  if (threadIdx.x == 0 && changes >= most) atomicAdd(many, 1u);
-}
-
 // Row entries of all samples in ascending order (the list of a node that
 // holds every sample).
 template <class IdxT, class LabT>

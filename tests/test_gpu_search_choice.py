@@ -1,8 +1,10 @@
-"""The list search's cost on features that suit it badly (needs an MI355X), seen
-in the context's kernel statistics."""
+"""The fit's own choice between sorted rows and sample lists (needs an MI355X),
+seen in the context's kernel statistics: by the sizes, by how the features'
+values are spread, and that either search is the one that ran."""
 import numpy as np
 import pytest
 
+import helpers
 from cudatree_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -34,11 +36,41 @@ def profiled(ctx, ds, T, o, ids=None):
     return f, ctx.kernel_stats()
 
 
+def search_of(stats):
+    """Row scans take chunk histograms, list fits have none."""
+    return "rows" if "k_scan_hist" in stats else "lists"
+
+
 def dense(N, F, K, seed):
     rng = np.random.Generator(np.random.PCG64(seed))
     y = rng.integers(0, K, size=N)
     X = rng.standard_normal((N, F), dtype=np.float32) + (y[:, None] * 0.3).astype(np.float32)
     return X, y
+
+
+def with_counts(N, F, K, share, rare, seed):
+    """`share` of the features are zeros with small counts in `rare` of the
+    samples, more in some classes than in others; the rest are continuous."""
+    X, y = dense(N, F, K, seed)
+    rng = np.random.Generator(np.random.PCG64(seed + 1))
+    k = int(round(share * F))
+    lam = rare * (0.2 + 1.6 * rng.random((K, k)))
+    X[:, :k] = (rng.random((N, k)) < lam[y]) * rng.integers(1, 9, size=(N, k))
+    return X[:, rng.permutation(F)].copy(), y
+
+
+@pytest.mark.parametrize("share,rare,want", [(1.0, 0.003, "rows"),    # long chains of large nodes
+                                             (1.0, 0.2, "lists"),
+                                             (0.6, 0.0003, "rows"),   # constant in nearly every node
+                                             (0.6, 0.02, "lists"),
+                                             (0.0, 0.0, "lists")])
+def test_choice_by_rare_values(ctx, share, rare, want):
+    N, F, K, T, m = 20000, 300, 5, 40, 18
+    X, y = with_counts(N, F, K, share, rare, 7)
+    ds = _lib.Dataset(ctx, X, y, K)
+    print("choice by rare values", share, rare, flush=True)
+    _, st = profiled(ctx, ds, T, opts(m))
+    assert search_of(st) == want
 
 
 def test_constant_columns_are_not_read(ctx):

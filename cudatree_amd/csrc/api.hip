@@ -790,7 +790,10 @@ struct Fitter {
     // split-scan tasks are sized per level
     const uint64_t cap_scan = units_for((uint64_t)Tb);
     const uint64_t cap_big = (uint64_t)Fr * (n_tot / kBigN + Tb + 1);
-    const uint64_t cap_small = cap_q + 2ull * Fr * n_tot / Cr + 64;
+    // (the bootstrap compaction moves segments of N samples, however few are in-bag)
+    const uint64_t boot_rpt = std::max<uint64_t>(1, Cr / (uint32_t)N);
+    const uint64_t boot_tasks = boot ? (uint64_t)Tb * ((Fr + boot_rpt - 1) / boot_rpt) : 0;
+    const uint64_t cap_small = std::max<uint64_t>(cap_q + 2ull * Fr * n_tot / Cr, boot_tasks) + 64;
     const uint64_t cap_fill = cap_q + n_tot / Cf + 64;
     const uint64_t cap_hist = (uint64_t)m * K * ((list ? n_tot / kListWave : 2 * n_tot / Cs) + 64);
     // (node, feature) tasks of nodes of more than kListWave / kListWg[0] / kListWg[1] samples

@@ -1360,21 +1360,32 @@ __device__ __forceinline__ uint32_t child_kind(const FitArgs<IdxT, LabT> &a, uin
   return 0u;
 }
 
-// List search: label of the first of the list's samples in feature 0's
-// presorted order -- the lowest value, then the lowest id -- among those that
-// take(entry) keeps (0xFFFFFFFF: none of them).
-template <class IdxT, class LabT, class Take>
-__device__ __forceinline__ uint32_t first_label(const FitArgs<IdxT, LabT> &a, const IdxT *list, uint32_t n,
-                                                const Take &take) {
-  uint64_t best = ~0ull;  // value index, sample, label
-  for (uint32_t p = lane_id(); p < n; p += kWave) {
-    const IdxT e = list[p];
-    const uint32_t s = sample_of(e), w = a.rank[s];
-    if (take(e)) best = min(best, (uint64_t)(w >> kLabBits) << 32 | (uint64_t)s << kLabBits | (w & kLabMask));
-  }
+// List search: a sample's place in feature 0's presorted order -- its value, then
+// its id -- with its label in the low kLabBits.
+template <class IdxT, class LabT>
+__device__ __forceinline__ uint64_t first_word(const FitArgs<IdxT, LabT> &a, uint32_t s) {
+  const uint32_t w = a.rank[s];
+  return (uint64_t)(w >> kLabBits) << 32 | (uint64_t)s << kLabBits | (w & kLabMask);
+}
+__device__ __forceinline__ uint64_t wave_min64(uint64_t v) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) best = min(best, (uint64_t)__shfl_xor((unsigned long long)best, o, kWave));
-  return best == ~0ull ? 0xFFFFFFFFu : (uint32_t)best & kLabMask;
+  for (int o = 32; o > 0; o >>= 1) v = min(v, (uint64_t)__shfl_xor((unsigned long long)v, o, kWave));
+  return v;
+}
+
+// List search: label of the first of the list's samples in that order.
+template <class IdxT, class LabT>
+__device__ __forceinline__ uint32_t first_label(const FitArgs<IdxT, LabT> &a, const IdxT *list, uint32_t n) {
+  uint64_t best = ~0ull;
+  constexpr uint32_t U = 8;
+  for (uint32_t p = lane_id(); p < n; p += U * kWave) {
+    uint32_t s[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) s[u] = sample_of(list[min(p + u * kWave, n - 1u)]);  // (the last one again past the end)
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) best = min(best, first_word(a, s[u]));
+  }
+  return (uint32_t)wave_min64(best) & kLabMask;
 }
 
 // Class counts of the samples of node i whose value index of feature f is at
@@ -1446,7 +1457,7 @@ __global__ __launch_bounds__(kBlock) void k_decide(FitArgs<IdxT, LabT> a) {
       // segment in feature 0's row (random_tree.py:628-634, 50-63)
       const IdxT *row0 = rows_of(a, nd.src, nd.tree, 0) + nd.start;
       uint32_t lab = 0;
-      if constexpr (kList) lab = first_label(a, row0, nd.n, [](IdxT) { return true; });
+      if constexpr (kList) lab = first_label(a, row0, nd.n);
       if (lane == 0) {
         a.arena.feat[id] = -1;
         a.arena.thr[id] = 0.f;
@@ -1563,6 +1574,10 @@ __global__ __launch_bounds__(kBlock) void k_decide(FitArgs<IdxT, LabT> a) {
       // looks it up after the fill
       if (kl == 2) labl = kFirstSample;
       if (kr == 2) labr = kFirstSample;
+      if (kList && (kl == 2 || kr == 2)) {
+        ax.flags |= (kl == 2 ? kFirstL : 0u) | (kr == 2 ? kFirstR : 0u);
+        ax.rl_num = ax.rl_den = ~0ull;
+      }
       ax.lab[0] = kl ? labl : kLeaf;
       ax.lab[1] = kr ? labr : kLeaf;
       if (kl == 0) ax.flags |= kLiveL;
@@ -1728,6 +1743,7 @@ __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, con
     const uint32_t *col = reinterpret_cast<const uint32_t *>(a.codes + fc_off(a.fcode[ax.best_f]));
     IndexCol ic = {nullptr, 0u};
     if (kList && !bycol) ic = index_col(a, (uint32_t)ax.best_f);
+    uint64_t firstl = ~0ull, firstr = ~0ull;
     for (uint32_t pb = p0; pb < p1; pb += kFillU * kWave) {
       uint32_t e[kFillU], low[kFillU];
 #pragma unroll
@@ -1751,6 +1767,26 @@ __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, con
         if (take[u]) atomicOr(&bits[s >> 5], 1u << (s & 31u));
       }
       if (count) rl_add(a, e, take, cnt);
+      if (kList && (ax.flags & (kFirstL | kFirstR))) {
+        // (a wave that read such a node through by itself: 300,000 x 64, 40 trees
+        // of leaves below 150,000 samples, k_children 9.0 ms, now 0.04)
+#pragma unroll
+        for (int u = 0; u < kFillU; ++u) {
+          if (e[u] == 0xFFFFFFFFu) continue;
+          const uint64_t w = first_word(a, sample_of((IdxT)e[u]));
+          if (low[u]) firstl = min(firstl, w);
+          else firstr = min(firstr, w);
+        }
+      }
+    }
+    if (kList && (ax.flags & (kFirstL | kFirstR))) {
+      firstl = wave_min64(firstl);
+      firstr = wave_min64(firstr);
+      if (lane == 0) {
+        NAux *to = a.aux + tk.node;
+        if (ax.flags & kFirstL) atomicMin(reinterpret_cast<unsigned long long *>(&to->rl_num), (unsigned long long)firstl);
+        if (ax.flags & kFirstR) atomicMin(reinterpret_cast<unsigned long long *>(&to->rl_den), (unsigned long long)firstr);
+      }
     }
   } else {
     // split feature's row: positions below nL go left, so the smaller side
@@ -1908,13 +1944,9 @@ __global__ __launch_bounds__(kBlock) void k_children_emit(FitArgs<IdxT, LabT> a)
       const uint32_t *bits = a.bits + (size_t)nd.tree * a.W;
       const uint32_t inv = (ax.flags & kInvert) ? 1u : 0u;  // the marks are on the right
       bool needl = lab[0] == kFirstSample, needr = lab[1] == kFirstSample;
-      if (a.rank) {  // (list search)
-        auto side = [&](IdxT e, uint32_t want) {
-          const uint32_t s = sample_of(e);
-          return (((bits[s >> 5] >> (s & 31u)) & 1u) ^ inv) == want;
-        };
-        if (needl) lab[0] = first_label(a, row0, nd.n, [&](IdxT e) { return side(e, 1u); });
-        if (needr) lab[1] = first_label(a, row0, nd.n, [&](IdxT e) { return side(e, 0u); });
+      if (a.rank) {  // list search: found by the fill
+        if (needl) lab[0] = (uint32_t)ax.rl_num & kLabMask;
+        if (needr) lab[1] = (uint32_t)ax.rl_den & kLabMask;
         needl = needr = false;
       }
       for (uint32_t pb = 0; pb < nd.n && (needl || needr); pb += kWave) {

@@ -49,6 +49,10 @@ constexpr uint32_t kCountRl = 8u;
 // Set by k_decide on a split node whose right child is the smaller: the side
 // bitmaps mark a split node's smaller child, so its marks are the right one's.
 constexpr uint32_t kInvert = 16u;
+// List search: the left / right child is a leaf labelled by its first sample in
+// feature 0's presorted order.  The fill tasks leave that sample's order word (see
+// first_word) in rl_num / rl_den, which k_decide set to ~0.
+constexpr uint32_t kFirstL = 32u, kFirstR = 64u;
 
 // A unit of wave work: node, first row/feature slot and count (low/high
 // 16 bits), chunk index and the node's chunk count.

@@ -2685,6 +2685,38 @@ __global__ __launch_bounds__(kBlock) void k_boot_tasks(FitArgs<IdxT, LabT> a, co
   flush_bytes(a, kBytesBoot, bytes);
 }
 
+// List search: label of the first of tree t's n in-bag samples in feature 0's
+// presorted order, by a whole workgroup of kPlanThreads.  The row of all N
+// samples is read from its start as long as that is likely to be the shorter
+// way (src 0: every sample is in-bag; the bitmaps still hold the in-bag marks),
+// then the tree's list.  (By one thread along the row: 20 trees of the last 50 of
+// 500,000 samples, a fit's setup 85 ms, this way 0.8; over sorted rows 0.3.)
+template <class IdxT, class LabT>
+__device__ uint32_t root_first_label(const FitArgs<IdxT, LabT> &a, uint32_t src, uint32_t t, uint32_t n) {
+  constexpr uint32_t kW = kPlanThreads / kWave, kTiles = 16;
+  __shared__ uint64_t low[kW];
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave, N = (uint32_t)a.N;
+  const uint32_t *bits = a.bits + (size_t)t * a.W;
+  auto lowest = [&](uint64_t v) {  // of the waves' values
+    __syncthreads();
+    if (lane == 0) low[wave] = v;
+    __syncthreads();
+    uint64_t m = low[0];
+    for (uint32_t w = 1; w < kW; ++w) m = min(m, low[w]);
+    return m;
+  };
+  for (uint32_t c = 0; c < kTiles && c * kPlanThreads < N; ++c) {
+    const uint32_t p = c * kPlanThreads + tid, s = sample_of(a.presorted[min(p, N - 1u)]);
+    const uint64_t mk = ballot(p < N && (src == 0 || ((bits[s >> 5] >> (s & 31u)) & 1u)));
+    const uint64_t at = lowest(mk ? p - lane + (uint64_t)__ffsll((unsigned long long)mk) - 1u : ~0ull);
+    if (at != ~0ull) return a.label(a.presorted[at]);
+  }
+  const IdxT *list = rows_of(a, src, t, 0);
+  uint64_t best = ~0ull;
+  for (uint32_t p = tid; p < n; p += kPlanThreads) best = min(best, first_word(a, sample_of(list[p])));
+  return (uint32_t)lowest(wave_min64(best)) & kLabMask;
+}
+
 // Roots: tree t's root (arena id t) is a leaf if pure, else enters the
 // frontier; one workgroup, so the frontier is in tree order.
 template <class IdxT, class LabT>
@@ -2693,6 +2725,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_roots(FitArgs<IdxT, LabT> a, c
   constexpr int kW = kPlanThreads / kWave;
   __shared__ uint32_t ws[kW];
   __shared__ uint32_t carry;
+  __shared__ uint32_t first[kPlanThreads];  // list search: in-bag samples of a tree that is a first-sample leaf, else 0
   const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const uint32_t K = (uint32_t)a.K;
   if (tid == 0) carry = 0;
@@ -2700,6 +2733,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_roots(FitArgs<IdxT, LabT> a, c
   for (uint32_t t0 = 0; t0 < T; t0 += kPlanThreads) {
     const uint32_t t = t0 + tid;
     uint32_t live = 0, n = 0;
+    bool find = false;
     if (t < T) {
       n = off ? (uint32_t)(off[t + 1] - off[t]) : (uint32_t)a.N;
       uint32_t nz = 0, only = 0;
@@ -2716,20 +2750,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_roots(FitArgs<IdxT, LabT> a, c
       uint32_t leaf_label = kLeaf;
       if (nz <= 1) leaf_label = only;
       else if ((int64_t)n < (int64_t)a.mss) {
-        if (a.rank) {
-          // list search: the first in-bag sample of the presorted row (src 0:
-          // every sample is; the bitmaps still hold the in-bag marks)
-          const uint32_t *bits = a.bits + (size_t)t * a.W;
-          uint32_t p = 0;
-          while (src != 0 && p + 1 < (uint32_t)a.N) {
-            const uint32_t s = sample_of(a.presorted[p]);
-            if ((bits[s >> 5] >> (s & 31u)) & 1u) break;
-            ++p;
-          }
-          leaf_label = a.label(a.presorted[p]);
-        } else {
-          leaf_label = a.label(rows_of(a, src, t, 0)[0]);
-        }
+        find = a.rank != nullptr;
+        leaf_label = find ? 0u : a.label(rows_of(a, src, t, 0)[0]);
       }
       if (leaf_label != kLeaf) {
         a.arena.feat[t] = -1;
@@ -2739,6 +2761,15 @@ __global__ __launch_bounds__(kPlanThreads) void k_roots(FitArgs<IdxT, LabT> a, c
         a.arena.value[t] = leaf_label;
       } else {
         live = 1;
+      }
+    }
+    if (__syncthreads_or(find)) {
+      first[tid] = find ? n : 0u;
+      __syncthreads();
+      for (uint32_t k = 0; k < (uint32_t)kPlanThreads && t0 + k < T; ++k) {
+        if (!first[k]) continue;
+        const uint32_t label = root_first_label(a, src, t0 + k, first[k]);
+        if (tid == 0) a.arena.value[t0 + k] = label;
       }
     }
     const uint32_t inc = wave_incl_scan(live);

@@ -541,8 +541,29 @@ Spread spread_of(const uint32_t *sampled, const int32_t *rl_of, const cta_datase
   return sp;
 }
 
-// The sizes from which lists are the faster search, in a fit of T trees on N
-// samples and Fr features with rows, m of them evaluated at a node.
+constexpr double kInBag = 0.632;  // in-bag share of a bootstrapped tree
+
+// What a fit's options say of its size, as the choice of search takes it.
+struct FitSize {
+  int64_t N, F, m, T;
+  double levels;  // of nodes that split, by the depth limit, the leaf size and the in-bag samples (a share of one
+                  // for in-bag sets smaller than a bootstrap's)
+  double moves;   // times that sorted rows of N samples are moved: the bootstrap's, then a level's in-bag share
+};
+// (inbag: mean in-bag samples of a tree; unbalanced trees have about half as
+// many levels again as balanced ones)
+FitSize fit_size(int64_t N, int64_t F, int64_t T, int64_t m, const cta_fit_opts &o, bool bagged, double inbag) {
+  FitSize z = {N, F, m, T, 0.0, 0.0};
+  const double leaf = std::max(1.0, (double)o.min_samples_split);
+  if (inbag >= leaf) z.levels = 1.0 + std::floor(1.5 * std::log2(inbag / leaf));
+  if (o.max_depth > 0) z.levels = std::min(z.levels, (double)o.max_depth);
+  z.moves = (bagged ? 1.0 : 0.0) + std::max(0.0, z.levels - 1.0) * inbag / (double)N;
+  z.levels *= std::min(1.0, inbag / (kInBag * (double)N));
+  return z;
+}
+
+// The sizes from which lists are the faster search, in a fit with Fr features
+// that have rows, m of them evaluated at a node.
 // Rows move Fr rows of every tree per level where lists sort max_features of
 // them, but a node's feature takes one workgroup where rows split it into
 // chunks, and the tables cost about a presort: lists need enough trees.
@@ -565,18 +586,31 @@ Spread spread_of(const uint32_t *sampled, const int32_t *rl_of, const cta_datase
 // constant tests: 20,000 x 1,000, 20 trees, 60% of the features of a rare share
 // of 0.0003 / 0.001 / 0.01: 13.1 / 16.0, 13.1 / 11.3, 13.9 / 8.4; small sets,
 // where the tests weigh more, 3,000 x 300, 20 trees, 30% of 0.003: 2.7 / 3.1.
-bool list_worth(int64_t N, double Fr, int64_t m, int64_t T, const Spread &sp) {
-  if ((double)m * sp.rare < 0.5) return false;
-  if (N <= (int64_t)kListWg[0]) return Fr * (1.0 - 5.0 * sp.drag) >= 10.0 * (double)m;
-  if ((Fr - 8.0 * (double)m) * (double)T >= 4000.0 && (Fr * (1.0 - sp.drag) - 8.0 * (double)m) * (double)T >= 2700.0)
+// A fit of few moves -- shallow trees, large leaves, small in-bag sets, few trees
+// of many features -- spares little against the tables and the large nodes of
+// its first levels.  Rows / lists, ms, by depth limit: 20,000 x 2,000, 50 trees
+// without bootstrap, 1 / 2 / 3: 1.1 / 3.5, 4.2 / 4.5, 7.0 / 5.5; 200,000 x 256, 100
+// trees, 1 / 2: 4.6 / 8.1, 17.3 / 13.1; 300,000 x 128, 200 trees, 6, bootstrap:
+// 92 / 58; 20,000 x 2,000, 8 trees, 7: 3.7 / 4.2; without a limit 20,000 x 4,096,
+// 3 / 6 trees: 5.7 / 6.2, 8.5 / 7.4; 3,000 x 400, 100 trees, 3 / 5: 0.87 / 0.99,
+// 1.25 / 1.14; few values, 600,000 x 49, 46 trees, 1 without / with bootstrap:
+// 1.6 / 1.8, 3.3 / 1.9.  Fitted to 440 such fits: of those that take lists 19 in
+// 20 are faster, the others lose 11% at most.
+bool list_worth(const FitSize &z, double Fr, const Spread &sp) {
+  const double m = (double)z.m, T = (double)z.T, N = (double)z.N;
+  if (m * sp.rare < 0.5) return false;
+  if (z.N <= (int64_t)kListWg[0]) return z.moves >= 4.5 && Fr * (1.0 - 5.0 * sp.drag) >= 10.0 * m;
+  const double Fd = Fr * (1.0 - sp.drag);
+  if ((Fr - 8.0 * m) * T >= 4000.0 && (Fd - 8.0 * m) * T >= 2700.0 &&
+      T * (std::min(z.moves, 16.0) * Fd - 7.0 * std::min(z.levels, 5.0) * m) >= 56.0 * (double)z.F)
     return true;
   const double Fc = Fr * (1.0 - 2.0 * sp.drag);  // (20,000 x 1,000, 95% two-valued of 0.003, 20 trees: 23 / 27)
-  return sp.few && Fc >= 6.0 * (double)m && Fc * (double)T * (double)N >= 0x1p27;
+  return sp.few && Fc >= 6.0 * m && Fc * T * N >= 0x1p27 && (10.0 * z.moves + 3.0) * T >= 360.0;
 }
 
 // Whether a fit of T trees searches its splits from sample lists instead of
-// sorted rows.
-bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T) {
+// sorted rows (off: the caller's in-bag sets).
+bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T, const int64_t *off) {
   if (!list_possible(ds->N, ds->K, o, ctx->lds_per_block)) return false;
   if (o.search == CTA_SEARCH_LISTS) return true;
   // (a workspace limit that holds the rows may not hold the tables' scratch,
@@ -591,7 +625,9 @@ bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T
   // A two-valued feature counts half: a rare value's list is read through in
   // the constant test, where its row shows both ends (of 201 features 140
   // such, 2,500 samples, 5 trees: 3.6 / 4.3; 990 of 1,000, 3,000: 12.5 / 10.0).
-  return list_worth(ds->N, (double)(ds->Fr - ds->two / 2), o.max_features, T, ds->spread);
+  const double inbag = off ? (double)(off[T] - off[0]) / T : o.bootstrap ? kInBag * ds->N : (double)ds->N;
+  return list_worth(fit_size(ds->N, ds->F, T, o.max_features, o, off || o.bootstrap, inbag),
+                    (double)(ds->Fr - ds->two / 2), ds->spread);
 }
 
 // The list search's tables of a training set (kept with it; built on the
@@ -1697,7 +1733,7 @@ void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, con
     if (ctx->lane) ctx->lane->ws_release();
     out->clear();
   };
-  if (list_search(ctx, ds, o, T)) {
+  if (list_search(ctx, ds, o, T, ids ? off : nullptr)) {
     try {
       list_tables<IdxT, LabT>(ctx, ds);
       if (o.lanes == 2) ctx->sync();  // (the other lane's stream reads them too)
@@ -2526,7 +2562,7 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
     // and the list search's words and distinct values, where the fit may choose
     // it for data that suit it best (every feature with a row, dense, of few values)
     if (list_possible(N, K, *opts, kMaxLds) &&
-        (opts->search == CTA_SEARCH_LISTS || list_worth(N, F, m, T, Spread{})))
+        (opts->search == CTA_SEARCH_LISTS || list_worth(fit_size(N, F, T, m, *opts, true, N), F, Spread{})))
       *dataset_bytes += nf * 8 + n * b + 20 * f;
     // the context's workspaces: radix-sort and code-column temporaries of the
     // build, then per resident tree (every feature keeping rows), the node

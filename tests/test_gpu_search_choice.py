@@ -90,3 +90,33 @@ def test_constant_columns_are_not_read(ctx):
         ms.append(profiled(ctx, ds, T, o)[1]["k_select"]["ms"])
     print(ms)
     assert ms[1] < 3.0 * ms[0], ms
+
+
+@pytest.mark.parametrize("N,F,T,kw,want", [
+    (20000, 1000, 50, {"max_depth": 1}, "rows"), (20000, 1000, 50, {"max_depth": 2, "bootstrap": 0}, "rows"),
+    (20000, 1000, 50, {"max_depth": 8}, "lists"), (20000, 1000, 50, {"min_samples_split": 9000}, "rows"),
+    (20000, 1000, 50, {"min_samples_split": 200}, "lists"),
+    (3000, 400, 20, {"max_depth": 3}, "rows"), (3000, 400, 20, {"max_depth": 8}, "lists"),
+    (3000, 190, 20, {}, "lists"), (3000, 179, 20, {}, "rows")])  # (both sides of 10 m)
+def test_choice_by_depth(ctx, N, F, T, kw, want):
+    """Trees of few levels spare too little for the list search's tables."""
+    X, y = dense(N, F, 5, 9)
+    m = 18 if F < 400 else int(np.ceil(F ** 0.5))
+    ds = _lib.Dataset(ctx, X, y, 5)
+    print("choice by depth", N, F, T, kw, flush=True)
+    f, st = profiled(ctx, ds, T, opts(m, **kw))
+    assert search_of(st) == want
+    g, st = profiled(ctx, ds, T, opts(m, search=_lib.CTA_SEARCH_ROWS if want == "lists" else _lib.CTA_SEARCH_LISTS, **kw))
+    assert search_of(st) != want and helpers.forest_diff(f, g) is None
+
+
+def test_choice_by_in_bag_sets(ctx):
+    """Few samples in-bag: rows of them are cheap to move after the compaction."""
+    N, F, T, m = 100000, 100, 50, 2
+    X, y = dense(N, F, 5, 10)
+    rng = np.random.Generator(np.random.PCG64(11))
+    ids = [np.sort(rng.choice(N, 50, replace=False)).astype(np.uint32) for _ in range(T)]
+    ds = _lib.Dataset(ctx, X, y, 5)
+    print("choice by in-bag sets", flush=True)
+    assert search_of(profiled(ctx, ds, T, opts(m), ids)[1]) == "rows"
+    assert search_of(profiled(ctx, ds, T, opts(m))[1]) == "lists"

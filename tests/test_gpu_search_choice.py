@@ -59,6 +59,19 @@ def with_counts(N, F, K, share, rare, seed):
     return X[:, rng.permutation(F)].copy(), y
 
 
+def test_statistics_name_the_search(ctx):
+    """The scans of either search have entries of their own, and only the row
+    scan's, whose bytes are counted, gives a rate."""
+    N, F, K, T, m = 6000, 40, 5, 4, 7
+    X, y = dense(N, F, K, 6)
+    ds = _lib.Dataset(ctx, X, y, K)
+    print("statistics", flush=True)
+    _, rows = profiled(ctx, ds, T, opts(m, search=_lib.CTA_SEARCH_ROWS))
+    _, lists = profiled(ctx, ds, T, opts(m, search=_lib.CTA_SEARCH_LISTS))
+    assert rows["k_scan"]["alg_bytes"] > 0 and "k_list_scan" not in rows
+    assert lists["k_list_scan"]["ms"] > 0 and lists["k_list_scan"]["alg_bytes"] == 0 and "k_scan" not in lists
+
+
 @pytest.mark.parametrize("share,rare,want", [(1.0, 0.003, "rows"),    # long chains of large nodes
                                              (1.0, 0.2, "lists"),
                                              (0.6, 0.0003, "rows"),   # constant in nearly every node

@@ -419,6 +419,7 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
       bool nonconst = false;
       uint32_t f = 0;
       int32_t jr = -1;
+      bool bits = false;
       Cand cd = {0, 1, 0, -1, 0};  // a row-free feature's one candidate
       if (k < F) {
         f = perm_at(pm, k);
@@ -426,6 +427,7 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
         jr = a.Frl ? a.rl_of[f] : -1;
         const int32_t slot = a.slot_of[f];
         const uint64_t fc = a.fcode[f];
+        bits = fc_kind(fc) == 1u;
         if (jr >= 0) {
           // row-free: constant when no or every sample holds the higher
           // value; its one candidate sends the samples holding the lower
@@ -473,7 +475,8 @@ __global__ __launch_bounds__(kBlock) void k_select(FitArgs<IdxT, LabT> a) {
       }
       if constexpr (kList) {
         // (a feature of one value over the whole set is not read at all)
-        const bool want = k < F && jr < 0 && a.ndist[f] > 1u;
+        // (its column is of the two-valued kind)
+        const bool want = k < F && jr < 0 && (!bits || a.ndist[f] > 1u);
         nonconst |= list_varies(list, n, index_col(a, want ? f : 0u), want, ballot(nonconst), m - nsel);
       }
       const uint64_t mk = ballot(nonconst);
@@ -1743,7 +1746,6 @@ __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, con
     const uint32_t *col = reinterpret_cast<const uint32_t *>(a.codes + fc_off(a.fcode[ax.best_f]));
     IndexCol ic = {nullptr, 0u};
     if (kList && !bycol) ic = index_col(a, (uint32_t)ax.best_f);
-    uint64_t firstl = ~0ull, firstr = ~0ull;
     for (uint32_t pb = p0; pb < p1; pb += kFillU * kWave) {
       uint32_t e[kFillU], low[kFillU];
 #pragma unroll
@@ -1767,19 +1769,17 @@ __device__ __forceinline__ void fill_task_bits(const FitArgs<IdxT, LabT> &a, con
         if (take[u]) atomicOr(&bits[s >> 5], 1u << (s & 31u));
       }
       if (count) rl_add(a, e, take, cnt);
-      if (kList && (ax.flags & (kFirstL | kFirstR))) {
-        // (a wave that read such a node through by itself: 300,000 x 64, 40 trees
-        // of leaves below 150,000 samples, k_children 9.0 ms, now 0.04)
-#pragma unroll
-        for (int u = 0; u < kFillU; ++u) {
-          if (e[u] == 0xFFFFFFFFu) continue;
-          const uint64_t w = first_word(a, sample_of((IdxT)e[u]));
-          if (low[u]) firstl = min(firstl, w);
-          else firstr = min(firstr, w);
-        }
-      }
     }
     if (kList && (ax.flags & (kFirstL | kFirstR))) {
+      // (a wave that read such a node through by itself: 300,000 x 64, 40 trees
+      // of leaves below 150,000 samples, k_children 9.0 ms, now 0.04)
+      uint64_t firstl = ~0ull, firstr = ~0ull;
+      for (uint32_t p = p0 + lane; p < p1; p += kWave) {
+        const uint32_t s = sample_of(row[p]);
+        const uint64_t w = first_word(a, s);
+        if (bycol ? !((col[s >> 5] >> (s & 31u)) & 1u) : ic.at(s) <= ax.lo) firstl = min(firstl, w);
+        else firstr = min(firstr, w);
+      }
       firstl = wave_min64(firstl);
       firstr = wave_min64(firstr);
       if (lane == 0) {
@@ -1945,8 +1945,8 @@ __global__ __launch_bounds__(kBlock) void k_children_emit(FitArgs<IdxT, LabT> a)
       const uint32_t inv = (ax.flags & kInvert) ? 1u : 0u;  // the marks are on the right
       bool needl = lab[0] == kFirstSample, needr = lab[1] == kFirstSample;
       if (a.rank) {  // list search: found by the fill
-        if (needl) lab[0] = (uint32_t)ax.rl_num & kLabMask;
-        if (needr) lab[1] = (uint32_t)ax.rl_den & kLabMask;
+        if (needl) lab[0] = (uint32_t)a.aux[i].rl_num & kLabMask;
+        if (needr) lab[1] = (uint32_t)a.aux[i].rl_den & kLabMask;
         needl = needr = false;
       }
       for (uint32_t pb = 0; pb < nd.n && (needl || needr); pb += kWave) {

@@ -525,10 +525,10 @@ Spread spread_of(const uint32_t *sampled, const int32_t *rl_of, const cta_datase
   double rare = 0, drag = 0;
   uint64_t vary = 0, many = 0;
   for (uint32_t f = 0; f < F; ++f) {
-    const uint32_t changes = sampled[f] & 0xFFFFu;
+    const uint32_t changes = sampled[f] >> 1 & ((1u << kSpreadBits) - 1u), mid = sampled[f] >> (1 + kSpreadBits);
     if (!changes) continue;
     // (one of the two ends is always another value)
-    const double r = std::max(0.0, kSpreadSamples - (double)(sampled[f] >> 16)) / kSpreadSamples;
+    const double r = std::max(0.0, kSpreadSamples - (double)mid) / kSpreadSamples;
     ++vary;
     rare += r;
     many += changes >= most;
@@ -1846,15 +1846,14 @@ void build_codes(cta_ctx *ctx, cta_dataset *ds, const uint32_t *keys, const uint
   k_code_flags<<<dim3(ntiles, F), kCodeThreads, 0, st>>>(keys, N, ntiles, pre, tsum, db + F);
   k_code_tscan<<<F, 1024, 0, st>>>(tsum, ntiles, db);
   k_code_scatter<<<dim3(ntiles, F), kCodeThreads, 0, st>>>(ids, pre, tsum, N, ntiles, d);
-  k_spread<<<F, 256, 0, st>>>(keys, N, tsum);  // (the tile totals are no longer needed)
-  uint32_t *h = static_cast<uint32_t *>(ctx->host("code_meta", 3 * (size_t)F * 4));
+  k_spread<<<F, 1024, 0, st>>>(keys, N, db + F);
+  uint32_t *h = static_cast<uint32_t *>(ctx->host("code_meta", 2 * (size_t)F * 4));
   HIPC(hipMemcpyAsync(h, db, 2 * (size_t)F * 4, hipMemcpyDeviceToHost, st));
-  HIPC(hipMemcpyAsync(h + 2 * (size_t)F, tsum, (size_t)F * 4, hipMemcpyDeviceToHost, st));
   ctx->sync();
   std::vector<uint64_t> fc(F);
   uint64_t off = 0;
   for (uint32_t f = 0; f < F; ++f) {
-    const uint32_t D = h[f], bad = h[F + f];
+    const uint32_t D = h[f], bad = h[F + f] & 1u;
     uint32_t kind = 0;
     uint64_t bytes = 0;
     if (!bad && D <= 2) {
@@ -1898,7 +1897,7 @@ void build_codes(cta_ctx *ctx, cta_dataset *ds, const uint32_t *keys, const uint
   ds->Frl = (int32_t)rl_feat.size();
   ds->Wsig = (ds->Frl + 31) / 32;
   ds->Fr = (int32_t)row_feat.size();
-  ds->spread = spread_of(h + 2 * (size_t)F, rl_of, ds, ctx->lds_per_block);
+  ds->spread = spread_of(h + F, rl_of, ds, ctx->lds_per_block);
   int32_t *ht = static_cast<int32_t *>(ctx->host("rl_tables", ((size_t)6 * F + 2) * 4));
   std::memcpy(ht, tab.data(), (size_t)4 * F * 4);
   std::memcpy(ht + 4 * F, row_feat.data(), row_feat.size() * 4);

@@ -456,11 +456,11 @@ __global__ __launch_bounds__(kCodeThreads) void k_code_flags(const uint32_t *key
 }
 
 // How a feature's values are spread (a workgroup each), from kSpreadSamples + 1
-// evenly spaced positions of its sorted keys, both ends among them: out[f] = the
-// value changes between neighbours (none: the feature has one value), and in
-// the high half how many positions hold the middle one's value.
-constexpr uint32_t kSpreadSamples = 2048;
-__global__ __launch_bounds__(256) void k_spread(const uint32_t *keys, uint32_t N, uint32_t *out) {
+// evenly spaced positions of its sorted keys, both ends among them: the value
+// changes between neighbours (none: the feature has one value) and how many
+// positions hold the middle one's value, beside the flag in bad[f].
+constexpr uint32_t kSpreadSamples = 2048, kSpreadBits = 12;
+__global__ __launch_bounds__(1024) void k_spread(const uint32_t *keys, uint32_t N, uint32_t *bad) {
   __shared__ uint32_t sum;
   if (threadIdx.x == 0) sum = 0;
   __syncthreads();
@@ -468,14 +468,15 @@ __global__ __launch_bounds__(256) void k_spread(const uint32_t *keys, uint32_t N
   auto key = [&](uint32_t i) { return k[(uint64_t)i * (N - 1u) / kSpreadSamples]; };
   const uint32_t mid = key(kSpreadSamples / 2);
   uint32_t mine = 0;
-  for (uint32_t i = threadIdx.x; i <= kSpreadSamples; i += blockDim.x) {
+#pragma unroll
+  for (uint32_t i = threadIdx.x; i < kSpreadSamples; i += 1024) {
     const uint32_t v = key(i);
-    mine += v == mid ? 1u << 16 : 0u;
-    mine += i < kSpreadSamples && v != key(i + 1u) ? 1u : 0u;
+    mine += (v == mid ? 1u << kSpreadBits : 0u) + (v != key(i + 1u) ? 1u : 0u);
   }
-  atomicAdd(&sum, mine);
+  mine = wave_sum32(mine);
+  if (lane_id() == 0 && mine) atomicAdd(&sum, mine);
   __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.x] = sum;
+  if (threadIdx.x == 0) atomicOr(&bad[blockIdx.x], (sum + (key(kSpreadSamples) == mid ? 1u << kSpreadBits : 0u)) << 1);
 }
 
 // Exclusive scan of feature f's tile totals (one workgroup per feature);

@@ -221,10 +221,14 @@ __device__ __forceinline__ void lane_masks(uint32_t (&M)[6]) {
 }
 
 // ---- scores --------------------------------------------------------------------
-// The score of a split is num / den (see q_cmp).  A node of n samples has
-// num <= n^3 and den <= n^2 / 4, so smaller nodes take narrower products;
-// the comparisons stay exact.
-struct Small {  // n <= 1,024: num < 2^31, den < 2^19, products in 64 bits
+// The score of a split is num / den, num = S_L nR + S_R nL and den = nL nR (see
+// q_cmp).  S_L <= nL^2 and S_R <= nR^2, so in a node of n samples
+// num <= nL nR n <= n^3 / 4 and den <= n^2 / 4: smaller nodes take narrower
+// products, and the comparisons stay exact.
+constexpr unsigned __int128 most_num(unsigned __int128 n) { return n * n * n / 4; }
+static_assert(most_num(CTA_MAX_SAMPLES) >> 64 == 0, "a score's numerator in 64 bits");
+static_assert(most_num(kListWave) >> 32 == 0, "and of one wave's nodes in 32");
+struct Small {  // n <= 1,024: num <= 2^28, den <= 2^18, products in 64 bits
   using Num = uint32_t;
   using Den = uint32_t;
   using Sum = uint32_t;
@@ -233,7 +237,7 @@ struct Small {  // n <= 1,024: num < 2^31, den < 2^19, products in 64 bits
     return a > b ? 1 : a < b ? -1 : 0;
   }
 };
-struct Mid {  // n <= 32,768: num < 2^46, den <= 2^28, products in 96 bits
+struct Mid {  // n <= 32,768: num <= 2^43, den <= 2^28, products in 96 bits
   using Num = uint64_t;
   using Den = uint32_t;
   using Sum = uint32_t;
@@ -844,7 +848,7 @@ __device__ __forceinline__ void wg_scan(const FitArgs<IdxT, LabT> &a, uint32_t n
 // or not, the scan about 250 per 64 kept, so it pays while a node holds more
 // than a small share of the samples: 200,000 x 256, 200 trees, nodes above
 // 32,768 samples (30% of the evaluated elements) 38 ms where moving their
-// rows took 60 and scanning them 30.
+// rows took 60 and scanning them 30, and 29 since tasks run in feature order.
 template <int W, bool kRegs, class IdxT, class LabT>
 __device__ __forceinline__ void wg_filter(const FitArgs<IdxT, LabT> &a, const IdxT *list, uint32_t n, uint32_t f,
                                           uint32_t *set, uint32_t *cnt, const uint32_t *tot, uint32_t *tail,

@@ -2562,8 +2562,10 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
                      nf * 4 + n * 4;
     // and the list search's words and distinct values, where the fit may choose
     // it for data that suit it best (every feature with a row, dense, of few values)
-    if (list_possible(N, K, *opts, kMaxLds) &&
-        (opts->search == CTA_SEARCH_LISTS || list_worth(fit_size(N, F, T, m, *opts, true, N), F, Spread{})))
+    // and in-bag sets that leave its scans nothing to do
+    FitSize most = fit_size(N, F, T, m, *opts, true, N);
+    most.levels = 0.0;
+    if (list_possible(N, K, *opts, kMaxLds) && (opts->search == CTA_SEARCH_LISTS || list_worth(most, F, Spread{})))
       *dataset_bytes += nf * 8 + n * b + 20 * f;
     // the context's workspaces: radix-sort and code-column temporaries of the
     // build, then per resident tree (every feature keeping rows), the node

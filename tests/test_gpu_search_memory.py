@@ -174,3 +174,24 @@ def test_limited_context_builds_tables_in_the_scratch_it_holds():
     assert limited(ctx) <= 20 << 20  # the scratch was given back
     ds.close()
     ctx.close()
+
+
+def test_limited_context_without_room_for_list_tasks():
+    """A limit at what a row fit holds: the list search's own workspaces do not
+    fit it, and the rows do, as they did."""
+    N, F, K, T, m = 3000, 2000, 5, 3, 45
+    X, y = gauss(N, F, K, 6)
+    ctx = _lib.Context(0)
+    ds = _lib.Dataset(ctx, X, y, K)
+
+    def fit(**kw):
+        return _lib.Forest.fit(ctx, ds, T, opts(m, **kw), None).export()
+
+    want = fit(search=_lib.CTA_SEARCH_ROWS)
+    print("limit at what rows hold", flush=True)
+    held = limited(ctx, 0)
+    got, rows, _ = searches(ctx, fit)
+    assert rows and helpers.forest_diff(got, want) is None
+    assert limited(ctx) <= held
+    ds.close()
+    ctx.close()

@@ -545,15 +545,17 @@ constexpr double kInBag = 0.632;  // in-bag share of a bootstrapped tree
 
 // What a fit's options say of its size, as the choice of search takes it.
 struct FitSize {
-  int64_t N, F, m, T;
+  int64_t N, F, K, m, T;
+  int64_t R;      // trees grown at a time
   double levels;  // of nodes that split, by the depth limit, the leaf size and the in-bag samples (a share of one
                   // for in-bag sets smaller than a bootstrap's)
   double moves;   // times that sorted rows of N samples are moved: the bootstrap's, then a level's in-bag share
 };
 // (inbag: mean in-bag samples of a tree; unbalanced trees have about half as
 // many levels again as balanced ones)
-FitSize fit_size(int64_t N, int64_t F, int64_t T, int64_t m, const cta_fit_opts &o, bool bagged, double inbag) {
-  FitSize z = {N, F, m, T, 0.0, 0.0};
+FitSize fit_size(int64_t N, int64_t F, int64_t K, int64_t T, int64_t m, const cta_fit_opts &o, bool bagged,
+                 double inbag) {
+  FitSize z = {N, F, K, m, T, o.trees_per_batch > 0 ? std::min<int64_t>(o.trees_per_batch, T) : T, 0.0, 0.0};
   const double leaf = std::max(1.0, (double)o.min_samples_split);
   if (inbag >= leaf) z.levels = 1.0 + std::floor(1.5 * std::log2(inbag / leaf));
   if (o.max_depth > 0) z.levels = std::min(z.levels, (double)o.max_depth);
@@ -596,16 +598,47 @@ FitSize fit_size(int64_t N, int64_t F, int64_t T, int64_t m, const cta_fit_opts 
 // 1.25 / 1.14; few values, 600,000 x 49, 46 trees, 1 without / with bootstrap:
 // 1.6 / 1.8, 3.3 / 1.9.  Fitted to 440 such fits: of those that take lists 19 in
 // 20 are faster, the others lose 11% at most.
+// Nodes above 32,768 samples take a workgroup a feature for long, so enough of
+// what lists spare has to be in flight: trees grown at a time x (features - 8
+// max_features) x classes, which cost rows more (few-valued features: trees x
+// features x samples).  Lists over rows in time, by samples x features, classes,
+// trees at a time: 200,000 x 256, 2, 1 / 4 / 6 / 8: 2.25 / 1.32 / 1.03 / 0.87; 10
+// classes, 1 / 2 / 4: 1.36 / 1.18 / 1.00; 100 classes, 1: 0.94; 60,000 x 256, 10,
+// 1 / 4: 1.05 / 0.95; 60,000 x 100, 10, 12: 1.12; 200,000 x 1,000, 10, 1: 0.66; few
+// values, 300,000 x 64, 2, 1 / 3: 1.27 / 0.99; 200,000 x 64, 10, 1 / 4 / 6: 1.20 /
+// 1.01 / 0.89.  Fits that grow all trees at once pass by their other sizes; with
+// nodes of up to 32,768 samples the trees at a time hardly matter (30,000 x 256,
+// 1 / 16: 0.89 / 0.87).
 bool list_worth(const FitSize &z, double Fr, const Spread &sp) {
-  const double m = (double)z.m, T = (double)z.T, N = (double)z.N;
+  const double m = (double)z.m, T = (double)z.T, N = (double)z.N, R = (double)z.R;
   if (m * sp.rare < 0.5) return false;
   if (z.N <= (int64_t)kListWg[0]) return z.moves >= 4.5 && Fr * (1.0 - 5.0 * sp.drag) >= 10.0 * m;
   const double Fd = Fr * (1.0 - sp.drag);
-  if ((Fr - 8.0 * m) * T >= 4000.0 && (Fd - 8.0 * m) * T >= 2700.0 &&
+  const bool large = z.N > (int64_t)kListWg[1];
+  if ((!large || R * (Fr - 8.0 * m) * (double)(z.K + 11) >= 10500.0) && (Fr - 8.0 * m) * T >= 4000.0 && (Fd - 8.0 * m) * T >= 2700.0 &&
       T * (std::min(z.moves, 16.0) * Fd - 7.0 * std::min(z.levels, 5.0) * m) >= 56.0 * (double)z.F)
     return true;
   const double Fc = Fr * (1.0 - 2.0 * sp.drag);  // (20,000 x 1,000, 95% two-valued of 0.003, 20 trees: 23 / 27)
-  return sp.few && Fc >= 6.0 * m && Fc * T * N >= 0x1p27 && (10.0 * z.moves + 3.0) * T >= 360.0;
+  return sp.few && (!large || R * Fr * N >= 0x1p26) && Fc >= 6.0 * m && Fc * T * N >= 0x1p27 && (10.0 * z.moves + 3.0) * T >= 360.0;
+}
+
+// Trees that a fit's options and the memory let it grow at a time on one stream:
+// as asked, else what 60% of the free memory holds (workspaces are reused by
+// the fit); in a context with a workspace limit, what the rest of it holds.
+int32_t trees_at_a_time(cta_ctx *ctx, const cta_fit_opts &o, int32_t T, size_t bytes_per_tree) {
+  int32_t per = o.trees_per_batch;
+  if (o.mode != CTA_MODE_BATCHED) per = 1;
+  if (per <= 0 && ctx->ws_limit) {
+    const size_t held = ctx->ws_bytes();
+    const size_t avail = ctx->ws_limit > held ? (size_t)(ctx->ws_limit - held) : 0;
+    per = (int32_t)std::max<size_t>(1, avail / bytes_per_tree);
+  } else if (per <= 0) {
+    size_t fr = 0, tot = 0;
+    HIPC(hipMemGetInfo(&fr, &tot));
+    fr += ctx->ws_bytes() + (ctx->lane ? ctx->lane->ws_bytes() : 0);
+    per = (int32_t)std::max<size_t>(1, (size_t)(0.6 * (double)fr) / bytes_per_tree);
+  }
+  return std::min(per, T);
 }
 
 // Whether a fit of T trees searches its splits from sample lists instead of
@@ -626,8 +659,12 @@ bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T
   // the constant test, where its row shows both ends (of 201 features 140
   // such, 2,500 samples, 5 trees: 3.6 / 4.3; 990 of 1,000, 3,000: 12.5 / 10.0).
   const double inbag = off ? (double)(off[T] - off[0]) / T : o.bootstrap ? kInBag * ds->N : (double)ds->N;
-  return list_worth(fit_size(ds->N, ds->F, T, o.max_features, o, off || o.bootstrap, inbag),
-                    (double)(ds->Fr - ds->two / 2), ds->spread);
+  FitSize z = fit_size(ds->N, ds->F, ds->K, T, o.max_features, o, off || o.bootstrap, inbag);
+  const double Fr = (double)(ds->Fr - ds->two / 2);
+  if (!list_worth(z, Fr, ds->spread)) return false;
+  if (z.N <= (int64_t)kListWg[1]) return true;  // (the trees at a time do not matter)
+  z.R = trees_at_a_time(ctx, o, T, tree_bytes(ds->N, ds->Fr, ds->K, o.max_features, (size_t)ds->idx_bits / 8));
+  return list_worth(z, Fr, ds->spread);
 }
 
 // The list search's tables of a training set (kept with it; built on the
@@ -1612,22 +1649,7 @@ template <class IdxT, class LabT>
 void fit_grow(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, const int64_t *off,
               const cta_fit_opts &o, bool lists, cta_forest *out) {
   Fitter<IdxT, LabT> fz(ctx, ds, o, lists);
-  // trees resident at once on one stream: as asked, else what 60% of the
-  // free memory holds (workspaces are reused by this fit)
-  int32_t per = o.trees_per_batch;
-  if (o.mode != CTA_MODE_BATCHED) per = 1;
-  if (per <= 0 && ctx->ws_limit) {
-    // a context with a workspace limit: the trees the rest of it holds
-    const size_t held = ctx->ws_bytes();
-    const size_t avail = ctx->ws_limit > held ? (size_t)(ctx->ws_limit - held) : 0;
-    per = (int32_t)std::max<size_t>(1, avail / fz.bytes_per_tree());
-  } else if (per <= 0) {
-    size_t fr = 0, tot = 0;
-    HIPC(hipMemGetInfo(&fr, &tot));
-    fr += ctx->ws_bytes() + (ctx->lane ? ctx->lane->ws_bytes() : 0);
-    per = (int32_t)std::max<size_t>(1, (size_t)(0.6 * (double)fr) / fz.bytes_per_tree());
-  }
-  per = std::min(per, T);
+  int32_t per = trees_at_a_time(ctx, o, T, fz.bytes_per_tree());
   // two lanes: batches alternate between this context's stream and a second
   // one, so that one lane's short late levels overlap the other's work; each
   // holds half the trees (two batches resident at once), at least
@@ -2563,7 +2585,7 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
     // and the list search's words and distinct values, where the fit may choose
     // it for data that suit it best (every feature with a row, dense, of few values)
     // and in-bag sets that leave its scans nothing to do
-    FitSize most = fit_size(N, F, T, m, *opts, true, N);
+    FitSize most = fit_size(N, F, K, T, m, *opts, true, N);
     most.levels = 0.0;
     if (list_possible(N, K, *opts, kMaxLds) && (opts->search == CTA_SEARCH_LISTS || list_worth(most, F, Spread{})))
       *dataset_bytes += nf * 8 + n * b + 20 * f;

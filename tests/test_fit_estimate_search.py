@@ -49,3 +49,12 @@ def test_only_fits_that_may_use_lists_are_charged_their_tables(size, lists):
     assert (ds - ROWS[size][0], ws) == (tables if lists else 0, ROWS[size][1])
     ds, ws = _lib.fit_estimate(N, F, K, T, opts(m, search=_lib.CTA_SEARCH_LISTS))
     assert (ds - ROWS[size][0], ws) == (tables, ROWS[size][1])
+
+
+@pytest.mark.parametrize("size,trees_per_batch,lists", [((200000, 256, 20, 200, 16), 1, False),
+                                                        ((200000, 256, 20, 200, 16), 4, True),
+                                                        ((20000, 4096, 5, 100, 64), 1, True)])  # no large nodes
+def test_few_trees_at_a_time_leave_large_nodes_to_rows(size, trees_per_batch, lists):
+    rows = _lib.fit_estimate(*size[:4], opts(size[4], search=_lib.CTA_SEARCH_ROWS, trees_per_batch=trees_per_batch))
+    auto = _lib.fit_estimate(*size[:4], opts(size[4], trees_per_batch=trees_per_batch))
+    assert (auto[0] > rows[0]) == lists and auto[1] == rows[1]

@@ -133,3 +133,39 @@ def test_choice_by_in_bag_sets(ctx):
     print("choice by in-bag sets", flush=True)
     assert search_of(profiled(ctx, ds, T, opts(m), ids)[1]) == "rows"
     assert search_of(profiled(ctx, ds, T, opts(m))[1]) == "lists"
+
+
+@pytest.mark.parametrize("N,F,K,levels,T,R,want", [
+    (40000, 300, 2, 0, 60, 4, "rows"), (40000, 300, 2, 0, 60, 6, "lists"),      # R (F - 8 m) (K + 11) from 10,500
+    (40000, 300, 100, 0, 60, 2, "lists"),
+    (32768, 300, 2, 0, 60, 2, "lists"),                                          # no node of more than 32,768
+    (100000, 100, 5, 17, 40, 2, "rows"), (100000, 100, 5, 17, 40, 8, "lists")])  # few values: R F N from 2^26
+def test_choice_by_trees_at_a_time(ctx, N, F, K, levels, T, R, want):
+    """Few trees at a time leave too few workgroups for large nodes."""
+    X, y = dense(N, F, K, 12)
+    if levels:
+        X = np.clip(np.round(X * 2 + levels // 2), 0, levels - 1).astype(np.float32)
+    m = 17 if not levels else 10
+    ds = _lib.Dataset(ctx, X, y, K)
+    print("choice by trees at a time", N, F, K, levels, R, flush=True)
+    f, st = profiled(ctx, ds, T, opts(m, trees_per_batch=R, max_depth=12))
+    assert search_of(st) == want
+    g, st = profiled(ctx, ds, T, opts(m, trees_per_batch=T, max_depth=12))
+    assert search_of(st) == "lists" and helpers.forest_diff(f, g) is None
+
+
+def test_choice_by_the_memory_for_trees(ctx):
+    """The same where the workspace limit holds one tree at a time."""
+    N, F, K, T, m = 40000, 300, 2, 60, 17
+    X, y = dense(N, F, K, 13)
+    c = _lib.Context(0)
+    ds = _lib.Dataset(c, X, y, K)
+    print("choice by the memory for trees", flush=True)
+    want, st = profiled(c, ds, T, opts(m, max_depth=12))
+    assert search_of(st) == "lists"
+    c.release_workspace()
+    _lib.check(c.lib.cta_ctx_set_workspace_limit(c.h, 140 << 20))
+    f, st = profiled(c, ds, T, opts(m, max_depth=12))
+    assert search_of(st) == "rows" and helpers.forest_diff(f, want) is None
+    ds.close()
+    c.close()

@@ -71,6 +71,19 @@ int guarded(F &&f) {
   }
 }
 
+// What a thread's failing device allocations may give back before they fail
+// (see SpareLists); the innermost one in scope is asked.
+struct Spare {
+  static thread_local Spare *cur;
+  Spare *outer;
+  Spare() : outer(cur) { cur = this; }
+  virtual ~Spare() { cur = outer; }
+  Spare(const Spare &) = delete;
+  Spare &operator=(const Spare &) = delete;
+  virtual bool give_back() = 0;  // false: there was nothing
+};
+thread_local Spare *Spare::cur = nullptr;
+
 // Device allocation owned by RAII.
 struct DevMem {
   void *p = nullptr;
@@ -81,6 +94,11 @@ struct DevMem {
     release();
     if (n == 0) n = 1;
     hipError_t e = hipMalloc(&p, n);
+    if (e == hipErrorOutOfMemory && Spare::cur) {
+      p = nullptr;
+      (void)hipGetLastError();
+      if (Spare::cur->give_back()) e = hipMalloc(&p, n);
+    }
     if (e != hipSuccess) {
       p = nullptr;
       (void)hipGetLastError();
@@ -118,6 +136,7 @@ struct KStat {
 
 struct cta_ctx {
   int device = 0;
+  std::vector<cta_dataset *> listed;  // training sets that hold list tables
   hipStream_t stream = nullptr;
   // second fit lane: a context of its own (stream, workspaces, staging) on
   // the same device, created by the first fit that runs two lanes
@@ -282,6 +301,7 @@ struct cta_dataset {
   DevMem rank, dval, voff, gapw, ndist, all;  // (all: the list of every sample)
   void drop_lists() {
     for (DevMem *m : {&rank, &dval, &voff, &gapw, &ndist, &all}) m->release();
+    if (listed) ctx->listed.erase(std::find(ctx->listed.begin(), ctx->listed.end(), this));
     listed = false;
   }
   // row-free features (two-valued, other than feature 0): tables of the fits
@@ -311,6 +331,23 @@ struct cta_forest {
     threshold.clear();
     for (DevMem *m : {&nodes, &roots, &blocks, &broots}) m->release();
     device_ready = false;
+  }
+};
+
+// The list tables that a context's training sets hold beyond the fits that made
+// them, but for those of `keep`: given back to allocations under its lock.
+struct SpareLists : Spare {
+  cta_ctx *ctx;
+  const cta_dataset *keep;
+  explicit SpareLists(cta_ctx *c, const cta_dataset *k = nullptr) : ctx(c), keep(k) {}
+  bool give_back() override {
+    std::vector<cta_dataset *> drop;
+    for (cta_dataset *d : ctx->listed)
+      if (d != keep) drop.push_back(d);
+    if (drop.empty()) return false;
+    ctx->sync();
+    for (cta_dataset *d : drop) d->drop_lists();
+    return true;
   }
 };
 
@@ -722,6 +759,7 @@ void list_tables(cta_ctx *ctx, cta_dataset *ds) {
     ctx->sync();
     ctx->ws_drop("code_pre");
   }
+  ctx->listed.push_back(ds);
   ds->listed = true;
 }
 
@@ -1745,7 +1783,8 @@ void fit_grow(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, con
 
 // Grows the forest.  The list search needs tables, and task lists of other
 // sizes than the rows': where they cannot be had the rows are searched, and
-// rows that lack the memory the tables of an earlier fit hold take it.
+// rows that lack the memory the tables of an earlier fit hold take it (in the
+// second lane's thread too, which has nothing to give back).
 template <class IdxT, class LabT>
 void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, const int64_t *off,
               const cta_fit_opts &o, cta_forest *out) {
@@ -1759,6 +1798,7 @@ void fit_impl(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *ids, con
   };
   if (list_search(ctx, ds, o, T, ids ? off : nullptr)) {
     try {
+      SpareLists spare(ctx, ds);
       list_tables<IdxT, LabT>(ctx, ds);
       if (o.lanes == 2) ctx->sync();  // (the other lane's stream reads them too)
       return fit_grow<IdxT, LabT>(ctx, ds, T, ids, off, o, true, out);
@@ -2051,6 +2091,7 @@ static int dataset_create_common(cta_ctx *ctx, const float *X, const uint32_t *y
     if (idx_bits == 16 && N > 65535) fail(CTA_EINVAL, "16-bit indices need N <= 65535");
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     HIPC(hipSetDevice(ctx->device));
+    SpareLists spare(ctx);
     std::unique_ptr<cta_dataset> ds(new cta_dataset());
     ds->ctx = ctx;
     ds->N = N;
@@ -2116,6 +2157,7 @@ int cta_dataset_create_keys(cta_ctx *ctx, const float *X, const void *keys, int3
     if (idx_bits == 16 && N > 65535) fail(CTA_EINVAL, "16-bit indices need N <= 65535");
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     HIPC(hipSetDevice(ctx->device));
+    SpareLists spare(ctx);
     hipStream_t st = ctx->stream;
     DevMem dX((size_t)N * F * 4), dk((size_t)N * 8), dy((size_t)N * 4);
     HIPC(hipMemcpyAsync(dX.p, X, (size_t)N * F * 4, hipMemcpyHostToDevice, st));
@@ -2163,6 +2205,7 @@ int cta_dataset_destroy(cta_dataset *ds) {
     std::lock_guard<std::recursive_mutex> lk(ds->ctx->mu);
     (void)hipSetDevice(ds->ctx->device);
     (void)hipStreamSynchronize(ds->ctx->stream);
+    ds->drop_lists();
     delete ds;
   });
 }
@@ -2235,6 +2278,7 @@ int cta_fit(cta_ctx *ctx, cta_dataset *ds, int32_t T, const uint32_t *boot_ids, 
     }
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     HIPC(hipSetDevice(ctx->device));
+    SpareLists spare(ctx);
     std::unique_ptr<cta_forest> f(new cta_forest());
     f->ctx = ctx;
     f->F = ds->F;
@@ -2331,6 +2375,7 @@ static cta_forest *import_arrays(cta_ctx *ctx, int32_t T, int32_t F, int32_t K, 
   if (depth) f->depth.assign(depth, depth + n);
   for (int64_t j = 0; j < n; ++j)
     if (f->left[j] == 0 || f->right[j] == 0) f->left[j] = f->right[j] = 0;
+  SpareLists spare(ctx);
   upload_forest(f.get());
   return f.release();
 }
@@ -2482,6 +2527,7 @@ int cta_predict(cta_ctx *ctx, cta_forest *f, const float *X, int64_t R, int32_t 
     if (R == 0) return;
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     HIPC(hipSetDevice(ctx->device));
+    SpareLists spare(ctx);
     float *dX = ctx->ws_as<float>("pred_x", (size_t)R * F);
     uint32_t *dl = ctx->ws_as<uint32_t>("pred_labels", (size_t)R);
     uint32_t *dv = votes ? ctx->ws_as<uint32_t>("pred_vout", (size_t)R * f->K) : nullptr;
@@ -2502,6 +2548,7 @@ int cta_predict_device(cta_ctx *ctx, cta_forest *f, const float *X_dev, int64_t 
     if (R == 0) return;
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     HIPC(hipSetDevice(ctx->device));
+    SpareLists spare(ctx);
     predict_dev(ctx, f, X_dev, R, labels_dev, votes_dev);
     ctx->sync();
   });

@@ -195,3 +195,39 @@ def test_limited_context_without_room_for_list_tasks():
     assert limited(ctx) <= held
     ds.close()
     ctx.close()
+
+
+def test_tables_make_way_for_another_training_set():
+    """The tables of a fit on 60,000 x 1,000 (480 MB) stay with that training set;
+    with 450 MB free, another one of 20,000 x 1,000 (700 MB while it is built) and
+    its fit take their memory, and a later fit builds them again."""
+    N, F, K, T, m = 60000, 1000, 5, 5, 10
+    X, y = gauss(N, F, K, 7)
+    ctx = _lib.Context(0)
+    a = _lib.Dataset(ctx, X, y, K)
+
+    def fit(ds):
+        return _lib.Forest.fit(ctx, ds, T, opts(m), None).export()
+
+    want, rows, lists = searches(ctx, lambda: fit(a))
+    assert lists and not rows
+    n = 20000
+    b = _lib.Dataset(ctx, X[:n], y[:n], K)
+    want_b = fit(b)
+    b.close()
+    fit(a)
+    ctx.release_workspace()
+    print("another training set", flush=True)
+    hog = Hog(ctx, 450 << 20)
+    try:
+        b = _lib.Dataset(ctx, X[:n], y[:n], K)
+        ctx.release_workspace()
+        got_b = fit(b)
+    finally:
+        hog.free()
+    assert helpers.forest_diff(got_b, want_b) is None
+    got, rows, lists = searches(ctx, lambda: fit(a))
+    assert lists and not rows and helpers.forest_diff(got, want) is None
+    b.close()
+    a.close()
+    ctx.close()

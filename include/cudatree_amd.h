@@ -133,7 +133,8 @@ typedef struct {
                                 sorted rows of every feature, moved at every level) or CTA_SEARCH_LISTS (2: from
                                 the nodes' sample lists, sorting the features a node evaluates, where the sizes
                                 and the memory for its tables allow it, else rows); other values are taken as 0.
-                                The trees are identical */
+                                The tables stay with the dataset for its next fit, until it is destroyed or a
+                                device allocation of its context needs their memory.  The trees are identical */
 } cta_fit_opts;
 
 #define CTA_SEARCH_AUTO 0

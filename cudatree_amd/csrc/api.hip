@@ -586,16 +586,18 @@ struct FitSize {
   int64_t R;      // trees grown at a time
   double levels;  // of nodes that split, by the depth limit, the leaf size and the in-bag samples (a share of one
                   // for in-bag sets smaller than a bootstrap's)
+  double cut;     // levels below those that the limits take off
   double moves;   // times that sorted rows of N samples are moved: the bootstrap's, then a level's in-bag share
 };
 // (inbag: mean in-bag samples of a tree; unbalanced trees have about half as
 // many levels again as balanced ones)
 FitSize fit_size(int64_t N, int64_t F, int64_t K, int64_t T, int64_t m, const cta_fit_opts &o, bool bagged,
                  double inbag) {
-  FitSize z = {N, F, K, m, T, o.trees_per_batch > 0 ? std::min<int64_t>(o.trees_per_batch, T) : T, 0.0, 0.0};
+  FitSize z = {N, F, K, m, T, o.trees_per_batch > 0 ? std::min<int64_t>(o.trees_per_batch, T) : T, 0.0, 0.0, 0.0};
   const double leaf = std::max(1.0, (double)o.min_samples_split);
   if (inbag >= leaf) z.levels = 1.0 + std::floor(1.5 * std::log2(inbag / leaf));
   if (o.max_depth > 0) z.levels = std::min(z.levels, (double)o.max_depth);
+  z.cut = 1.0 + 1.5 * std::log2(std::max(1.0, inbag)) - z.levels;
   z.moves = (bagged ? 1.0 : 0.0) + std::max(0.0, z.levels - 1.0) * inbag / (double)N;
   z.levels *= std::min(1.0, inbag / (kInBag * (double)N));
   return z;
@@ -645,18 +647,24 @@ FitSize fit_size(int64_t N, int64_t F, int64_t K, int64_t T, int64_t m, const ct
 // values, 300,000 x 64, 2, 1 / 3: 1.27 / 0.99; 200,000 x 64, 10, 1 / 4 / 6: 1.20 /
 // 1.01 / 0.89.  Fits that grow all trees at once pass by their other sizes; with
 // nodes of up to 32,768 samples the trees at a time hardly matter (30,000 x 256,
-// 1 / 16: 0.89 / 0.87).
+// 1 / 16: 0.89 / 0.87), but they do without the small nodes that a depth limit or
+// the leaf size takes off, where lists spare the most: 22,232 x 222, depth 6, 1:
+// 1.33; 81,901 x 463, 100 classes, depth 6, 1: 1.62; leaves of 200, 7,261 x 387, 3:
+// 1.29; of 500, 10,502 x 1,917, 8: 1.29; small sets, 3,926 x 1,051, leaves of 200,
+// 2 trees in all: 1.30.
 bool list_worth(const FitSize &z, double Fr, const Spread &sp) {
   const double m = (double)z.m, T = (double)z.T, N = (double)z.N, R = (double)z.R;
   if (m * sp.rare < 0.5) return false;
+  if (z.cut > 4.0 && ((z.R < z.T && z.R <= 8) || (z.N <= (int64_t)kListWg[0] && z.R <= 5))) return false;
   if (z.N <= (int64_t)kListWg[0]) return z.moves >= 4.5 && Fr * (1.0 - 5.0 * sp.drag) >= 10.0 * m;
   const double Fd = Fr * (1.0 - sp.drag);
   const bool large = z.N > (int64_t)kListWg[1];
-  if ((!large || R * (Fr - 8.0 * m) * (double)(z.K + 11) >= 10500.0) && (Fr - 8.0 * m) * T >= 4000.0 && (Fd - 8.0 * m) * T >= 2700.0 &&
-      T * (std::min(z.moves, 16.0) * Fd - 7.0 * std::min(z.levels, 5.0) * m) >= 56.0 * (double)z.F)
+  if ((!large || R * (Fr - 8.0 * m) * (double)(z.K + 11) >= 10500.0) && (Fr - 8.0 * m) * T >= 4000.0 &&
+      (Fd - 8.0 * m) * T >= 2700.0 && T * (std::min(z.moves, 16.0) * Fd - 7.0 * std::min(z.levels, 5.0) * m) >= 56.0 * (double)z.F)
     return true;
   const double Fc = Fr * (1.0 - 2.0 * sp.drag);  // (20,000 x 1,000, 95% two-valued of 0.003, 20 trees: 23 / 27)
-  return sp.few && (!large || R * Fr * N >= 0x1p26) && Fc >= 6.0 * m && Fc * T * N >= 0x1p27 && (10.0 * z.moves + 3.0) * T >= 360.0;
+  return sp.few && (!large || R * Fr * N >= 0x1p26) && Fc >= 6.0 * m && Fc * T * N >= 0x1p27 &&
+         (10.0 * z.moves + 3.0) * T >= 360.0;
 }
 
 // Trees that a fit's options and the memory let it grow at a time on one stream:
@@ -699,7 +707,7 @@ bool list_search(cta_ctx *ctx, cta_dataset *ds, const cta_fit_opts &o, int32_t T
   FitSize z = fit_size(ds->N, ds->F, ds->K, T, o.max_features, o, off || o.bootstrap, inbag);
   const double Fr = (double)(ds->Fr - ds->two / 2);
   if (!list_worth(z, Fr, ds->spread)) return false;
-  if (z.N <= (int64_t)kListWg[1]) return true;  // (the trees at a time do not matter)
+  if (z.N <= (int64_t)kListWg[1] && z.cut <= 4.0) return true;  // (the trees at a time do not matter)
   z.R = trees_at_a_time(ctx, o, T, tree_bytes(ds->N, ds->Fr, ds->K, o.max_features, (size_t)ds->idx_bits / 8));
   return list_worth(z, Fr, ds->spread);
 }
@@ -2633,7 +2641,7 @@ int cta_fit_estimate(int32_t N, int32_t F, int32_t K, int32_t T, const cta_fit_o
     // it for data that suit it best (every feature with a row, dense, of few values)
     // and in-bag sets that leave its scans nothing to do
     FitSize most = fit_size(N, F, K, T, m, *opts, true, N);
-    most.levels = 0.0;
+    most.levels = most.cut = 0.0;
     if (list_possible(N, K, *opts, kMaxLds) && (opts->search == CTA_SEARCH_LISTS || list_worth(most, F, Spread{})))
       *dataset_bytes += nf * 8 + n * b + 20 * f;
     // the context's workspaces: radix-sort and code-column temporaries of the

@@ -148,9 +148,9 @@ def test_choice_by_trees_at_a_time(ctx, N, F, K, levels, T, R, want):
     m = 17 if not levels else 10
     ds = _lib.Dataset(ctx, X, y, K)
     print("choice by trees at a time", N, F, K, levels, R, flush=True)
-    f, st = profiled(ctx, ds, T, opts(m, trees_per_batch=R, max_depth=12))
+    f, st = profiled(ctx, ds, T, opts(m, trees_per_batch=R))
     assert search_of(st) == want
-    g, st = profiled(ctx, ds, T, opts(m, trees_per_batch=T, max_depth=12))
+    g, st = profiled(ctx, ds, T, opts(m, trees_per_batch=T))
     assert search_of(st) == "lists" and helpers.forest_diff(f, g) is None
 
 
@@ -161,11 +161,25 @@ def test_choice_by_the_memory_for_trees(ctx):
     c = _lib.Context(0)
     ds = _lib.Dataset(c, X, y, K)
     print("choice by the memory for trees", flush=True)
-    want, st = profiled(c, ds, T, opts(m, max_depth=12))
+    want, st = profiled(c, ds, T, opts(m))
     assert search_of(st) == "lists"
     c.release_workspace()
     _lib.check(c.lib.cta_ctx_set_workspace_limit(c.h, 140 << 20))
-    f, st = profiled(c, ds, T, opts(m, max_depth=12))
+    f, st = profiled(c, ds, T, opts(m))
     assert search_of(st) == "rows" and helpers.forest_diff(f, want) is None
     ds.close()
     c.close()
+
+
+@pytest.mark.parametrize("kw,R,want", [({"min_samples_split": 200}, 4, "rows"), ({"min_samples_split": 200}, 30, "lists"),
+                                       ({"max_depth": 7}, 8, "rows"), ({"max_depth": 7}, 9, "lists"), ({}, 4, "lists")])
+def test_choice_by_cut_trees_at_a_time(ctx, kw, R, want):
+    """Few trees at a time without their small nodes."""
+    N, F, T, m = 8000, 500, 30, 17
+    X, y = dense(N, F, 5, 14)
+    ds = _lib.Dataset(ctx, X, y, 5)
+    print("choice by cut trees at a time", kw, R, flush=True)
+    f, st = profiled(ctx, ds, T, opts(m, trees_per_batch=R, **kw))
+    assert search_of(st) == want
+    g, st = profiled(ctx, ds, T, opts(m, **kw))
+    assert search_of(st) == "lists" and helpers.forest_diff(f, g) is None

@@ -183,3 +183,20 @@ def test_choice_by_cut_trees_at_a_time(ctx, kw, R, want):
     assert search_of(st) == want
     g, st = profiled(ctx, ds, T, opts(m, **kw))
     assert search_of(st) == "lists" and helpers.forest_diff(f, g) is None
+
+
+@pytest.mark.parametrize("T,want", [(5, "rows"), (12, "lists")])
+def test_choice_by_partly_rare_few_values(ctx, T, want):
+    """Features of 17 levels beside zeros in 0 to 100% of the samples: a share of
+    them is rare enough to drag the constant tests of a large set."""
+    N, F, m = 350000, 98, 10
+    rng = np.random.Generator(np.random.PCG64(15))
+    y = rng.integers(0, 2, size=N)
+    X = np.clip(np.round(rng.standard_normal((N, F), dtype=np.float32) * 2 + 8 + y[:, None]), 0, 16)
+    X *= rng.random((N, F), dtype=np.float32) < rng.random(F, dtype=np.float32) ** 2
+    ds = _lib.Dataset(ctx, X.astype(np.float32), y, 2)
+    print("choice by partly rare few values", T, flush=True)
+    f, st = profiled(ctx, ds, T, opts(m))
+    assert search_of(st) == want
+    g, _ = profiled(ctx, ds, T, opts(m, search=_lib.CTA_SEARCH_ROWS if want == "lists" else _lib.CTA_SEARCH_LISTS))
+    assert helpers.forest_diff(f, g) is None
